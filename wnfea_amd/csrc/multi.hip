@@ -31,123 +31,224 @@ __device__ __forceinline__ void load_cols(const XT* __restrict__ p, XT (&v)[NR])
 }
 
 // Sliced-ELL block SpMM (layout of sell.hpp) on NR interleaved columns.
-template <int BR, int BC, typename VT, typename XT, int W, int NR, class Op>
-__global__ __launch_bounds__(64 * W) void sell_spmm_kernel(SellView<VT> A, const XT* __restrict__ x, Op op,
-                                                           int xcd_remap, const int* flags, int guard) {
+//
+// Bound: L1 and instruction issue.  A block's BC x rows (96 bytes for FP32
+// 3x3 and 8 columns) are contiguous, and loads of a line that is still on its
+// way stall the L1 pipeline (40 % of the cycles of a kernel whose lanes load
+// their block's x rows one after the other), so each line is asked for once:
+// a wavefront takes 64 blocks at a time, one per lane, its lanes load the x
+// of those blocks as one stream of 16-byte chunks (lane t of load i takes
+// chunk 64 i + t; CH chunks per block) into LDS, and every lane reads its own
+// block's rows from there.  A row's blocks are split over G >= max(8, L)
+// lanes (lane group q takes blocks q, q + G, ...; L divides G), so a
+// wavefront works on RW = 64 / G rows of one slice, its addresses advance by
+// a constant per step, and no row waits for another wavefront.  The groups'
+// sums meet in a reduce-scatter (at each level a lane keeps half of its
+// columns), and one more exchange turns the lanes to the outputs' memory
+// order: lane n has column n mod NR of row (n / NR) mod RW, so that the
+// epilogue's loads (issued before the block loop) and stores of a row are
+// contiguous.  Idx: 32-bit offsets into x where they suffice.
+// Measured with 8 columns on 212 355 rows (24 blocks of 3x3 per row), FP32
+// Chebyshev step / FP64 product / 6x6 level-1 step, us: all columns per lane
+// with x from L1 and four wavefronts per slice 72 / 107 / 50; four columns
+// per lane with x from L1 and the reduce-scatter 45 / 72 / 27; this kernel
+// 44 / 58 / 26.  (Loading a step's x during the one before costs 22 registers
+// and gains nothing; one scalar column per lane, three times the loads, takes
+// 75 / 80 / 45.)
+template <int BR, int BC, typename XT, int NR>
+constexpr int spmm_waves() {  // wavefronts per workgroup: at most 56 KB of LDS
+  return BC * NR * (int)sizeof(XT) > 208 ? 2 : 4;
+}
+
+template <int BR, int BC, typename VT, typename XT, int NR, typename Idx, class Op>
+__global__ __launch_bounds__(64 * (spmm_waves<BR, BC, XT, NR>())) void sell_spmm_kernel(
+    SellView<VT> A, const XT* __restrict__ x, Op op, int gsh, int xcd_remap, const int* flags, int guard) {
   if (guard_skip(flags, guard)) return;
   using AT = typename AccT<VT>::type;
-  constexpr int BB = BR * BC;
-  constexpr int kLoads = 1 + (BB * (int)sizeof(VT) + 15) / 16 + BC * ((NR * (int)sizeof(XT) + 15) / 16);
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int s = slice_of_block(A.n_slices, xcd_remap);
-  double dot[Op::kDots > 0 ? Op::kDots : 1];
+  constexpr int BB = BR * BC, W = spmm_waves<BR, BC, XT, NR>();
+  constexpr int V = 16 / (int)sizeof(VT), FULL = BB / V, REM = BB - FULL * V;
+  constexpr int XV = 16 / (int)sizeof(XT), CH = BC * NR / XV;  // x values per chunk, chunks per block
+  static_assert(NR % XV == 0 && (NR & (NR - 1)) == 0, "column split");
+  using Chunk = XT __attribute__((ext_vector_type(XV)));
+  __shared__ Chunk xs[W][64 * CH];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lsh = __ffs(A.lanes) - 1, rsh = 6 - lsh;  // log2 of L and of the rows per slice
+  const int G = 1 << gsh, RW = 64 >> gsh;             // lsh <= gsh: a wavefront stays in one slice
+  // this wavefront's row positions pos0 .. pos0 + RW, below end
+  const int end = A.n_slices << rsh;
+  const int pos0 = (slice_of_block((end + W * RW - 1) / (W * RW), xcd_remap) * W + wave) * RW;
+  double dot = 0.0;
+  if (pos0 < end) {
+    // this lane's outputs: column ek, rows es, es + RS, ... of block row erow
+    const int ek = lane % NR, el = (lane / NR) & (RW - 1), es = lane / NR >> (6 - gsh), RS = G / NR;
+    const int erow = A.rinfo[pos0 + el].x;
+    const long long eo = (long long)(erow < 0 ? 0 : erow) * BR * NR + ek;
+    typename Op::Pre pre[BR];
+    if (erow >= 0) {
 #pragma unroll
-  for (int k = 0; k < (Op::kDots > 0 ? Op::kDots : 1); ++k) dot[k] = 0.0;
-  if (s < A.n_slices) {
-    const int rps = 64 / A.lanes;  // rows per slice; a row's lanes are r, r + rps, ...
-    const int2 ri = A.rinfo[(long long)s * rps + lane % rps];
-    const int len = lane_steps(ri.y, lane / rps, A.lanes);
+      for (int r = 0; r < BR; ++r)
+        if ((r & (RS - 1)) == es) op.load(eo + r * NR, (long long)erow * BR + r, pre[r]);
+    }
+    // this lane's blocks: q, q + G, ... of row position pos0 + rl, found in
+    // step (q >> lsh) + t (G / L) of the slice at lane r0 + R (q mod L)
+    const int rl = lane & (RW - 1), q = lane >> (6 - gsh);
+    const int s = pos0 >> rsh, r0 = (pos0 & ((1 << rsh) - 1)) + rl;
+    const int len = A.rinfo[pos0 + rl].y;
     const long long base = A.off[s];
-    AT acc[BR * NR];
-#pragma unroll
-    for (int t = 0; t < BR * NR; ++t) acc[t] = AT(0);
-    const int* __restrict__ colp = A.col + base + lane;
+    const int n_steps = (int)((A.off[s + 1] - base) >> 6);  // of the slice, L blocks of a row each
+    const int steps = (n_steps + (1 << (gsh - lsh)) - 1) >> (gsh - lsh);
+    const int sl = r0 + ((q & (A.lanes - 1)) << rsh);
+    int step = q >> lsh;
+    const int* __restrict__ colp = A.col + base;
     const VT* __restrict__ valp = A.val + base * BB;
-    for (int j = wave; j < len; j += W) {
-      const int c = load_col(colp + (long long)j * 64);
+    AT acc[BR][NR];
+#pragma unroll
+    for (int r = 0; r < BR; ++r)
+#pragma unroll
+      for (int k = 0; k < NR; ++k) acc[r][k] = AT(0);
+    // a lane without a block in a step loads its row's first one again, unused
+    const auto column = [&](int b, int st) { return load_col(colp + (b < len ? 64 * st + sl : sl)); };
+    int b = q, cn = steps > 0 ? column(b, step) : 0;
+    for (int t = 0; t < steps; ++t) {
+      const bool have = b < len;
+      // chunk 64 i + lane belongs to block (64 i + lane) / CH of the wavefront
+      Chunk xc[CH];
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int ch = 64 * i + lane;
+        const Idx c = (Idx)__shfl(cn, ch / CH, 64);
+        xc[i] = *reinterpret_cast<const Chunk*>(reinterpret_cast<const char*>(x) +
+                                                (c * (Idx)(BC * NR * sizeof(XT)) + (Idx)(ch % CH * 16)));
+      }
       VT v[BB];
-      load_block<VT, BB>(valp + (long long)j * 64 * BB, lane, v);
+      {
+        const unsigned st = have ? step : 0;
+        const VT* __restrict__ region = valp;
+        const unsigned o = st * (64 * BB);
 #pragma unroll
-      for (int q = 0; q < BC; ++q) {
-        XT xv[NR];
-        load_cols<XT, NR>(x + ((long long)c * BC + q) * NR, xv);
-#pragma unroll
-        for (int r = 0; r < BR; ++r)
-#pragma unroll
-          for (int k = 0; k < NR; ++k) acc[r * NR + k] = fma(AT(v[r * BC + q]), AT(xv[k]), acc[r * NR + k]);
+        for (int g = 0; g < FULL; ++g) load_vec<VT, V>(region + (o + g * 64 * V + sl * V), v + g * V);
+        if constexpr (REM > 0) load_vec<VT, REM>(region + (o + FULL * 64 * V + sl * REM), v + FULL * V);
       }
-      // FP32 3x3 blocks: all of the block's loads (column index, values, the
-      // NR-wide x rows) in flight together before its FMAs; left to itself
-      // the compiler reuses the x registers and waits between the x loads
-      // (I-beam, 8 columns: 277 -> 258 us).  The FP64 and 6x6 forms are left
-      // to the compiler: the hint raised their registers and slowed the FP64
-      // product (370 -> 467 us).
-      if constexpr (sizeof(XT) == 4 && BB <= 9) {
-        __builtin_amdgcn_sched_group_barrier(0x020, kLoads, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 2 * BB * NR, 0);
+      b += G;
+      step += 1 << (gsh - lsh);
+      if (t + 1 < steps) cn = column(b, step);  // one step ahead of its x
+#pragma unroll
+      for (int i = 0; i < CH; ++i) xs[wave][64 * i + lane] = xc[i];
+      // only this wavefront's part of xs is read: LDS operations of a
+      // wavefront complete in order
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (have) {
+#pragma unroll
+        for (int k = 0; k < BC; ++k) {
+          XT xv[NR];
+#pragma unroll
+          for (int i = 0; i < NR / XV; ++i) {
+            const Chunk c = xs[wave][lane * CH + k * (NR / XV) + i];
+#pragma unroll
+            for (int e = 0; e < XV; ++e) xv[i * XV + e] = c[e];
+          }
+#pragma unroll
+          for (int r = 0; r < BR; ++r)
+#pragma unroll
+            for (int c = 0; c < NR; ++c) acc[r][c] = fma(AT(v[r * BC + k]), AT(xv[c]), acc[r][c]);
+        }
       }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
-    if constexpr (W > 1) {
-      __shared__ AT red[W - 1][BR * NR][64];
-      if (wave > 0) {
+    // reduce-scatter over the low bits of q (bit m keeps the half
+    // NR >> (m + 1) of its columns), plain sums over the rest
 #pragma unroll
-        for (int t = 0; t < BR * NR; ++t) red[wave - 1][t][lane] = acc[t];
+    for (int r = 0; r < BR; ++r) {
+#pragma unroll
+      for (int m = 0; (NR >> m) > 1; ++m) {
+        const int half = NR >> (m + 1);
+        const bool hi = (q >> m) & 1;
+#pragma unroll
+        for (int c = 0; c < half; ++c) {
+          const AT give = hi ? acc[r][c] : acc[r][c + half], keep = hi ? acc[r][c + half] : acc[r][c];
+          acc[r][c] = keep + __shfl_xor(give, RW << m, 64);
+        }
       }
-      __syncthreads();
-      if (wave == 0) {
-#pragma unroll
-        for (int w = 0; w < W - 1; ++w)
-#pragma unroll
-          for (int t = 0; t < BR * NR; ++t) acc[t] += red[w][t][lane];
-      }
+      for (int off = NR; off < G; off *= 2) acc[r][0] += __shfl_xor(acc[r][0], off * RW, 64);
     }
-    for (int off = 32; off >= rps; off >>= 1)
+    // to the outputs' order: column ek is in the groups whose low bits, read
+    // backwards, are ek
+    int qe = 0;
 #pragma unroll
-      for (int t = 0; t < BR * NR; ++t) acc[t] += __shfl_xor(acc[t], off, 64);
-    const int row = ri.x;
-    // every lane of the row holds the full sums after the butterfly: the row's
-    // L lanes share the NR columns of the epilogue (column k on sub-lane k mod L)
-    if (wave == 0 && row >= 0) op.row(row, acc, dot, lane / rps, A.lanes);
+    for (int m = 0; (NR >> m) > 1; ++m) qe |= ((ek / (NR >> (m + 1))) & 1) << m;
+    const int src = el + RW * (qe + NR * es);
+#pragma unroll
+    for (int r = 0; r < BR; ++r) {
+      const AT a = __shfl(acc[r][0], src, 64);
+      if (erow >= 0 && (r & (RS - 1)) == es) op.out(eo + r * NR, a, dot, pre[r]);
+    }
   }
   if constexpr (Op::kDots > 0) {
-    __shared__ double sred[W];
-    double v[Op::kDots];
 #pragma unroll
-    for (int k = 0; k < Op::kDots; ++k) v[k] = block_sum(dot[k], sred);
-    store_block_partials<Op::kDots>(v, op.partials);
+    for (int off = 32; off >= NR; off >>= 1) dot += __shfl_xor(dot, off, 64);
+    __shared__ double sm[W][NR];
+    if (lane < NR) sm[wave][lane] = dot;
+    __syncthreads();
+    if (threadIdx.x < NR) {
+      double t = 0.0;
+#pragma unroll
+      for (int w = 0; w < W; ++w) t += sm[w][threadIdx.x];
+      op.partials[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
+    }
   }
 }
 
-// ---------------------------------------------------------------- epilogues (index (i*BR + r)*NR + k)
-template <int BR, int NR, typename YT, typename AT>
+// ---------------------------------------------------------------- epilogues
+// One output: o = (i BR + r) NR + k of the interleaved columns, i_r = i BR + r.
+template <typename YT, typename AT>
 struct MOpStore {  // y = A x, or y += A x with add
   static constexpr int kDots = 0;
   YT* y;
   int add;
   double* partials = nullptr;
-  __device__ __forceinline__ void row(int i, const AT (&acc)[BR * NR], double*, int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r)
-#pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        if ((k & (L - 1)) != q) continue;
-        const long long o = ((long long)i * BR + r) * NR + k;
-        y[o] = add ? YT(AT(y[o]) + acc[r * NR + k]) : YT(acc[r * NR + k]);
-      }
+  struct Pre { AT y; };
+  __device__ __forceinline__ void load(long long o, long long, Pre& p) const { p.y = add ? AT(y[o]) : AT(0); }
+  __device__ __forceinline__ void out(long long o, AT a, double&, const Pre& p) const { y[o] = YT(p.y + a); }
+};
+
+// y = R x and the coarse level's first Chebyshev iterate x1 = d1 = c2 dinv y
+// (the expression of the separate first-step kernel).
+template <typename T, typename AT>
+struct MOpRestrictFirst {
+  static constexpr int kDots = 0;
+  T* y;
+  const T* dinv;
+  T* x1;
+  T* d1;
+  T c2;
+  double* partials = nullptr;
+  struct Pre { T dinv; };
+  __device__ __forceinline__ void load(long long, long long i_r, Pre& p) const { p.dinv = dinv[i_r]; }
+  __device__ __forceinline__ void out(long long o, AT a, double&, const Pre& p) const {
+    const T b = T(a), v = c2 * p.dinv * b;
+    y[o] = b;
+    d1[o] = v;
+    x1[o] = v;
   }
 };
 
-template <int BR, int NR, typename T>
+template <typename T>
 struct MOpSpmvDot {  // q = A p, gamma_k = p_k . q_k
-  static constexpr int kDots = NR;
+  static constexpr int kDots = 1;
   T* y;
   const T* p;
   double* partials;
-  __device__ __forceinline__ void row(int i, const T (&acc)[BR * NR], double* d, int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r)
-#pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        if ((k & (L - 1)) != q) continue;
-        const long long o = ((long long)i * BR + r) * NR + k;
-        y[o] = acc[r * NR + k];
-        d[k] += double(p[o]) * double(acc[r * NR + k]);
-      }
+  struct Pre { T p; };
+  __device__ __forceinline__ void load(long long o, long long, Pre& pr) const { pr.p = p[o]; }
+  __device__ __forceinline__ void out(long long o, T a, double& d, const Pre& pr) const {
+    y[o] = a;
+    d += double(pr.p) * double(a);
   }
 };
 
-template <int BR, int NR, typename T>
+template <typename T>
 struct MOpCheb {  // res = b - A x_in; d = c1 d + c2 dinv res; x_out = x_in + d
   static constexpr int kDots = 0;
   const T* b;
@@ -157,56 +258,66 @@ struct MOpCheb {  // res = b - A x_in; d = c1 d + c2 dinv res; x_out = x_in + d
   T* d;
   T c1, c2;
   double* partials = nullptr;
-  __device__ __forceinline__ void row(int i, const T (&acc)[BR * NR], double*, int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r) {
-      const T di = dinv[(long long)i * BR + r];
-#pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        if ((k & (L - 1)) != q) continue;
-        const long long o = ((long long)i * BR + r) * NR + k;
-        const T dn = c1 * d[o] + c2 * di * (b[o] - acc[r * NR + k]);
-        d[o] = dn;
-        x_out[o] = x_in[o] + dn;
-      }
-    }
+  struct Pre { T b, dinv, x, d; };
+  __device__ __forceinline__ void load(long long o, long long i_r, Pre& p) const {
+    p.b = b[o];
+    p.dinv = dinv[i_r];
+    p.x = x_in[o];
+    p.d = d[o];
+  }
+  __device__ __forceinline__ void out(long long o, T a, double&, const Pre& p) const {
+    const T dn = c1 * p.d + c2 * p.dinv * (p.b - a);
+    d[o] = dn;
+    x_out[o] = p.x + dn;
   }
 };
 
-template <int BR, int NR, typename T>
+template <typename T>
 struct MOpDefect {
   static constexpr int kDots = 0;
   const T* b;
   T* res;
   double* partials = nullptr;
-  __device__ __forceinline__ void row(int i, const T (&acc)[BR * NR], double*, int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r)
-#pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        if ((k & (L - 1)) != q) continue;
-        const long long o = ((long long)i * BR + r) * NR + k;
-        res[o] = b[o] - acc[r * NR + k];
-      }
-  }
+  struct Pre { T b; };
+  __device__ __forceinline__ void load(long long o, long long, Pre& p) const { p.b = b[o]; }
+  __device__ __forceinline__ void out(long long o, T a, double&, const Pre& p) const { res[o] = p.b - a; }
 };
 
 // ---------------------------------------------------------------- launch
+// log2 of the lanes per row, at least those of the layout: 8, or 16 where the
+// matrix would leave the chip with few wavefronts (under about four per SIMD)
+// and its rows hold two blocks per lane (8 columns; 12 285 rows of 23 3x3
+// blocks: 4.75 -> 4.57 ms per 8 load cases; 4 441 rows of 60 6x6 blocks, the
+// level below 70 785 rows: 36.4 -> 35.5 ms per 12; the 70 785 rows
+// themselves: 36.4 -> 38.8 ms, so they keep 8).
+static int spmm_group_shift(const SellMatrix& A) {
+  int g = 3;
+  if (((long long)A.n_rows << g) < 64LL * 4096 && A.nnzb >= 16LL * A.n_rows) ++g;
+  while ((1 << g) < A.lanes) ++g;
+  return g;
+}
+
+// workgroups of the SpMM (each writes one partial per column of a fused dot);
+// xs: bytes per value of x
+static int spmm_grid(const SellMatrix& A, int nr, int xs, int xcd) {
+  const int waves = A.bc * nr * xs > 208 ? 2 : 4;  // spmm_waves
+  const int rows = waves * (64 >> spmm_group_shift(A));
+  const int n = ceil_div((long)A.n_slices * (64 / A.lanes), rows);
+  return xcd ? 8 * ceil_div(n, 8) : n;
+}
+
 template <int BR, int BC, typename VT, typename XT, int NR, class Op>
 static int launch_spmm(const SellMatrix& A, const XT* x, const Op& op, const SpmvTune& t, hipStream_t s) {
   const SellView<VT> v = A.view<VT>();
   if (A.n_slices == 0) return kOk;
-  const int xcd = t.xcd_for<VT>();
-  const int grid = xcd ? 8 * ((A.n_slices + 7) / 8) : A.n_slices;
-  // four waves per slice where the partial accumulators fit in LDS (3-row
-  // blocks), one for the 6-row blocks
-  if constexpr (BR * NR <= 32) {
-    hipLaunchKernelGGL((sell_spmm_kernel<BR, BC, VT, XT, 4, NR, Op>), dim3(grid), dim3(256), 0, s, v, x, op,
-                       xcd, t.flags, t.guard);
-  } else {
-    hipLaunchKernelGGL((sell_spmm_kernel<BR, BC, VT, XT, 1, NR, Op>), dim3(grid), dim3(64), 0, s, v, x, op,
-                       xcd, t.flags, t.guard);
-  }
+  const int xcd = t.xcd_for<VT>(), g = spmm_group_shift(A);
+  const dim3 grid(spmm_grid(A, NR, sizeof(XT), xcd)), block(64 * spmm_waves<BR, BC, XT, NR>());
+  if ((long long)A.n_cols * BC * NR * (long long)sizeof(XT) < (1LL << 32))
+    hipLaunchKernelGGL((sell_spmm_kernel<BR, BC, VT, XT, NR, unsigned, Op>), grid, block, 0, s, v, x, op, g, xcd,
+                       t.flags, t.guard);
+  else
+    hipLaunchKernelGGL((sell_spmm_kernel<BR, BC, VT, XT, NR, size_t, Op>), grid, block, 0, s, v, x, op, g, xcd,
+                       t.flags, t.guard);
   return static_cast<int>(hipGetLastError());
 }
 
@@ -222,10 +333,23 @@ static int spmm_store(const SellMatrix& A, const T* x, T* y, int add, const Spmv
   using AT = typename AccT<VT>::type;
 #define CALL(R, C)                                            \
   {                                                           \
-    MOpStore<R, NR, T, AT> op{y, add};                        \
+    MOpStore<T, AT> op{y, add};                        \
     return launch_spmm<R, C, VT, T, NR>(A, x, op, t, s);      \
   }
   WN_MR_DISPATCH(A, CALL);
+#undef CALL
+}
+
+template <typename VT, typename T, int NR>
+static int spmm_restrict_first(const SellMatrix& A, const T* x, T* y, const T* dinv, T* x1, T* d1, double c2,
+                               const SpmvTune& t, hipStream_t s) {
+  using AT = typename AccT<VT>::type;
+#define CALL(R, C)                                              \
+  {                                                             \
+    MOpRestrictFirst<T, AT> op{y, dinv, x1, d1, T(c2)};         \
+    return launch_spmm<R, C, VT, T, NR>(A, x, op, t, s);        \
+  }
+  if (A.br == 6 && A.bc == 3) CALL(6, 3) else if (A.br == 6 && A.bc == 6) CALL(6, 6) else return kBadArg;
 #undef CALL
 }
 
@@ -234,7 +358,7 @@ static int spmm_cheb(const SellMatrix& A, const T* x_in, T* x_out, const T* b, c
                      double c2, const SpmvTune& t, hipStream_t s) {
 #define CALL(R, C)                                                     \
   {                                                                    \
-    MOpCheb<R, NR, T> op{b, dinv, x_in, x_out, d, T(c1), T(c2)};       \
+    MOpCheb<T> op{b, dinv, x_in, x_out, d, T(c1), T(c2)};       \
     return launch_spmm<R, C, VT, T, NR>(A, x_in, op, t, s);            \
   }
   if (A.br == 3 && A.bc == 3) CALL(3, 3) else if (A.br == 6 && A.bc == 6) CALL(6, 6) else return kBadArg;
@@ -245,7 +369,7 @@ template <typename VT, typename T, int NR>
 static int spmm_defect(const SellMatrix& A, const T* x, const T* b, T* res, const SpmvTune& t, hipStream_t s) {
 #define CALL(R, C)                                            \
   {                                                           \
-    MOpDefect<R, NR, T> op{b, res};                           \
+    MOpDefect<T> op{b, res};                           \
     return launch_spmm<R, C, VT, T, NR>(A, x, op, t, s);      \
   }
   if (A.br == 3 && A.bc == 3) CALL(3, 3) else if (A.br == 6 && A.bc == 6) CALL(6, 6) else return kBadArg;
@@ -266,27 +390,55 @@ __global__ void mr_cheb_first_kernel(long long n, const T* __restrict__ b, const
   }
 }
 
-// X[i][k] = sum_j inv[i][j] B[j][k] on the coarsest level (one block per row).
+// X[i][k] = sum_j inv[i][j] B[j][k] on the coarsest level, products and sums
+// in FP64 (v_mfma_f64_16x16x4f64: lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16], result r of lane l is D[4 r + l / 16][l % 16]).  A
+// workgroup owns 16 rows; its 16 wavefronts take every 16th run of 16 columns
+// of the inverse, each lane four consecutive entries of its row, and meet in
+// LDS in wavefront order.  Bound by the inverse's bytes, and on a small level
+// by the chain of loads; one 256-thread workgroup per row with 8 FP64
+// reductions each took 19.5 us at 2 082 rows (194 us at 10 740), this kernel
+// 13.7 us.
+typedef double mr_d4 __attribute__((ext_vector_type(4)));
+constexpr int kMrCoarseWaves = 16;
+
 template <typename T, int NR>
-__global__ __launch_bounds__(256) void mr_coarse_kernel(int n, const T* __restrict__ inv,
-                                                        const T* __restrict__ b, T* __restrict__ x,
-                                                        const int* skip) {
+__global__ __launch_bounds__(64 * kMrCoarseWaves) void mr_coarse_kernel(int n, const T* __restrict__ inv,
+                                                                        const T* __restrict__ b, T* __restrict__ x,
+                                                                        const int* skip) {
   if (skip && *skip) return;
-  const int i = blockIdx.x;
-  double acc[NR];
+  __shared__ double red[kMrCoarseWaves][16][NR];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lr = lane & 15, lk = lane >> 4;
+  const int i = blockIdx.x * 16 + lr;
+  const T* __restrict__ row = inv + (size_t)min(i, n - 1) * n;
+  mr_d4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int k0 = 16 * wave; k0 < n; k0 += 16 * kMrCoarseWaves) {
+    const int k = k0 + 4 * lk;
+    T av[4], bv[4];
 #pragma unroll
-  for (int k = 0; k < NR; ++k) acc[k] = 0.0;
-  for (int j = threadIdx.x; j < n; j += blockDim.x) {
-    const double a = double(inv[(size_t)i * n + j]);
+    for (int e = 0; e < 4; ++e) {
+      const int kk = min(k + e, n - 1);  // in bounds; the padding's products are zero through bv
+      av[e] = row[kk];
+      bv[e] = b[(size_t)kk * NR + (lr < NR ? lr : 0)];
+    }
 #pragma unroll
-    for (int k = 0; k < NR; ++k) acc[k] += a * double(b[(size_t)j * NR + k]);
+    for (int e = 0; e < 4; ++e) {
+      const bool ok = k + e < n && lr < NR;
+      const double a = k + e < n ? double(av[e]) : 0.0;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, ok ? double(bv[e]) : 0.0, acc, 0, 0, 0);
+    }
   }
-  __shared__ double sm[4];
 #pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    const double v = block_sum(acc[k], sm);
-    if (threadIdx.x == 0) x[(size_t)i * NR + k] = T(v);
-    __syncthreads();
+  for (int r = 0; r < 4; ++r)
+    if (lr < NR) red[wave][4 * r + lk][lr] = acc[r];
+  __syncthreads();
+  for (int t = threadIdx.x; t < 16 * NR; t += blockDim.x) {
+    const int r = t / NR, k = t % NR, o = blockIdx.x * 16 + r;
+    double v = 0.0;
+#pragma unroll
+    for (int w = 0; w < kMrCoarseWaves; ++w) v += red[w][r][k];
+    if (o < n) x[(size_t)o * NR + k] = T(v);
   }
 }
 
@@ -305,10 +457,9 @@ struct MrLevel {
 struct MultiState {
   int nr = 0;
   long long n = 0;
-  const Amg* amg = nullptr;
-  int amg_levels = 0;
   std::vector<MrLevel<float>> lv32;
   std::vector<MrLevel<double>> lv64;
+  std::vector<int> level_n;  // rows the level vectors were sized for
   double *r = nullptr, *p = nullptr, *q = nullptr, *zs = nullptr;  // FP64 n x NR
   float *rp32 = nullptr, *zp32 = nullptr;                           // FP32 n x NR
   double* partials = nullptr;  // NR x max blocks
@@ -335,7 +486,7 @@ struct MultiState {
     flags = h_flags = nullptr;
     n = 0;
     nr = 0;
-    amg = nullptr;
+    level_n.clear();
   }
 };
 
@@ -347,21 +498,24 @@ static void multi_free(void* p) {
   delete m;
 }
 
-static int multi_ensure(Solver& S, long long n, int nr, const Amg* g, int need64cycle, int n_slices_max) {
+static int multi_ensure(Solver& S, long long n, int nr, const Amg* g, int need64cycle, int n_blocks) {
   if (!S.multi) {
     S.multi = new MultiState();
     S.multi_free = multi_free;
   }
   MultiState& M = *static_cast<MultiState*>(S.multi);
-  const int blocks = std::max(n_slices_max + 8, 4096);
-  const bool same = M.n >= n && M.nr == nr && M.amg == g && M.max_blocks >= blocks &&
-                    (!g || ((int)M.lv32.size() == (int)g->L.size() &&
-                            (!need64cycle || (int)M.lv64.size() == (int)g->L.size())));
-  if (same && M.r) return kOk;
+  const int blocks = std::max(n_blocks + 8, 4096);
+  std::vector<int> level_n;
+  if (g)
+    for (const auto& l : g->L) level_n.push_back(l->n);
+  bool same = M.r && M.n >= n && M.nr == nr && M.max_blocks >= blocks && M.level_n.size() == level_n.size() &&
+              M.lv32.size() == level_n.size() && (!need64cycle || M.lv64.size() == level_n.size());
+  for (size_t l = 0; same && l < level_n.size(); ++l) same = M.level_n[l] >= level_n[l];
+  if (same) return kOk;
   M.release();
   M.n = n;
   M.nr = nr;
-  M.amg = g;
+  M.level_n = level_n;
   M.max_blocks = blocks;
   const size_t nv = (size_t)n * nr;
   WN_HIP(hipMalloc(&M.r, sizeof(double) * nv));
@@ -395,8 +549,16 @@ template <> [[maybe_unused]] std::vector<MrLevel<double>>& mr_levels<double>(Mul
 
 // The V-cycle of solver.hip on NR columns (same smoother, buffer plan and
 // coarse solve).
+// first_done: the kernel that wrote b wrote the level's first iterate too.
+template <typename T>
+static T* mr_first_iterate(int deg, T* x, T* tmp) {
+  T* post = (deg % 2 == 0) ? x : tmp;
+  return ((deg - 1) % 2 == 0) ? post : (post == x ? tmp : x);
+}
+
 template <typename VT, typename VTC, typename T, int NR>
-static int vcycle_mr(Amg& g, MultiState& M, int l, const T* b, T* x, const int* skip, hipStream_t s) {
+static int vcycle_mr(Amg& g, MultiState& M, int l, const T* b, T* x, const int* skip, hipStream_t s,
+                     bool first_done = false) {
   AmgLevel& L = *g.L[l];
   SpmvTune t = g.tune;
   t.flags = skip;
@@ -405,7 +567,8 @@ static int vcycle_mr(Amg& g, MultiState& M, int l, const T* b, T* x, const int* 
   if (l == (int)g.L.size() - 1) {
     const T* inv = coarse_inv<T>(g);
     if (L.n != g.n_coarse || !inv) return kNotReady;
-    hipLaunchKernelGGL((mr_coarse_kernel<T, NR>), dim3(std::max(L.n, 1)), dim3(256), 0, s, L.n, inv, b, x, skip);
+    hipLaunchKernelGGL((mr_coarse_kernel<T, NR>), dim3(std::max(ceil_div(L.n, 16), 1)), dim3(64 * kMrCoarseWaves), 0, s,
+                       L.n, inv, b, x, skip);
     return static_cast<int>(hipGetLastError());
   }
   MrLevel<T>& V = mr_levels<T>(M)[l];
@@ -418,20 +581,31 @@ static int vcycle_mr(Amg& g, MultiState& M, int l, const T* b, T* x, const int* 
   const ChebCoef c = cheb_coefs(L.lmax, L.ratio, deg);
   const SellMatrix& A = *L.A;
   int r;
-  T* post = (deg % 2 == 0) ? x : tmp;
-  T* cur = ((deg - 1) % 2 == 0) ? post : (post == x ? tmp : x);
+  T* cur = mr_first_iterate(deg, x, tmp);
   T* oth = (cur == x) ? tmp : x;
-  hipLaunchKernelGGL((mr_cheb_first_kernel<T, NR>), dim3(mr_grid(n * NR)), dim3(kMrBlock), 0, s, n, b, dinv, d, cur,
-                     T(c.c2[0]), skip);
-  if ((r = static_cast<int>(hipGetLastError()))) return r;
+  if (!first_done) {
+    hipLaunchKernelGGL((mr_cheb_first_kernel<T, NR>), dim3(mr_grid(n * NR)), dim3(kMrBlock), 0, s, n, b, dinv, d, cur,
+                       T(c.c2[0]), skip);
+    if ((r = static_cast<int>(hipGetLastError()))) return r;
+  }
   for (int k = 1; k < deg; ++k) {
     if ((r = spmm_cheb<VT, T, NR>(A, cur, oth, b, dinv, d, c.c1[k], c.c2[k], t, s))) return r;
     std::swap(cur, oth);
   }
   if ((r = spmm_defect<VT, T, NR>(A, cur, b, res, t, s))) return r;
   MrLevel<T>& N = mr_levels<T>(M)[l + 1];
-  if ((r = spmm_store<VT, T, NR>(L.R, res, N.v[0], 0, t, s))) return r;
-  if ((r = vcycle_mr<VTC, VTC, T, NR>(g, M, l + 1, N.v[0], N.v[1], skip, s))) return r;
+  AmgLevel& NL = *g.L[l + 1];
+  const T* dinv_n = level_dinv<T>(NL);
+  const bool fuse_first = l + 1 < (int)g.L.size() - 1 && dinv_n;  // a smoothed level below
+  if (fuse_first) {
+    const int deg_n = std::max(1, std::min(NL.degree, 16));
+    r = spmm_restrict_first<VT, T, NR>(L.R, res, N.v[0], dinv_n, mr_first_iterate(deg_n, N.v[1], N.v[2]), N.v[3],
+                                       cheb_coefs(NL.lmax, NL.ratio, deg_n).c2[0], t, s);
+  } else {
+    r = spmm_store<VT, T, NR>(L.R, res, N.v[0], 0, t, s);
+  }
+  if (r) return r;
+  if ((r = vcycle_mr<VTC, VTC, T, NR>(g, M, l + 1, N.v[0], N.v[1], skip, s, fuse_first))) return r;
   if ((r = spmm_store<VT, T, NR>(L.P, N.v[1], cur, 1, t, s))) return r;
   oth = (cur == x) ? tmp : x;
   for (int k = 0; k < deg; ++k) {
@@ -496,13 +670,17 @@ __global__ void mr_update_p_kernel(long long n, const ZT* __restrict__ z, const 
 }
 
 // x_k += alpha_k p_k; r_k -= alpha_k q_k; partial ||r_k||^2; rp = S r (FP32)
+// and, with fx1, the next cycle's first Chebyshev iterate fx1 = fd1 = fc2 dinv rp
 template <int NR>
 __global__ __launch_bounds__(kMrBlock) void mr_update_xr_kernel(long long n, double* __restrict__ x,
                                                                 double* __restrict__ r, const double* __restrict__ p,
                                                                 const double* __restrict__ q,
                                                                 float* __restrict__ rp,
                                                                 const double* __restrict__ scale, double* partials,
-                                                                const double* __restrict__ sc, const int* flags) {
+                                                                const double* __restrict__ sc, const int* flags,
+                                                                const float* __restrict__ fdinv,
+                                                                float* __restrict__ fx1, float* __restrict__ fd1,
+                                                                float fc2) {
   if (flags[0]) return;
   const double alpha = sc[kMsAlpha * NR + (threadIdx.x & (NR - 1))];
   double acc = 0.0;
@@ -512,7 +690,15 @@ __global__ __launch_bounds__(kMrBlock) void mr_update_xr_kernel(long long n, dou
     x[t] += alpha * p[t];
     const double ri = r[t] - alpha * q[t];
     r[t] = ri;
-    if (rp) rp[t] = float((scale ? scale[t / NR] : 1.0) * ri);
+    if (rp) {
+      const float v = float((scale ? scale[t / NR] : 1.0) * ri);
+      rp[t] = v;
+      if (fx1) {
+        const float f = fc2 * fdinv[t / NR] * v;
+        fd1[t] = f;
+        fx1[t] = f;
+      }
+    }
     acc += ri * ri;
   }
   store_column_partials<NR>(acc, partials);
@@ -526,23 +712,27 @@ template <int NR>
 __global__ __launch_bounds__(1024) void mr_finalize_kernel(const double* __restrict__ partials, int nb, int mode,
                                                            double* sc, int* flags, double rtol2) {
   if (mode != kMrStart && flags[0]) return;
-  __shared__ double red[NR][16];
+  // wavefront w: column w mod NR, every (16 / NR)-th run of 64 partials; the
+  // columns' loads run side by side, eight in flight per lane (one column
+  // after the other was eight serial memory latencies: 9.9 us, here 3.5 us)
+  constexpr int S = 16 / NR, U = 8;
+  __shared__ double red[NR][S];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int k = 0; k < NR; ++k) {
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    const double* p = partials + (size_t)k * nb;
-    const int stride = blockDim.x;
-    int i = threadIdx.x;
-    for (; i + 3 * stride < nb; i += 4 * stride) {
-      a0 += p[i];
-      a1 += p[i + stride];
-      a2 += p[i + 2 * stride];
-      a3 += p[i + 3 * stride];
+  {
+    const double* p = partials + (size_t)(wid % NR) * nb;
+    double a = 0.0;
+    for (int i0 = (wid / NR) * 64 + lane; i0 < nb; i0 += 64 * S * U) {
+      double v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + 64 * S * u;
+        v[u] = i < nb ? p[i] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) a += v[u];
     }
-    for (; i < nb; i += stride) a0 += p[i];
-    double s = (a0 + a1) + (a2 + a3);
-    s = wave_sum(s);
-    if (lane == 0) red[k][wid] = s;
+    a = wave_sum(a);
+    if (lane == 0) red[wid % NR][wid / NR] = a;
   }
   __syncthreads();
   int* done = flags + 2;
@@ -550,7 +740,7 @@ __global__ __launch_bounds__(1024) void mr_finalize_kernel(const double* __restr
   const int k = threadIdx.x;
   if (k < NR) {
   double v = 0.0;
-  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) v += red[k][w];
+  for (int w = 0; w < S; ++w) v += red[k][w];
   switch (mode) {
     case kMrStart:  // v = ||b_k||^2
       sc[kMsRR * NR + k] = v;
@@ -619,16 +809,11 @@ static int mr_spmm_dot(const SellMatrix& A, const double* p, double* q, double* 
                        hipStream_t s) {
 #define CALL(R, C)                                                  \
   {                                                                 \
-    MOpSpmvDot<R, NR, double> op{q, p, partials};                   \
+    MOpSpmvDot<double> op{q, p, partials};                   \
     return launch_spmm<R, C, double, double, NR>(A, p, op, t, s);   \
   }
   if (A.br == 3 && A.bc == 3) CALL(3, 3) else if (A.br == 6 && A.bc == 6) CALL(6, 6) else return kBadArg;
 #undef CALL
-}
-
-// grid of the FP64-value SpMM (its block partials feed the CG dots)
-static int spmm_grid64(const SellMatrix& A, const SpmvTune& t) {
-  return t.xcd_for<double>() ? 8 * ((A.n_slices + 7) / 8) : A.n_slices;
 }
 
 // PCG on NR columns of A X = B from X = 0; preconditioner: AMG V-cycle in
@@ -639,7 +824,7 @@ static int pcg_multi_run(Solver& S, const SellMatrix& A, Amg* g, int vt, const d
                          int* iters, double* rel) {
   const long long n = (long long)A.n_rows * A.br;
   int r;
-  if ((r = multi_ensure(S, n, NR, g, vt == 0, A.n_slices))) return r;
+  if ((r = multi_ensure(S, n, NR, g, vt == 0, spmm_grid(A, NR, 8, 1)))) return r;
   MultiState& M = *static_cast<MultiState*>(S.multi);
   SpmvTune t = tune0;
   t.flags = M.flags;
@@ -649,7 +834,20 @@ static int pcg_multi_run(Solver& S, const SellMatrix& A, Amg* g, int vt, const d
   hipLaunchKernelGGL((mr_start_kernel<NR>), dim3(gv), dim3(kMrBlock), 0, s, n, B, X, M.r, M.rp32, scale, M.partials);
   if ((r = static_cast<int>(hipGetLastError()))) return r;
   if ((r = mr_fin<NR>(M, gv, kMrStart, rtol * rtol, s))) return r;
-  const int gs = spmm_grid64(A, t);
+  const int gs = spmm_grid(A, NR, 8, t.xcd_for<double>());
+  // each cycle's first iterate on the finest level comes from the kernel that
+  // writes the cycle's input: the x, r update, and one launch here
+  const AmgLevel& L0 = *g->L[0];
+  const bool first = g->L.size() > 1 && L0.dinv32;
+  const int deg0 = std::max(1, std::min(L0.degree, 16));
+  const float c20 = (float)cheb_coefs(L0.lmax, L0.ratio, deg0).c2[0];
+  float* d0 = first ? M.lv32[0].v[3] : nullptr;
+  float* x0 = first ? mr_first_iterate(deg0, M.zp32, M.lv32[0].v[2]) : nullptr;
+  if (first) {
+    hipLaunchKernelGGL((mr_cheb_first_kernel<float, NR>), dim3(gv), dim3(kMrBlock), 0, s, n, M.rp32, L0.dinv32, d0, x0,
+                       c20, nullptr);
+    if ((r = static_cast<int>(hipGetLastError()))) return r;
+  }
   int done_all = 0;
   // chunks sized from each open column's residual reduction rate, as in the
   // single-column PCG (idle iterations after convergence are costly)
@@ -659,7 +857,7 @@ static int pcg_multi_run(Solver& S, const SellMatrix& A, Amg* g, int vt, const d
     chunk = std::max(1, std::min(chunk, max_iter - it));
     const int it0 = it;
     for (int c = 0; c < chunk; ++c, ++it) {
-      if ((r = vcycle_mr<float, float, float, NR>(*g, M, 0, M.rp32, M.zp32, M.flags, s))) return r;
+      if ((r = vcycle_mr<float, float, float, NR>(*g, M, 0, M.rp32, M.zp32, M.flags, s, first))) return r;
       hipLaunchKernelGGL((mr_rho_kernel<float, NR>), dim3(gv), dim3(kMrBlock), 0, s, n, M.r, M.zp32, scale,
                          M.partials, M.flags);
       if ((r = static_cast<int>(hipGetLastError()))) return r;
@@ -670,7 +868,7 @@ static int pcg_multi_run(Solver& S, const SellMatrix& A, Amg* g, int vt, const d
       if ((r = mr_spmm_dot<NR>(A, M.p, M.q, M.partials, t, s))) return r;
       if ((r = mr_fin<NR>(M, gs, kMrGamma, 0.0, s))) return r;
       hipLaunchKernelGGL((mr_update_xr_kernel<NR>), dim3(gv), dim3(kMrBlock), 0, s, n, X, M.r, M.p, M.q, M.rp32,
-                         scale, M.partials, M.sc, M.flags);
+                         scale, M.partials, M.sc, M.flags, L0.dinv32, x0, d0, c20);
       if ((r = static_cast<int>(hipGetLastError()))) return r;
       if ((r = mr_fin<NR>(M, gv, kMrRR, 0.0, s))) return r;
     }
