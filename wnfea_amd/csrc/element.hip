@@ -735,6 +735,68 @@ __device__ __forceinline__ void gauss_point_consts(int g, T (&c4)[4], T (&cc)[4]
   }
 }
 
+// The edge between vertices v and v ^ m of a tetrahedron, as its midside node
+// (Abaqus order): kEdgeOf[v][m - 1].
+__host__ __device__ constexpr int kEdgeOf[4][3] = {{4, 6, 7}, {4, 8, 5}, {9, 6, 5}, {9, 8, 7}};
+
+// The element forces of an affine element by vertices instead of Gauss points:
+// its strain is linear, so the strains at the four vertices determine it, and
+// the integral of B^T D B (a quadratic, which the 4-point rule integrates
+// exactly) is V/20 (1 + delta_vw) over pairs of vertex values.  One quad of
+// lanes per element, lane v at vertex v; k = v ^ m (m = 1, 2, 3) names the
+// other vertices, so every exchange is one fixed quad permutation.
+//   du/dx at v = sum_m grad L_k (x) (Q_k - Q_v),  Q_k - Q_v =
+//     -u_k + 4 u_vk - 3 u_v = (u_vk - u_k) + 3 (u_vk - u_v)
+//   T_v = V/20 (S_v + sum_w S_w),  R_k = T_v grad L_k
+//   f_v  = -3 sum_m R_k(v) - sum_m R_v(k)
+//   f_vk = 4 (R_k(v) + R_v(k)),  R_v(k) from lane k by the permutation
+// u: own vertex; ue[m - 1]: edge (v, k); g: grad L_v in lanes 1..3 (lane 0
+// takes minus their sum); lam, mu: Lame moduli times 4 V/20 = 0.8 (det J / 24).
+// Out: fv the vertex's force, fe[m - 1] the edges' (both lanes of an edge hold
+// it).  About 175 FP32 operations per lane and four nodal values, against 400
+// and ten at a Gauss point.
+template <typename T>
+__device__ __forceinline__ void vertex_forces(int v, const T (&u)[3], const T (&ue)[3][3], const T (&graw)[3], T lam,
+                                              T mu, T (&fv)[3], T (&fe)[3][3]) {
+  T gk[3][3], D[3][3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const T r = v == 0 ? T(0) : graw[c], s = quad_sum(r), own = v == 0 ? -s : r;
+    gk[0][c] = quad_perm<0xB1>(own);
+    gk[1][c] = quad_perm<0x4E>(own);
+    gk[2][c] = quad_perm<0x1B>(own);
+    const T uk[3] = {quad_perm<0xB1>(u[c]), quad_perm<0x4E>(u[c]), quad_perm<0x1B>(u[c])};
+#pragma unroll
+    for (int m = 0; m < 3; ++m) D[m][c] = (ue[m][c] - uk[m]) + T(3) * (ue[m][c] - u[c]);
+  }
+  T H[3][3];  // H[r][c] = du_c / dx_r
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) H[r][c] = gk[0][r] * D[0][c] + gk[1][r] * D[1][c] + gk[2][r] * D[2][c];
+  const T lt = lam * (H[0][0] + H[1][1] + H[2][2]), mu2 = mu + mu;
+  T S[6] = {mu2 * H[0][0] + lt,        mu2 * H[1][1] + lt,        mu2 * H[2][2] + lt,
+            mu * (H[1][0] + H[0][1]), mu * (H[2][1] + H[1][2]), mu * (H[2][0] + H[0][2])};
+#pragma unroll
+  for (int k = 0; k < 6; ++k) S[k] += quad_sum(S[k]);
+  T sr[3] = {T(0), T(0), T(0)}, st[3] = {T(0), T(0), T(0)};
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const T R[3] = {S[0] * gk[m][0] + S[3] * gk[m][1] + S[5] * gk[m][2],
+                    S[3] * gk[m][0] + S[1] * gk[m][1] + S[4] * gk[m][2],
+                    S[5] * gk[m][0] + S[4] * gk[m][1] + S[2] * gk[m][2]};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const T t = m == 0 ? quad_perm<0xB1>(R[c]) : m == 1 ? quad_perm<0x4E>(R[c]) : quad_perm<0x1B>(R[c]);
+      sr[c] += R[c];
+      st[c] += t;
+      fe[m][c] = R[c] + t;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) fv[c] = -(T(0.75) * sr[c] + T(0.25) * st[c]);
+}
+
 // fe = K_e (sc .* u)_e from the quadrature data, stored [i][e][3] for local
 // node i, where sc is a per-DOF scaling that also carries the Dirichlet rule
 // (0 on a fixed DOF: its column of the operator is zero).  Four lanes per
@@ -1034,26 +1096,30 @@ __global__ __launch_bounds__(64 * kGatherWaves) void mf_gather_op_kernel(
 // One workgroup of 4 P lanes per patch of P consecutive element slots
 // (elements sorted along a Morton curve, so a patch is a compact piece of the
 // mesh), one quad of lanes per element (lane g: Gauss point g):
-//  1. loads addressed by the patch index alone are issued first: each
-//     element's 16-bit local connectivity and quadrature data, the patch's
-//     slot codes (into LDS) and its local nodes' global ids and list starts
-//     (fixed stride per patch); then those addressed through them: the
-//     scaled nodal values sc .* U of the local nodes (into LDS, four entries
-//     per node; up to three nodes per lane, loads issued together) and,
-//     unfolded, the element moduli;
-//  2. each quad computes its element's forces as c3d10_pa_elem_kernel does,
-//     every lane reading the element's ten nodal values from LDS, and keeps
-//     them in LDS;
+//  1. loads addressed by the patch index alone are issued first: each lane's
+//     four 16-bit local nodes (its vertex and that vertex's three edges, 8
+//     bytes), its part of the element's record, the patch's slot codes (into
+//     LDS) and its local nodes' global ids and list starts (fixed stride per
+//     patch); then those addressed through them: the scaled nodal values
+//     sc .* U of the local nodes (into LDS, four entries per node; up to NS
+//     nodes per lane, loads issued together) and, unfolded, the element moduli;
+//  2. each quad computes its element's forces (vertex_forces, lane v at vertex
+//     v, four nodal values per lane read from LDS) and keeps them in LDS;
 //  3. each local node adds its element forces in slot order (slot codes
 //     ascending, from LDS) and writes the sum to its partial slot
 //     p stride + j (contiguous per patch).
-// The quadrature data is one record per slot: Ji and det J / 24 ([M][10],
-// the moduli read through the slot's element id), or Folded, Ji and the
-// weighted moduli w c11, w c12, w c44 ([M][12], made when a smoother is
-// attached).
+// The record per slot is the gradients of L_1, L_2, L_3 after det J / 24
+// ([M][10], the moduli read through the slot's element id), or Folded, after
+// lambda, mu times 0.8 det J / 24 and a pad ([M][12], made when a smoother is
+// attached): lane v > 0 reads its own gradient, lane 0 the rest.
 // The element forces never leave the chip; a node interior to a patch has a
 // single partial, a node on a patch boundary one per patch that touches it.
-constexpr int kStageSlots = 3;  // local nodes per lane in step 1: 3 * 4 P >= the stride
+// Bound: latency (two dependent load levels, two barriers and the slot lists
+// of the corner nodes) and the gathers of the nodal values.  Lanes at the
+// Gauss points needed 444 VALU instructions and ten 16-byte LDS reads each in
+// FP32 (581 and 88 VGPRs in FP64; here 33 and 60 VGPRs), and the slot lists
+// were walked one entry at a time: I-beam, 208 800 elements, FP32 11.1 ->
+// 10.7 us, FP64 17.4 -> 15.7 us; 3 840 elements, 5.5 -> 4.5 us and 6.2 -> 5.3 us.
 
 __device__ __forceinline__ void lds_node(const float* xs, int li, float (&u)[3]) {
   const float4 v = *reinterpret_cast<const float4*>(xs + 4 * li);
@@ -1075,19 +1141,36 @@ __device__ __forceinline__ void lds_store_node(double* xs, int j, const double (
   xs[4 * j + 2] = v[2];
 }
 
-template <typename T, int P, bool Folded>
+// Entries per element force in LDS: FP32 padded to 16 bytes (one LDS
+// instruction per force), FP64 packed (a fifth workgroup fits the CU).
+template <typename T>
+__host__ __device__ constexpr int force_stride() {
+  return sizeof(T) == 4 ? 4 : 3;
+}
+__device__ __forceinline__ void lds_store_force(float* fl, int i, const float (&v)[3]) { lds_store_node(fl, i, v); }
+__device__ __forceinline__ void lds_store_force(double* fl, int i, const double (&v)[3]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) fl[3 * i + c] = v[c];
+}
+__device__ __forceinline__ void lds_force(const float* fl, int i, float (&v)[3]) { lds_node(fl, i, v); }
+__device__ __forceinline__ void lds_force(const double* fl, int i, double (&v)[3]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) v[c] = fl[3 * i + c];
+}
+
+template <typename T, int P, int NS, bool Folded>
 __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
-    int n_patch, int M, int stride, const int* __restrict__ pnode, const unsigned short* __restrict__ pconn,
-    const unsigned short* __restrict__ poff, const unsigned short* __restrict__ pslot, const int* __restrict__ pe,
+    int n_patch, int M, int stride, const int* __restrict__ pnode, const ushort4* __restrict__ pconn,
+    const unsigned short* __restrict__ poff, const uint2* __restrict__ pslot, const int* __restrict__ pe,
     const T* __restrict__ qdp, const double* __restrict__ E, const double* __restrict__ nu,
     const T* __restrict__ sc, const T* __restrict__ U, T* __restrict__ part, const int* skip) {
-  constexpr int NT = 4 * P;
+  constexpr int NT = 4 * P, FS = force_stride<T>(), NC = 10 * P / 4;  // NC: 8-byte runs of slot codes
   if (skip && *skip) return;
   extern __shared__ __align__(16) unsigned char patch_lds[];
-  T* xs = reinterpret_cast<T*>(patch_lds);                              // [stride][4] scaled nodal values
-  T* fl = xs + 4 * stride;                                               // [P][10][3] element forces
-  unsigned short* ls = reinterpret_cast<unsigned short*>(fl + 30 * P);  // [10 P] slot codes
-  unsigned short* lo = ls + 10 * P;                                       // [stride] list starts
+  T* xs = reinterpret_cast<T*>(patch_lds);                                    // [stride][4] scaled nodal values
+  T* fl = xs + 4 * stride;                                                     // [P][10][FS] element forces
+  unsigned short* ls = reinterpret_cast<unsigned short*>(fl + 10 * FS * P);  // [10 P] slot codes
+  unsigned short* lo = ls + 10 * P;                                            // [stride] list starts
   const int p = slice_of_block(n_patch, 1);  // XCD-contiguous patch ranges
   if (p >= n_patch) return;
   const int t = (int)threadIdx.x;
@@ -1097,49 +1180,26 @@ __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
   const int e0 = p * P, ne = min(P, M - e0);
   const size_t pb = (size_t)p * stride;
   // step 1, first round: addressed by the patch index
-  const int el = t >> 2, g = t & 3;
+  const int el = t >> 2, v = t & 3;
   const bool live = el < ne;
   const unsigned su = (unsigned)(e0 + (live ? el : 0));  // clamped: the loads stay unconditional
-  int lc[10];
+  const ushort4 lc = pconn[4 * su + v];
+  // this lane's three entries of the slot's record
+  T rec[3];
   {
-    const unsigned short* pc = pconn + (size_t)su * 10;
+    const T* q = qdp + (Folded ? 12 * su + 3 * v : 10 * su + (v == 0 ? 0 : 3 * v - 2));
 #pragma unroll
-    for (int i = 0; i < 10; ++i) lc[i] = pc[i];
+    for (int c = 0; c < 3; ++c) rec[c] = q[c];
   }
-  // the slot's quadrature record: 16-byte aligned (48 B folded FP32, 80 B FP64)
-  constexpr int QW = Folded ? 12 : 10;
-  T qv[QW];
-  {
-    const T* q = qdp + (size_t)su * QW;
-#pragma unroll
-    for (int k = 0; k < QW; ++k) qv[k] = q[k];
-  }
-  T Ji[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) Ji[k] = qv[k];
-  T w11 = T(0), w12 = T(0), w44 = T(0), wd = T(0);
   int ee = 0;
-  if constexpr (Folded) {
-    w11 = qv[QW - 3];
-    w12 = qv[QW - 2];
-    w44 = qv[QW - 1];
-  } else {
-    wd = qv[9];
-    ee = pe[su];
-  }
-  const unsigned short* psl = pslot + (size_t)e0 * 10;
-  unsigned short code[3];  // slot codes t, t + NT, t + 2 NT (10 P < 3 NT)
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const unsigned q = (unsigned)(t + k * NT);
-    code[k] = psl[q < (unsigned)(10 * ne) ? q : 0u];
-  }
+  if constexpr (!Folded) ee = pe[su];
+  const uint2 code = pslot[(size_t)p * NC + min(t, NC - 1)];
   const int* pn = pnode + pb;
   const unsigned short* po = poff + pb;
-  int gn[kStageSlots];
-  unsigned short off[kStageSlots];
+  int gn[NS];
+  unsigned short off[NS];
 #pragma unroll
-  for (int k = 0; k < kStageSlots; ++k) {
+  for (int k = 0; k < NS; ++k) {
     const unsigned j = (unsigned)min(t + k * NT, stride - 1);
     gn[k] = pn[j];
     off[k] = po[j];
@@ -1150,20 +1210,18 @@ __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
     Ev = E[ee];
     nv = nu[ee];
   }
-  T xv[kStageSlots][3];
+  T xv[NS][3];
 #pragma unroll
-  for (int k = 0; k < kStageSlots; ++k) {
+  for (int k = 0; k < NS; ++k) {
     const size_t n3 = 3 * (size_t)max(gn[k], 0);
     const T* uk = U + n3;
     const T* sk = sc + n3;
 #pragma unroll
     for (int c = 0; c < 3; ++c) xv[k][c] = uk[c] * sk[c];
   }
+  if (t < NC) reinterpret_cast<uint2*>(ls)[t] = code;
 #pragma unroll
-  for (int k = 0; k < 3; ++k)
-    if (t + k * NT < 10 * ne) ls[t + k * NT] = code[k];
-#pragma unroll
-  for (int k = 0; k < kStageSlots; ++k) {
+  for (int k = 0; k < NS; ++k) {
     const int j = t + k * NT;
     if (j < stride) {
       lo[j] = off[k];
@@ -1172,60 +1230,75 @@ __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
   }
   __syncthreads();
   // step 2: the element forces
-  if constexpr (!Folded) weighted_moduli<T>(wd, Ev, nv, w11, w12, w44);
-  T c4[4], cc[4];
-  gauss_point_consts<T>(g, c4, cc);
-  T out[3][3];
-  pa_forces<T>(g, c4, cc, Ji, w11, w12, w44, [&](int i, T (&u)[3]) { lds_node(xs, lc[i], u); }, out);
-  if (live) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int i = g + 4 * j;
-      if (i < 10) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) fl[(el * 10 + i) * 3 + c] = out[j][c];
-      }
+  T lam, mu;
+  if constexpr (Folded) {
+    lam = quad_bcast_c<0>(rec[0]);
+    mu = quad_bcast_c<0>(rec[1]);
+  } else {
+    const T w = T(0.8) * quad_bcast_c<0>(rec[0]);
+    lam = w * T(Ev * nv / ((1.0 + nv) * (1.0 - 2.0 * nv)));
+    mu = w * T(Ev / (2.0 * (1.0 + nv)));
+  }
+  {
+    T u[3], ue[3][3], fv[3], fe[3][3];
+    lds_node(xs, lc.x, u);
+    lds_node(xs, lc.y, ue[0]);
+    lds_node(xs, lc.z, ue[1]);
+    lds_node(xs, lc.w, ue[2]);
+    vertex_forces<T>(v, u, ue, rec, lam, mu, fv, fe);
+    if (live) {
+      // of the two lanes of an edge one stores its force
+      const int f0 = el * 10;
+      lds_store_force(fl, f0 + v, fv);
+      if (!(v & 1)) lds_store_force(fl, f0 + (v == 0 ? 4 : 9), fe[0]);
+      if (v == 0 || v == 3) lds_store_force(fl, f0 + (v == 0 ? 6 : 8), fe[1]);
+      if (v & 1) lds_store_force(fl, f0 + (v == 1 ? 5 : 7), fe[2]);
     }
   }
   __syncthreads();
   // step 3: per local node, its element forces in slot order (the entry
-  // after the last node holds the end of its list)
+  // after the last node holds the end of its list), four at a time: a corner
+  // node has up to 24 in a patch, each two LDS latencies when added one by one
 #pragma unroll
-  for (int k = 0; k < kStageSlots; ++k) {
+  for (int k = 0; k < NS; ++k) {
     const int j = t + k * NT;
     if (j < stride && gn[k] >= 0) {
       const int o0 = lo[j], o1 = lo[j + 1];
-      T a0 = T(0), a1 = T(0), a2 = T(0);
-      for (int q = o0; q < o1; ++q) {
-        const int f = 3 * ls[q];
-        a0 += fl[f];
-        a1 += fl[f + 1];
-        a2 += fl[f + 2];
+      T a[3] = {T(0), T(0), T(0)};
+      for (int q = o0; q < o1; q += 4) {
+        int c[4];
+        T f[4][3];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] = ls[min(q + i, o1 - 1)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lds_force(fl, c[i], f[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) a[d] += q + i < o1 ? f[i][d] : T(0);
       }
       T* o = part + pb * 3;
       const unsigned j3 = 3u * (unsigned)j;
-      o[j3] = a0;
-      o[j3 + 1] = a1;
-      o[j3 + 2] = a2;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) o[j3 + d] = a[d];
     }
   }
 }
 
-// Folded FP32 quadrature records of the patch layout: per slot the rounded
-// inverse Jacobian and w c11, w c12, w c44 (formed in FP64 from the slot's
-// element moduli), [M][12].
+// Folded FP32 records of the patch layout: per slot lambda and mu times 0.8
+// det J / 24 (formed in FP64 from the slot's element moduli), a pad and the
+// rounded gradients of L_1, L_2, L_3, [M][12].
 __global__ void qdata_fold_kernel(int M, const int* __restrict__ pe, const double* __restrict__ qdp,
                                   const double* __restrict__ E, const double* __restrict__ nu,
                                   float* __restrict__ out) {
   for (int sl = blockIdx.x * blockDim.x + threadIdx.x; sl < M; sl += gridDim.x * blockDim.x) {
     const double* q = qdp + (size_t)sl * 10;
     float* o = out + (size_t)sl * 12;
-    for (int k = 0; k < 9; ++k) o[k] = (float)q[k];
-    const double wd = q[9], Ev = E[pe[sl]], nv = nu[pe[sl]];
-    const double f = Ev / ((1.0 + nv) * (1.0 - 2.0 * nv));
-    o[9] = (float)(wd * f * (1.0 - nv));
-    o[10] = (float)(wd * f * nv);
-    o[11] = (float)(wd * Ev / (2.0 * (1.0 + nv)));
+    const double w = 0.8 * q[0], Ev = E[pe[sl]], nv = nu[pe[sl]];
+    o[0] = (float)(w * (Ev * nv / ((1.0 + nv) * (1.0 - 2.0 * nv))));
+    o[1] = (float)(w * (Ev / (2.0 * (1.0 + nv))));
+    o[2] = 0.0f;
+    for (int k = 0; k < 9; ++k) o[3 + k] = (float)q[1 + k];
   }
 }
 
@@ -1330,13 +1403,16 @@ struct OpMfMode {
   }
 };
 
-// qdp[s][k] = qd[k][pe[s]] (affine quadrature data as one record per slot)
+// The FP64 record of slot s: det J / 24, then the gradients of L_1, L_2, L_3
+// (grad L_{a+1}[r] = J^-1[r][a]), from the affine quadrature data
+// qd[3 r + a][e], qd[9][e] of its element e = pe[s].
 __global__ void qdata_permute_kernel(int M, const int* __restrict__ pe, const double* __restrict__ qd,
                                      double* __restrict__ qdp) {
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < 10LL * M;
        i += (long long)gridDim.x * blockDim.x) {
-    const long long sl = i / 10, k = i % 10;
-    qdp[i] = qd[k * M + pe[sl]];
+    const long long sl = i / 10;
+    const int k = (int)(i % 10), from = k == 0 ? 9 : 3 * ((k - 1) % 3) + (k - 1) / 3;
+    qdp[i] = qd[(long long)from * M + pe[sl]];
   }
 }
 
@@ -1420,10 +1496,12 @@ static void mf_patch_release(MfOp& op) {
 
 // LDS of one patch workgroup: staged nodal values and element forces
 static size_t patch_lds_bytes(const MfOp& op, size_t elem) {
-  return (4 * (size_t)op.stride + 30 * (size_t)op.patch) * elem + 2 * (10 * (size_t)op.patch + (size_t)op.stride);
+  const size_t fs = elem == sizeof(float) ? force_stride<float>() : force_stride<double>();
+  return (4 * (size_t)op.stride + 10 * fs * op.patch) * elem + 2 * (10 * (size_t)op.patch + (size_t)op.stride);
 }
 constexpr size_t kPatchLdsMax = 64 * 1024;
 constexpr int kDefaultPatch = 64;
+constexpr int kStageSlots = 3;  // most local nodes a lane stages: 3 * 4 P >= the stride
 
 int mf_set_patch(MfOp& op, int elems, hipStream_t s) {
   if (elems < 0 || elems > 256 || elems % 64) return kBadArg;
@@ -1459,6 +1537,16 @@ int mf_set_patch(MfOp& op, int elems, hipStream_t s) {
     return kBadArg;
   }
   novf.resize((size_t)std::max<long long>(nov, 1));
+  // per lane of a slot's quad: its vertex and that vertex's three edges
+  std::vector<unsigned short> lconn((size_t)M * 16);
+  for (size_t sl = 0; sl < (size_t)M; ++sl)
+    for (int v = 0; v < 4; ++v) {
+      const unsigned short* c = pconn.data() + sl * 10;
+      unsigned short* o = lconn.data() + sl * 16 + 4 * v;
+      o[0] = c[v];
+      for (int m = 0; m < 3; ++m) o[1 + m] = c[kEdgeOf[v][m]];
+    }
+  pslot.resize((size_t)op.n_patch * P * 10, 0);  // whole patches: the last one's codes are read in full
   auto up = [&](auto*& dst, const auto& v) -> int {
     using E = typename std::decay_t<decltype(v)>::value_type;
     WN_HIP(hipMalloc(&dst, sizeof(E) * std::max<size_t>(v.size(), 1)));
@@ -1466,7 +1554,7 @@ int mf_set_patch(MfOp& op, int elems, hipStream_t s) {
     return kOk;
   };
   int r;
-  if ((r = up(op.pe, order)) || (r = up(op.pnode, pnode)) || (r = up(op.pconn, pconn)) || (r = up(op.poff, poff)) ||
+  if ((r = up(op.pe, order)) || (r = up(op.pnode, pnode)) || (r = up(op.pconn, lconn)) || (r = up(op.poff, poff)) ||
       (r = up(op.pslot, pslot)) || (r = up(op.nhead, nhead)) || (r = up(op.novf, novf))) {
     mf_patch_release(op);
     return r;
@@ -1566,9 +1654,12 @@ static void launch_patch(const MfOp& op, const T* qdp, const T* sc, const T* U, 
                          hipStream_t s) {
   const dim3 grid(patch_grid(op.n_patch));
   const size_t lds = patch_lds_bytes(op, sizeof(T));
+#define WN_PATCH_LAUNCH1(PP, NS)                                                                                    \
+  hipLaunchKernelGGL((mf_patch_kernel<T, PP, NS, Folded>), grid, dim3(4 * (PP)), lds, s, op.n_patch, op.M,          \
+                     op.stride, op.pnode, reinterpret_cast<const ushort4*>(op.pconn), op.poff,                      \
+                     reinterpret_cast<const uint2*>(op.pslot), op.pe, qdp, op.E, op.nu, sc, U, part, skip)
 #define WN_PATCH_LAUNCH(PP)                                                                                         \
-  hipLaunchKernelGGL((mf_patch_kernel<T, PP, Folded>), grid, dim3(4 * (PP)), lds, s, op.n_patch, op.M, op.stride,   \
-                     op.pnode, op.pconn, op.poff, op.pslot, op.pe, qdp, op.E, op.nu, sc, U, part, skip)
+  if (op.stride <= 8 * (PP)) WN_PATCH_LAUNCH1(PP, 2); else WN_PATCH_LAUNCH1(PP, kStageSlots)
   switch (op.patch) {
     case 64: WN_PATCH_LAUNCH(64); break;
     case 128: WN_PATCH_LAUNCH(128); break;
@@ -1576,6 +1667,7 @@ static void launch_patch(const MfOp& op, const T* qdp, const T* sc, const T* U, 
     default: WN_PATCH_LAUNCH(256); break;
   }
 #undef WN_PATCH_LAUNCH
+#undef WN_PATCH_LAUNCH1
 }
 
 // blocks of the per-element path's node gather, padded to a multiple of the 8 XCDs

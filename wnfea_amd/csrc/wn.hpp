@@ -112,12 +112,12 @@ struct MfOp {
   int gen = 0;                           // layout generation: smoothers built on another one fall back
   int* pe = nullptr;                     // [M] element of each slot
   int* pnode = nullptr;                  // [n_patch][stride] global node of each local node (-1: none)
-  unsigned short* pconn = nullptr;       // [M][10] local node of each element corner
+  unsigned short* pconn = nullptr;       // [M][4][4] local nodes of each vertex v and its edges to v ^ 1, v ^ 2, v ^ 3
   unsigned short* poff = nullptr;        // [n_patch][stride] start of the local node's slot list (patch-relative)
-  unsigned short* pslot = nullptr;       // [M][10] per patch: the local nodes' slot lists (slot = 10 e + corner)
+  unsigned short* pslot = nullptr;       // [n_patch * patch][10] per patch: the local nodes' slot lists (slot = 10 e + corner)
   int4* nhead = nullptr;                 // [n_nodes] first three partial slots and the count (or overflow)
   int* novf = nullptr;                   // overflow lists of nodes with more than three partials
-  double* qdp = nullptr;                 // [M][10] affine quadrature data, one record per slot
+  double* qdp = nullptr;                 // [M][10] per slot det J / 24 and the gradients of L_1, L_2, L_3
   double* part = nullptr;                // [n_patch * stride][3]
   std::vector<int> order;                // host: elements in Morton order of their centroids
 };
@@ -134,7 +134,7 @@ struct MfSmooth {
   float* s32e = nullptr;
   float* qd32 = nullptr;  // rounded copy of the operator's qd (same layout)
   float* fe32 = nullptr;  // [10][M][3]
-  float* qdp32 = nullptr;   // [M][12] patch layout: rounded inverse Jacobians and w c11, w c12, w c44
+  float* qdp32 = nullptr;   // [M][12] patch layout: weighted lambda, mu, a pad and the rounded gradients
   float* part32 = nullptr;  // [n_patch * stride][3]
   int gen = -1;             // the operator's layout generation the copies were made for
 };
