@@ -464,6 +464,17 @@ int wnfea_pcg_multi(void *solver, void *bsr, void *amg, int amg_vt, const double
  * (wnfea/solver/native/hip_kernels.cpp:2975,3032). */
 int wnfea_bsr_spmm(void *h, int prec, int nrhs, const void *X, void *Y, void *stream);
 
+
+/* out[g] = the sum over the nodes of group g of (a - b)^2, FP64, in a fixed
+ * order (b may be NULL = 0; dpn values per node; all arrays device).  The
+ * nodes of all groups are listed in perm, cut into n_chunks chunks that each
+ * lie in one group: chunk c is perm[chunk[c]] .. perm[chunk[c + 1]] (chunk has
+ * n_chunks + 1 entries), group g holds chunks cptr[g] .. cptr[g + 1];
+ * partials has room for n_chunks values.  No reference counterpart (it solves
+ * one model at a time, wnfea/solver/solid_solver.py:132-194); it serves the
+ * per-mesh residuals of a batch. */
+int wnfea_group_norms2(int n_groups, int n_chunks, int dpn, const int *cptr, const int *chunk, const int *perm,
+                       const double *a, const double *b, double *partials, double *out, void *stream);
 /* r = f - K u (FP64; r may be NULL) and out[0] = ||r||, out[1] = ||f||. */
 int wnfea_residual(void *solver, void *bsr, const double *u, const double *f, double *r, double *out, void *stream);
 

@@ -77,6 +77,7 @@ SIGNATURES = {
     "wnfea_solver_set_graphs": (_i, [_p, _i]),
     "wnfea_pcg": (_i, [_p, _p, _i, _i, _p, _p, _i, _p, _p, _p, _d, _i, _i, _pi, _pd, _p]),
     "wnfea_ir": (_i, [_p, _p, _p, _i, _p, _p, _i, _p, _p, _d, _d, _i, _i, _i, _i, _pi, _pi, _pd, _p]),
+    "wnfea_group_norms2": (_i, [_i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p]),
     "wnfea_residual": (_i, [_p, _p, _p, _p, _p, _pd, _p]),
     "wnfea_mf_create": (_i, [_i, _i, _p, _p, _p, _p, _p, _p, _p, _p, ctypes.POINTER(_p), _p]),
     "wnfea_mf_destroy": (None, [_p]),

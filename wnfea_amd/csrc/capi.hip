@@ -610,6 +610,12 @@ int wnfea_mf_apply(void* h, const double* u, double* y, void* stream) {
   return mf_apply(static_cast<WnMf*>(h)->op, u, nullptr, y, nullptr, 0, nullptr, 0, S(stream));
 }
 
+int wnfea_group_norms2(int n_groups, int n_chunks, int dpn, const int* cptr, const int* chunk, const int* perm,
+                       const double* a, const double* b, double* partials, double* out, void* stream) {
+  if (n_groups < 0 || n_chunks < 0 || dpn <= 0 || !cptr || !chunk || !perm || !a || !partials || !out) return kBadArg;
+  return launch_group_norms2(n_groups, n_chunks, dpn, cptr, chunk, perm, a, b, partials, out, S(stream));
+}
+
 // r = f - K u and out[0] = ||r||, out[1] = ||f|| (as wnfea_residual, matrix-free)
 int wnfea_mf_residual(void* solver, void* h, const double* u, const double* f, double* r, double* out, void* stream) {
   if (!solver || !h || !u || !f || !r || !out) return kBadArg;

@@ -202,6 +202,8 @@ int launch_adjoint_dot(int M, const int* conn, const double* E, const double* fe
 
 // -------- vector kernels (blas.hip)
 int vec_grid(long long n);
+int launch_group_norms2(int n_groups, int n_chunks, int dpn, const int* cptr, const int* chunk, const int* perm,
+                        const double* a, const double* b, double* partials, double* out, hipStream_t s);
 // one-block finalisation of block partials (FinMode in common.hpp)
 int launch_finalize(const double* partials, int nb, int K, int mode, double* out, double* sc, int* flags, int first,
                     const int* skip, hipStream_t s);

@@ -23,6 +23,7 @@ import time
 
 import numpy as np
 
+from .. import _lib
 from ..model import FEAModel
 
 
@@ -109,11 +110,31 @@ class BatchedSolids:
         self.timings = {"assembly_sec": t1 - t0, "amg_setup_sec": time.perf_counter() - t1}
         import torch
         dev = self.system.K.device
-        self._owner = torch.as_tensor(np.repeat(self.owner_host, 3), device=dev)
         self.n_meshes = len(models)
-        f2 = torch.zeros(self.n_meshes, dtype=torch.float64, device=dev)
-        f2.index_add_(0, self._owner, self.system.F * self.system.F)
-        self.f_norms = torch.sqrt(f2)
+        # nodes by mesh, cut into chunks of one mesh each (wnfea_group_norms2)
+        counts = np.bincount(self.owner_host, minlength=self.n_meshes)
+        n_chunks = -(-counts // self._CHUNK)
+        starts = np.concatenate([[0], np.cumsum(counts)])
+        chunk = np.concatenate([starts[k] + self._CHUNK * np.arange(n_chunks[k]) for k in range(self.n_meshes)]
+                               + [starts[-1:]])
+        t = lambda a: torch.as_tensor(np.ascontiguousarray(a, dtype=np.int32), device=dev)  # noqa: E731
+        self._groups = (t(np.concatenate([[0], np.cumsum(n_chunks)])), t(chunk),
+                        t(np.argsort(self.owner_host, kind="stable")))
+        self.f_norms = self._mesh_norms(self.system.F)
+
+    _CHUNK = 1024  # nodes per workgroup of the per-mesh norms
+
+    def _mesh_norms(self, a, b=None):
+        """||a_k - b_k|| of every mesh (device FP64; b defaults to zero)."""
+        import torch
+        cptr, chunk, perm = self._groups
+        n_chunks = len(chunk) - 1
+        part = torch.empty(max(n_chunks, 1), dtype=torch.float64, device=a.device)
+        out = torch.empty(self.n_meshes, dtype=torch.float64, device=a.device)
+        _lib.check(_lib.load().wnfea_group_norms2(self.n_meshes, n_chunks, 3, _lib.dptr(cptr), _lib.dptr(chunk),
+                                                  _lib.dptr(perm), _lib.dptr(a.contiguous()), _lib.dptr(b), _lib.dptr(part),
+                                                  _lib.dptr(out), _lib.stream_of()), "wnfea_group_norms2")
+        return torch.sqrt(out)
 
     def close(self):
         self.amg.close()
@@ -124,10 +145,8 @@ class BatchedSolids:
     def per_mesh_residuals(self, u):
         """||f_k - K_k u_k|| / ||f_k|| for every mesh (device FP64 residual)."""
         import torch
-        r = self.system.F - self.system.K.spmv(u)
-        r2 = torch.zeros(self.n_meshes, dtype=torch.float64, device=u.device)
-        r2.index_add_(0, self._owner, r * r)
-        return (torch.sqrt(r2) / torch.where(self.f_norms > 0, self.f_norms, torch.ones_like(self.f_norms)))
+        r = self._mesh_norms(self.system.F, self.system.K.spmv(u))
+        return r / torch.where(self.f_norms > 0, self.f_norms, torch.ones_like(self.f_norms))
 
     def solve(self, tol: float = 1e-8):
         """All meshes to tol (FP64-verified per mesh).  Returns (u in the merged
