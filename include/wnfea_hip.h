@@ -157,7 +157,8 @@ int wnfea_adjoint_grad(int M, const int *conn, const double *nodes, const double
 
 /* Co-rotational internal forces of 2-node beams, FP64, deterministic.
  * conn[M][2], nodes[N][3], props[M][6] = (E, G, A, Iy, Iz, J), U[N][6]
- * (device); fe_work[M][12] device scratch; n2e_ptr/n2e the node incidence
+ * (device); fe_work[M][12] device scratch (required, not used: the element
+ * forces stay on the chip); n2e_ptr/n2e the node incidence
  * (wnfea_node_incidence with npe = 2); F[N][6] (accumulate != 0 adds).
  * Replaces hip_compute_beam_forces (wnfea/solver/native/hip_kernels.cpp:53-241),
  * compute_corotational_element_forces (wnfea/solver/corotational_beam.py:178-233)
@@ -464,7 +465,6 @@ int wnfea_pcg_multi(void *solver, void *bsr, void *amg, int amg_vt, const double
  * (wnfea/solver/native/hip_kernels.cpp:2975,3032). */
 int wnfea_bsr_spmm(void *h, int prec, int nrhs, const void *X, void *Y, void *stream);
 
-
 /* out[g] = the sum over the nodes of group g of (a - b)^2, FP64, in a fixed
  * order (b may be NULL = 0; dpn values per node; all arrays device).  The
  * nodes of all groups are listed in perm, cut into n_chunks chunks that each
@@ -475,6 +475,7 @@ int wnfea_bsr_spmm(void *h, int prec, int nrhs, const void *X, void *Y, void *st
  * per-mesh residuals of a batch. */
 int wnfea_group_norms2(int n_groups, int n_chunks, int dpn, const int *cptr, const int *chunk, const int *perm,
                        const double *a, const double *b, double *partials, double *out, void *stream);
+
 /* r = f - K u (FP64; r may be NULL) and out[0] = ||r||, out[1] = ||f||. */
 int wnfea_residual(void *solver, void *bsr, const double *u, const double *f, double *r, double *out, void *stream);
 

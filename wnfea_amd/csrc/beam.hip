@@ -13,13 +13,14 @@
 //   elongation u_l = (2 v0.du + du.du)/(L + L0); local rotations
 //   th_y = r2.theta + r3.du/L, th_z = r3.theta - r2.du/L, th_x = r1.(theta2 -
 //   theta1); q = (N, My1, Mz1, Tx, My2, Mz2) of the linear beam; f = B^T q.
-// One thread per element (the element is ~300 flops with transcendental
-// functions; no reuse between elements), forces per element in fe[M][12],
-// then a deterministic per-node gather (no atomics).
+// One thread per (node, element at it), which computes the element's forces
+// and keeps its own end's; the node's ends are added in element order in LDS
+// (no atomics, no element forces in memory).
 //
 // The linear stiffness follows build_element_stiffness_3d_beam and
 // build_transformation_matrix (wnfea/solver/assembler.py:13-148), including
 // its axis-aligned frame rules.
+#include <algorithm>
 #include <type_traits>
 #include "common.hpp"
 
@@ -118,9 +119,7 @@ __host__ __device__ void corot_force(const BeamGeom& g, const S* u, S* f) {
   const V3 ref = fabs(e1.z) < 0.9 ? v3<double>(0.0, 0.0, 1.0) : v3<double>(0.0, 1.0, 0.0);
   V3 e2d = cross(ref, e1);
   e2d = (1.0 / norm(e2d)) * e2d;
-  V3 e3d = cross(e1, e2d);
-  e3d = (1.0 / norm(e3d)) * e3d;
-  const V3T<S> e2 = lift<S>(e2d), e3 = lift<S>(e3d), E1 = lift<S>(e1);
+  const V3T<S> e2 = lift<S>(e2d), E1 = lift<S>(e1);
   const V3T<S> u1 = v3<S>(u[0], u[1], u[2]), th1 = v3<S>(u[3], u[4], u[5]);
   const V3T<S> u2 = v3<S>(u[6], u[7], u[8]), th2 = v3<S>(u[9], u[10], u[11]);
   const V3T<S> du = u2 - u1;
@@ -129,20 +128,17 @@ __host__ __device__ void corot_force(const BeamGeom& g, const S* u, S* f) {
   V3T<S> r1 = (S(1.0) / (val(L) > 1e-15 ? L : S(1e-15))) * v;
   const V3T<S> cr = cross(E1, r1);
   const S cphi = dot(E1, r1);
-  V3T<S> r2 = e2, r3 = e3;
+  V3T<S> r2 = e2, r3;  // r3 follows from r1 x r2 after the twist
   if constexpr (std::is_same<S, double>::value) {
     const double sphi = norm(cr);
     if (sphi > 1e-12) {
+      // cos(phi) and sin(phi) are cphi and sphi themselves (unit vectors): sin(phi) a = cr
       const V3 ax = (1.0 / sphi) * cr;
-      const double phi = atan2(sphi, cphi);
-      const double cp = cos(phi), sp = sin(phi);
-      r2 = cp * e2 + sp * cross(ax, e2) + (dot(ax, e2) * (1.0 - cp)) * ax;
-      r3 = cp * e3 + sp * cross(ax, e3) + (dot(ax, e3) * (1.0 - cp)) * ax;
+      r2 = cphi * e2 + cross(cr, e2) + (dot(ax, e2) * (1.0 - cphi)) * ax;
     }
   } else {
     const S k = S(1.0) / (S(1.0) + cphi);
     r2 = cphi * e2 + cross(cr, e2) + (dot(cr, e2) * k) * cr;
-    r3 = cphi * e3 + cross(cr, e3) + (dot(cr, e3) * k) * cr;
   }
   const S tw = S(0.5) * dot(th1 + th2, r1);
   const S ct = cos(tw), st = sin(tw);
@@ -150,7 +146,7 @@ __host__ __device__ void corot_force(const BeamGeom& g, const S* u, S* f) {
   r1 = (S(1.0) / norm(r1)) * r1;
   r2 = r2t - dot(r2t, r1) * r1;
   r2 = (S(1.0) / norm(r2)) * r2;
-  r3 = cross(r1, r2);  // the reference recomputes r3 from r1 x r2 after the twist
+  r3 = cross(r1, r2);
   r3 = (S(1.0) / norm(r3)) * r3;
   const V3T<S> V0 = lift<S>(v0);
   const S ul = (S(2.0) * dot(V0, du) + dot(du, du)) / (L + S(L0));
@@ -193,17 +189,50 @@ __device__ __forceinline__ void load_u(int e, const int* __restrict__ conn, cons
   }
 }
 
-__global__ void beam_force_kernel(int M, const int* __restrict__ conn, const double* __restrict__ nodes,
-                                  const double* __restrict__ props, const double* __restrict__ U,
-                                  double* __restrict__ fe) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= M) return;
-  const BeamGeom g = load_geom(e, conn, nodes, props);
-  double u[12], f[12];
-  load_u(e, conn, U, u);
-  corot_force<double>(g, u, f);
+// F[n] (+)= the sum of the element forces at node n's end of the elements at
+// it (incidence codes e * 2 + local, in element order).  A workgroup owns
+// `nodes_per_block` consecutive nodes and takes their incidences
+// kForceThreads at a time, one per thread, into LDS; thread k < nodes_per_block
+// then adds node k's of them in order.  Each element is computed by both its
+// nodes: one thread per element with the forces in memory and a gather were
+// two chains of latencies at 1-3 wavefronts per SIMD, and its rotation took an
+// arc tangent, a sine and a cosine of it (12^3 cells, 6 084 beams, a forces
+// call with its zero fill 18.9 us, here without one 11.7 us).
+constexpr int kForceThreads = 256;
+
+__global__ __launch_bounds__(kForceThreads) void beam_node_force_kernel(
+    int n_nodes, int nodes_per_block, const int* __restrict__ conn, const double* __restrict__ nodes,
+    const double* __restrict__ props, const double* __restrict__ U, const int* __restrict__ n2e_ptr,
+    const int* __restrict__ n2e, double* __restrict__ F, int accumulate) {
+  __shared__ double sf[kForceThreads][6];
+  const int t = (int)threadIdx.x;
+  const int n0 = blockIdx.x * nodes_per_block, n1 = min(n0 + nodes_per_block, n_nodes);
+  const int n = n0 + t;
+  const bool owns = t < nodes_per_block && n < n1;
+  const int k0 = n2e_ptr[n0], k1 = n2e_ptr[n1];
+  const int own0 = owns ? n2e_ptr[n] : 0, own1 = owns ? n2e_ptr[n + 1] : 0;
+  double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int base = k0; base < k1; base += kForceThreads) {
+    const int k = base + t;
+    if (k < k1) {
+      const int code = n2e[k], e = code >> 1;
+      const BeamGeom g = load_geom(e, conn, nodes, props);
+      double u[12], f[12];
+      load_u(e, conn, U, u);
+      corot_force<double>(g, u, f);
 #pragma unroll
-  for (int k = 0; k < 12; ++k) fe[12 * (size_t)e + k] = f[k];
+      for (int c = 0; c < 6; ++c) sf[t][c] = code & 1 ? f[6 + c] : f[c];
+    }
+    __syncthreads();
+    for (int q = max(own0, base); q < min(own1, base + kForceThreads); ++q)
+#pragma unroll
+      for (int c = 0; c < 6; ++c) s[c] += sf[q - base][c];
+    __syncthreads();
+  }
+  if (!owns) return;
+  double* o = F + 6 * (size_t)n;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) o[c] = accumulate ? o[c] + s[c] : s[c];
 }
 
 // Column j of the element tangent d f / d u_j, one thread per (element,
@@ -332,35 +361,14 @@ __global__ void beam_ke_linear_kernel(int M, const int* __restrict__ conn, const
   }
 }
 
-// out[n][0..5] (+)= sum of the element forces of the elements at node n
-// (incidence codes e*2 + local, in element order).
-__global__ void gather6_kernel(int n_nodes, const int* __restrict__ n2e_ptr, const int* __restrict__ n2e,
-                               const double* __restrict__ fe, double* __restrict__ out, int accumulate) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= n_nodes) return;
-  double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int k = n2e_ptr[n]; k < n2e_ptr[n + 1]; ++k) {
-    const int code = n2e[k];
-    const double* p = fe + 12 * (size_t)(code >> 1) + 6 * (code & 1);
-#pragma unroll
-    for (int c = 0; c < 6; ++c) s[c] += p[c];
-  }
-  double* o = out + 6 * (size_t)n;
-#pragma unroll
-  for (int c = 0; c < 6; ++c) o[c] = accumulate ? o[c] + s[c] : s[c];
-}
-
 int launch_beam_forces(int M, int n_nodes, const int* conn, const double* nodes, const double* props,
-                       const double* U, const int* n2e_ptr, const int* n2e, double* fe, double* F, int accumulate,
-                       hipStream_t s) {
-  if (M > 0) {
-    hipLaunchKernelGGL(beam_force_kernel, dim3(ceil_div(M, 128)), dim3(128), 0, s, M, conn, nodes, props, U, fe);
-    const int e = static_cast<int>(hipGetLastError());
-    if (e) return e;
-  }
+                       const double* U, const int* n2e_ptr, const int* n2e, double* F, int accumulate, hipStream_t s) {
   if (n_nodes <= 0) return kOk;
-  hipLaunchKernelGGL(gather6_kernel, dim3(ceil_div(n_nodes, 256)), dim3(256), 0, s, n_nodes, n2e_ptr, n2e, fe, F,
-                     accumulate);
+  // nodes whose incidences (two per element) fill a workgroup on average
+  long long per = M > 0 ? (long long)kForceThreads * n_nodes / (2LL * M) : kForceThreads;
+  const int npb = (int)std::min<long long>(std::max<long long>(per, 1), kForceThreads);
+  hipLaunchKernelGGL(beam_node_force_kernel, dim3(ceil_div(n_nodes, npb)), dim3(kForceThreads), 0, s, n_nodes, npb,
+                     conn, nodes, props, U, n2e_ptr, n2e, F, accumulate);
   return static_cast<int>(hipGetLastError());
 }
 

@@ -155,7 +155,7 @@ int wnfea_beam_forces(int M, int n_nodes, const int* conn, const double* nodes, 
   if (M < 0 || n_nodes < 0) return kBadArg;
   if (M > 0 && (!conn || !nodes || !props || !U || !fe_work)) return kBadArg;
   if (n_nodes > 0 && (!n2e_ptr || !n2e || !F)) return kBadArg;
-  return launch_beam_forces(M, n_nodes, conn, nodes, props, U, n2e_ptr, n2e, fe_work, F, accumulate, S(stream));
+  return launch_beam_forces(M, n_nodes, conn, nodes, props, U, n2e_ptr, n2e, F, accumulate, S(stream));
 }
 
 int wnfea_beam_tangent(int M, const int* conn, const double* nodes, const double* props, const double* U,

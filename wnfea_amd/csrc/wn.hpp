@@ -191,8 +191,7 @@ int launch_stress(int M, const int* conn, const double* nodes, const double* E, 
 int launch_nodal_average(int n_nodes, const int* n2e_ptr, const int* n2e, const double* cell_vm, double* nodal_vm,
                          hipStream_t s);
 int launch_beam_forces(int M, int n_nodes, const int* conn, const double* nodes, const double* props,
-                       const double* U, const int* n2e_ptr, const int* n2e, double* fe, double* F, int accumulate,
-                       hipStream_t s);
+                       const double* U, const int* n2e_ptr, const int* n2e, double* F, int accumulate, hipStream_t s);
 int launch_beam_tangent(int M, const int* conn, const double* nodes, const double* props, const double* U,
                         double h_rel, double* Kt, hipStream_t s);
 int launch_beam_ke_linear(int M, const int* conn, const double* nodes, const double* props, double* Ke,
@@ -202,9 +201,9 @@ int launch_adjoint_dot(int M, const int* conn, const double* E, const double* fe
 
 // -------- vector kernels (blas.hip)
 int vec_grid(long long n);
+// one-block finalisation of block partials (FinMode in common.hpp)
 int launch_group_norms2(int n_groups, int n_chunks, int dpn, const int* cptr, const int* chunk, const int* perm,
                         const double* a, const double* b, double* partials, double* out, hipStream_t s);
-// one-block finalisation of block partials (FinMode in common.hpp)
 int launch_finalize(const double* partials, int nb, int K, int mode, double* out, double* sc, int* flags, int first,
                     const int* skip, hipStream_t s);
 template <typename T> int launch_fill(long long n, T* x, T v, hipStream_t s);

@@ -103,7 +103,9 @@ class _ForceContext:
         """F_int (device, 6 per node) of device U (6 per node)."""
         import torch
         L = _lib.load()
-        F = torch.zeros(6 * self.n, dtype=torch.float64, device=U.device)
+        # the beams' kernel writes every node; without beams the solids add to zeros
+        make = torch.zeros if self.beams is None else torch.empty
+        F = make(6 * self.n, dtype=torch.float64, device=U.device)
         acc = 0
         if self.beams is not None:
             b = self.beams
