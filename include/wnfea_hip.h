@@ -329,6 +329,25 @@ int wnfea_bsr_get_values(void *h, double *vals_std, void *stream);
 int wnfea_bsr_assemble(void *h, const int *rowidx, const int *colidx, const long long *cptr, const int *codes,
                        const double *Ke, const unsigned char *node_fix, double *vals_std, void *stream);
 
+/* Element records of a C3D10 mesh for wnfea_bsr_assemble_affine: rec[M][16]
+ * (device, 16-byte aligned) gets the four barycentric gradients and the
+ * weighted Lame moduli of each element taken as affine.  flags[2] (device
+ * int, zeroed by the caller): flags[0] = e + 1 of an element whose corners
+ * have det J <= 0, flags[1] = 1 when some element is not affine (midside nodes
+ * off the edge midpoints by more than 1e-12 of the element); the records of
+ * such a mesh do not describe it.  With wnfea_bsr_assemble_affine it replaces
+ * the element stiffness loop and COO summation of assemble_c3d10_sparse_3dof
+ * (wnfea/solver/solid_solver.py:62-127) where every element is affine. */
+int wnfea_c3d10_affine_records(int M, const int *conn, const double *nodes, const double *E, const double *nu,
+                               double *rec, int *flags, void *stream);
+
+/* FP64 values of the 3x3-block matrix h from element records and the
+ * contribution lists (codes e*100 + a*10 + b), with the Dirichlet rule of
+ * wnfea_bsr_assemble: the same blocks to FP64 rounding, exactly symmetric,
+ * without element matrices. */
+int wnfea_bsr_assemble_affine(void *h, const long long *cptr, const int *codes, const double *rec,
+                              const unsigned char *node_fix, void *stream);
+
 /* Element matrices Ke[M][npe*b][npe*b] of b x b-block matrix h (b = 3 or 6)
  * through the contribution lists (codes e*npe*npe + a*npe + c); sym != 0
  * assembles 0.5 (Ke + Ke^T); node_fix bits as wnfea_bsr_assemble (bit c =

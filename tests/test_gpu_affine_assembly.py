@@ -1,0 +1,108 @@
+"""Assembly from affine element records and the layout-ordered value kernels:
+against the element-matrix path, the CPU oracle and plain index arithmetic."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(kind):
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_ibeam, generate_c3d10_structured_block
+    if kind == "cell":
+        m, _ = generate_c3d10_structured_block(0.1, 0.2, 0.3, 1, 1, 1, tets_per_hex=6)
+    elif kind == "five":  # mirrored neighbours, uneven sides
+        m, _ = generate_c3d10_structured_block(1.0, 0.1, 0.3, 7, 2, 3, tets_per_hex=5)
+    else:
+        m, _ = generate_c3d10_ibeam(n_layers=3, length=0.03)
+    rng = np.random.default_rng(5)
+    M = len(m.solid_elements)
+    m.solid_E, m.solid_nu = rng.uniform(1e9, 3e11, M), rng.uniform(0.0, 0.45, M)
+    return m
+
+
+@pytest.mark.parametrize("bcs", [True, False])
+@pytest.mark.parametrize("kind", ["cell", "five", "ibeam", "curved"])
+def test_assembly_paths_agree(kind, bcs):
+    import torch
+    from oracle import oracle as O
+    from wnfea_amd import _lib
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr, reassemble_c3d10_values
+    m = _model("five" if kind == "curved" else kind)
+    if kind == "curved":
+        X, mid = m.mesh_nodes, np.unique(m.solid_elements[:, 4:])
+        X[mid] += 1e-3 * np.sin(37 * X[mid][:, [1, 2, 0]])
+    s = assemble_c3d10_bsr(m, apply_bcs=bcs, keep_plan=True)
+    K = s.K.get_values()
+    Ko = None
+    if bcs:
+        Ko, _ = O.assemble_csr(m.mesh_nodes, m.solid_elements, m.solid_E, m.solid_nu, m.fixed_dof_mask(3),
+                               m.load_vector(3))
+    L, mesh, plan = _lib.load(), s.mesh, s.mesh["plan"]
+    M = mesh["n_elements"]
+    Ke = torch.empty((M, 30, 30), dtype=torch.float64, device="cuda")
+    bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+    std = torch.full_like(K, float("nan"))
+    _lib.check(L.wnfea_c3d10_ke(M, *[_lib.dptr(mesh[k]) for k in ("conn", "nodes", "E", "nu")], _lib.dptr(Ke),
+                                _lib.dptr(bad), _lib.stream_of()), "ke")
+    _lib.check(L.wnfea_bsr_assemble(s.K.handle, _lib.dptr(s.K.d_rowidx), _lib.dptr(s.K.d_colidx),
+                                    _lib.dptr(plan["cptr"]), _lib.dptr(plan["codes"]), _lib.dptr(Ke),
+                                    _lib.dptr(plan["fix"]), _lib.dptr(std), _lib.stream_of()), "assemble")
+    # the layout's values read back are the ones written in standard order
+    assert torch.equal(s.K.get_values(), std)
+    # gradients carry the coordinates' rounding, eps L / h <= 1e-13 here, twice
+    tol = 1e-12 * float(std.abs().max())
+    assert float((K - std).abs().max()) <= tol
+    if Ko is not None:
+        D = (s.K.to_scipy_bsr(K).tocsr() - Ko).tocoo()
+        assert np.abs(D.data).max(initial=0.0) <= tol
+    if kind != "curved":  # exactly symmetric
+        A = s.K.to_scipy_bsr(K).tocsr()
+        assert (A != A.T).nnz == 0
+    # new moduli: K is linear in E
+    reassemble_c3d10_values(s, E=2.0 * mesh["E"])
+    free = (~torch.as_tensor(s.fixed_mask, device="cuda")).view(-1, 3)
+    both = (free[s.K.d_rowidx.long()][:, :, None] & free[s.K.d_colidx.long()][:, None, :]).view(-1, 9)
+    assert float((s.K.get_values() - 2.0 * K)[both].abs().max()) <= 2.0 * tol
+
+
+def test_inverted_affine_element_is_refused():
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr
+    m = _model("five")
+    T = m.solid_elements
+    T[3] = T[3][[0, 2, 1, 3, 6, 5, 4, 7, 9, 8]]  # mirrored, still affine
+    with pytest.raises(ValueError, match="Non-positive Jacobian determinant in C3D10 element 3"):
+        assemble_c3d10_bsr(m)
+
+
+@pytest.mark.parametrize("b,lanes", [(3, 1), (3, 4), (3, 64), (6, 2), (6, 16), (2, 4)])
+def test_equilibrated_copies(b, lanes):
+    import torch
+    from wnfea_amd import _lib
+    from wnfea_amd.solver.bsr_matrix import DeviceBSR
+    rng = np.random.default_rng([b, lanes])
+    n = 131
+    count = rng.integers(0, 30, n)
+    cols = [np.sort(rng.choice(n, c, replace=False)) for c in count]
+    rowptr = np.concatenate([[0], np.cumsum(count)]).astype(np.int32)
+    A = DeviceBSR(b, b, n, n, rowptr, np.concatenate(cols).astype(np.int32), lanes=lanes)
+    vals = torch.as_tensor(rng.standard_normal((A.nnzb, b * b)), device="cuda")
+    A.set_values(vals, 1)
+    assert torch.equal(A.get_values(), vals)
+    S = torch.as_tensor(rng.uniform(0.5, 2.0, n * b), device="cuda")
+    L = _lib.load()
+    _lib.check(L.wnfea_bsr_equilibrate(A.handle, _lib.dptr(A.d_rowidx), _lib.dptr(A.d_colidx), _lib.dptr(S), 1, 1,
+                                       _lib.stream_of()), "equilibrate")
+    info = A.info()
+    assert info["has_fp32"] and info["has_fp64_equilibrated"] and info["has_fp16"]
+    if b == 2:
+        return  # no product kernels for this block size
+    r, c = A.d_rowidx.long(), A.d_colidx.long()
+    E = (S.view(-1, b)[r][:, :, None] * vals.view(-1, b, b)) * S.view(-1, b)[c][:, None, :]
+    import scipy.sparse as sp
+    x = rng.standard_normal(n * b)
+    for prec, V, eps in (("fp64_equilibrated", E, 2.3e-16), ("fp32", E.float().double(), 1.2e-7)):
+        xd = torch.as_tensor(x, device="cuda").to(torch.float32 if prec == "fp32" else torch.float64)
+        M = sp.bsr_matrix((V.cpu().numpy(), A.colidx, A.rowptr), shape=A.shape)
+        xr = xd.double().cpu().numpy()
+        err = np.abs(A.spmv(xd, precision=prec).double().cpu().numpy() - M @ xr)
+        assert np.all(err <= 30 * b * eps * (abs(M) @ np.abs(xr)))  # at most 30 b products per row

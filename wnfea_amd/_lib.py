@@ -58,6 +58,8 @@ SIGNATURES = {
     "wnfea_bsr_set_values": (_i, [_p, _p, _i, _p]),
     "wnfea_bsr_get_values": (_i, [_p, _p, _p]),
     "wnfea_bsr_assemble": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _p]),
+    "wnfea_c3d10_affine_records": (_i, [_i, _p, _p, _p, _p, _p, _p, _p]),
+    "wnfea_bsr_assemble_affine": (_i, [_p, _p, _p, _p, _p, _p]),
     "wnfea_bsr_diag": (_i, [_p, _p, _p, _p]),
     "wnfea_bsr_equilibrate": (_i, [_p, _p, _p, _p, _i, _i, _p]),
     "wnfea_bsr_spmv": (_i, [_p, _i, _p, _p, _d, _d, _p]),

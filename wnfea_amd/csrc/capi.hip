@@ -330,15 +330,30 @@ int wnfea_bsr_assemble(void* h, const int* rowidx, const int* colidx, const long
   if (!h) return kBadArg;
   auto* b = static_cast<WnBsr*>(h);
   if (b->m.nnzb > 0 && (!rowidx || !colidx || !cptr || !codes || !Ke)) return kBadArg;
-  return assemble_gather(b->m, rowidx, colidx, cptr, codes, Ke, node_fix, vals_std, S(stream));
+  return b->m.br == 3 ? assemble_elem(b->m, 10, 0, cptr, codes, Ke, node_fix, vals_std, S(stream)) : kBadArg;
 }
 
 int wnfea_bsr_assemble_elem(void* h, int npe, int sym, const int* rowidx, const int* colidx, const long long* cptr,
                             const int* codes, const double* Ke, const unsigned char* node_fix, double* vals_std,
                             void* stream) {
   if (!h || !rowidx || !colidx || !cptr || !codes || !Ke) return kBadArg;
-  return assemble_elem(static_cast<WnBsr*>(h)->m, npe, sym, rowidx, colidx, cptr, codes, Ke, node_fix, vals_std,
-                       S(stream));
+  return assemble_elem(static_cast<WnBsr*>(h)->m, npe, sym, cptr, codes, Ke, node_fix, vals_std, S(stream));
+}
+
+int wnfea_c3d10_affine_records(int M, const int* conn, const double* nodes, const double* E, const double* nu,
+                               double* rec, int* flags, void* stream) {
+  if (M < 0 || !flags || (M > 0 && (!conn || !nodes || !E || !nu || !rec)) ||
+      (reinterpret_cast<uintptr_t>(rec) & 15))
+    return kBadArg;
+  return affine_records(M, conn, nodes, E, nu, rec, flags, S(stream));
+}
+
+int wnfea_bsr_assemble_affine(void* h, const long long* cptr, const int* codes, const double* rec,
+                              const unsigned char* node_fix, void* stream) {
+  if (!h) return kBadArg;
+  auto* b = static_cast<WnBsr*>(h);
+  if (b->m.nnzb > 0 && (!cptr || !codes || !rec || (reinterpret_cast<uintptr_t>(rec) & 15))) return kBadArg;
+  return assemble_affine(b->m, cptr, codes, rec, node_fix, S(stream));
 }
 
 int wnfea_bsr_diag(void* h, const long long* diag_block, double* diag, void* stream) {

@@ -29,7 +29,7 @@ void SellMatrix::release() {
     delete eq_alias;  // non-owning view: nothing of its own to free
     eq_alias = nullptr;
   }
-  for (void* p : {(void*)d_off, (void*)d_rinfo, (void*)d_col, (void*)d_slot, (void*)d_v64, (void*)d_v64e,
+  for (void* p : {(void*)d_off, (void*)d_rinfo, (void*)d_col, (void*)d_slot, (void*)d_rstart, (void*)d_v64, (void*)d_v64e,
                   (void*)d_v32, (void*)d_v16})
     if (p) (void)hipFree(p);
   d_v16 = nullptr;
@@ -37,6 +37,7 @@ void SellMatrix::release() {
   d_rinfo = nullptr;
   d_col = nullptr;
   d_slot = nullptr;
+  d_rstart = nullptr;
   d_v64 = nullptr;
   d_v64e = nullptr;
   d_v32 = nullptr;
@@ -49,7 +50,7 @@ SellMatrix& SellMatrix::equilibrated() {
   a.br = br; a.bc = bc; a.n_rows = n_rows; a.n_cols = n_cols; a.n_slices = n_slices; a.sigma = sigma;
   a.lanes = lanes;
   a.nnzb = nnzb; a.slots = slots; a.d_off = d_off; a.d_rinfo = d_rinfo; a.d_col = d_col;
-  a.d_slot = d_slot; a.d_v64 = d_v64e; a.d_v64e = nullptr; a.d_v32 = d_v32; a.d_v16 = d_v16;
+  a.d_slot = d_slot; a.d_rstart = d_rstart; a.d_v64 = d_v64e; a.d_v64e = nullptr; a.d_v32 = d_v32; a.d_v16 = d_v16;
   return a;
 }
 
@@ -108,6 +109,7 @@ int SellMatrix::build(int br_, int bc_, int n_rows_, int n_cols_, const int* row
   }
   std::vector<long long> off(n_slices + 1, 0);
   std::vector<int2> rinfo((size_t)n_slices * rows_per_slice, make_int2(-1, 0));
+  std::vector<int> rstart(rinfo.size() + 1, 0);
   for (int s = 0; s < n_slices; ++s) {
     int steps = 0;
     for (int r = 0; r < rows_per_slice; ++r) {
@@ -116,6 +118,7 @@ int SellMatrix::build(int br_, int bc_, int n_rows_, int n_cols_, const int* row
       const int g = order[k];
       const int rl = rowptr[g + 1] - rowptr[g];
       rinfo[(size_t)k] = make_int2(g, rl);
+      rstart[(size_t)k] = rowptr[g];
       steps = std::max(steps, (rl + lanes - 1) / lanes);  // sub-lane 0 has the most steps
     }
     off[s + 1] = off[s] + 64LL * steps;
@@ -140,6 +143,8 @@ int SellMatrix::build(int br_, int bc_, int n_rows_, int n_cols_, const int* row
   WN_HIP(hipMalloc(&d_rinfo, sizeof(int2) * rinfo.size()));
   WN_HIP(hipMalloc(&d_col, sizeof(int) * col.size()));
   WN_HIP(hipMalloc(&d_slot, sizeof(long long) * slot.size()));
+  WN_HIP(hipMalloc(&d_rstart, sizeof(int) * rstart.size()));
+  WN_HIP(hipMemcpy(d_rstart, rstart.data(), sizeof(int) * rstart.size(), hipMemcpyHostToDevice));
   WN_HIP(hipMemcpy(d_off, off.data(), sizeof(long long) * off.size(), hipMemcpyHostToDevice));
   WN_HIP(hipMemcpy(d_rinfo, rinfo.data(), sizeof(int2) * rinfo.size(), hipMemcpyHostToDevice));
   WN_HIP(hipMemcpy(d_col, col.data(), sizeof(int) * col.size(), hipMemcpyHostToDevice));
@@ -201,119 +206,12 @@ int sell_to_std(const SellMatrix& A, double* vals_std, hipStream_t s) {
   if (!A.d_v64) return kNotReady;
   const long long n = A.nnzb * A.br * A.bc;
   if (n == 0) return kOk;
+  if ((A.br == 3 || A.br == 6) && (A.bc == 3 || A.bc == 6)) {
+    launch_to_std_slots(A, vals_std, s);
+    return static_cast<int>(hipGetLastError());
+  }
   hipLaunchKernelGGL(sell_to_std_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, A.nnzb, A.br * A.bc, A.d_slot,
                      A.d_v64, vals_std);
-  return static_cast<int>(hipGetLastError());
-}
-
-// Deterministic assembly of 3x3 blocks.  Block k = (i, j) sums the entries of
-// its contributions in list order (element order, then local pair order), each
-// code = e*100 + a*10 + b addressing Ke[e][3a+r][3b+c].  Dirichlet semantics of
-// solid_solver.py:95-127 per scalar entry: a fixed row or column DOF zeroes the
-// entry, and the diagonal entry of a fixed DOF becomes 1.  node_fix[n] holds the
-// fixed-DOF bits of node n (bit c = DOF c fixed).
-__global__ void assemble_gather_kernel(long long nnzb, const int* __restrict__ rowidx, const int* __restrict__ colidx,
-                                       const long long* __restrict__ cptr, const int* __restrict__ codes,
-                                       const double* __restrict__ Ke, const unsigned char* __restrict__ node_fix,
-                                       const long long* __restrict__ slot, double* __restrict__ v64,
-                                       double* __restrict__ vstd) {
-  const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (k >= nnzb) return;
-  double acc[9] = {};
-  for (long long q = cptr[k]; q < cptr[k + 1]; ++q) {
-    const int code = codes[q];
-    const int e = code / 100, ab = code - e * 100, a = ab / 10, b = ab - a * 10;
-    const double* kp = Ke + (size_t)e * 900 + (3 * a) * 30 + 3 * b;
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) acc[r * 3 + c] += kp[r * 30 + c];
-  }
-  const int i = rowidx[k], j = colidx[k];
-  const unsigned fi = node_fix ? node_fix[i] : 0u, fj = node_fix ? node_fix[j] : 0u;
-  const long long sl = slot[k];
-#pragma unroll
-  for (int r = 0; r < 3; ++r)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      double v = acc[r * 3 + c];
-      if (((fi >> r) & 1u) || ((fj >> c) & 1u)) v = (i == j && r == c) ? 1.0 : 0.0;
-      v64[val_index<double>(sl, r * 3 + c, 9)] = v;
-      if (vstd) vstd[k * 9 + r * 3 + c] = v;
-    }
-}
-
-int assemble_gather(SellMatrix& A, const int* d_rowidx, const int* d_colidx, const long long* cptr, const int* codes,
-                    const double* Ke, const unsigned char* node_fix, double* vals_std, hipStream_t s) {
-  if (A.br != 3 || A.bc != 3) return kBadArg;
-  int r = A.ensure_values(1, 0);
-  if (r) return r;
-  if (A.nnzb == 0) return kOk;
-  hipLaunchKernelGGL(assemble_gather_kernel, dim3(ceil_div(A.nnzb, 256)), dim3(256), 0, s, A.nnzb, d_rowidx, d_colidx,
-                     cptr, codes, Ke, node_fix, A.d_slot, A.d_v64, vals_std);
-  return static_cast<int>(hipGetLastError());
-}
-
-// Generic version for b x b blocks of npe-node elements (beams: b = 6, npe =
-// 2): code = e*npe*npe + a*npe + c addresses Ke[e][b*a + r][b*c + q].
-template <int B>
-__global__ void assemble_elem_kernel(long long nnzb, int npe, int sym, const int* __restrict__ rowidx,
-                                     const int* __restrict__ colidx, const long long* __restrict__ cptr,
-                                     const int* __restrict__ codes, const double* __restrict__ Ke,
-                                     const unsigned char* __restrict__ node_fix, const long long* __restrict__ slot,
-                                     double* __restrict__ v64, double* __restrict__ vstd) {
-  const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (k >= nnzb) return;
-  const int D = npe * B, nn = npe * npe;
-  double acc[B * B];
-#pragma unroll
-  for (int t = 0; t < B * B; ++t) acc[t] = 0.0;
-  for (long long q = cptr[k]; q < cptr[k + 1]; ++q) {
-    const int code = codes[q];
-    const int e = code / nn, ab = code - e * nn, a = ab / npe, b = ab - a * npe;
-    const double* kp = Ke + (size_t)e * D * D;
-#pragma unroll
-    for (int r = 0; r < B; ++r)
-#pragma unroll
-      for (int c = 0; c < B; ++c) {
-        double v = kp[(size_t)(B * a + r) * D + B * b + c];
-        if (sym) v = 0.5 * (v + kp[(size_t)(B * b + c) * D + B * a + r]);
-        acc[r * B + c] += v;
-      }
-  }
-  const int i = rowidx[k], j = colidx[k];
-  const unsigned fi = node_fix ? node_fix[i] : 0u, fj = node_fix ? node_fix[j] : 0u;
-  const long long sl = slot[k];
-#pragma unroll
-  for (int r = 0; r < B; ++r)
-#pragma unroll
-    for (int c = 0; c < B; ++c) {
-      double v = acc[r * B + c];
-      if (((fi >> r) & 1u) || ((fj >> c) & 1u)) v = (i == j && r == c) ? 1.0 : 0.0;
-      v64[val_index<double>(sl, r * B + c, B * B)] = v;
-      if (vstd) vstd[k * B * B + r * B + c] = v;
-    }
-}
-
-int assemble_elem(SellMatrix& A, int npe, int sym, const int* d_rowidx, const int* d_colidx, const long long* cptr,
-                  const int* codes, const double* Ke, const unsigned char* node_fix, double* vals_std, hipStream_t s) {
-  if (A.br != A.bc || npe <= 0 || npe > 27) return kBadArg;
-  int r = A.ensure_values(1, 0);
-  if (r) return r;
-  if (A.nnzb == 0) return kOk;
-  const dim3 grid(ceil_div(A.nnzb, 128)), blk(128);
-  switch (A.br) {
-    case 3:
-      hipLaunchKernelGGL(assemble_elem_kernel<3>, grid, blk, 0, s, A.nnzb, npe, sym, d_rowidx, d_colidx, cptr, codes,
-                         Ke, node_fix, A.d_slot, A.d_v64, vals_std);
-      break;
-    case 6:
-      hipLaunchKernelGGL(assemble_elem_kernel<6>, grid, blk, 0, s, A.nnzb, npe, sym, d_rowidx, d_colidx, cptr, codes,
-                         Ke, node_fix, A.d_slot, A.d_v64, vals_std);
-      break;
-    default:
-      return kBadArg;
-  }
   return static_cast<int>(hipGetLastError());
 }
 
@@ -367,6 +265,10 @@ int equilibrate(SellMatrix& A, const int* d_rowidx, const int* d_colidx, const d
   }
   const long long n = A.nnzb * A.br * A.bc;
   if (n == 0) return kOk;
+  if (A.br == 3 || A.br == 6) {
+    launch_equilibrate_slots(A, scale, want64e ? A.d_v64e : nullptr, s);
+    return static_cast<int>(hipGetLastError());
+  }
   hipLaunchKernelGGL(equilibrate_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, A.nnzb, A.br, d_rowidx, d_colidx,
                      A.d_slot, scale, A.d_v64, A.d_v32, want64e ? A.d_v64e : nullptr, A.d_v16);
   return static_cast<int>(hipGetLastError());

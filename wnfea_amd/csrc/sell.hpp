@@ -104,6 +104,23 @@ __device__ __forceinline__ void load_block(const VT* __restrict__ region, int la
   if constexpr (REM > 0) load_vec<VT, REM>(region + FULL * 64 * V + lane * REM, v + FULL * V);
 }
 
+// The same for a store: v rounded to VT, the whole chunks with 16-byte stores.
+template <typename VT, int BB, typename S>
+__device__ __forceinline__ void store_block(VT* __restrict__ region, int lane, const S (&v)[BB]) {
+  constexpr int V = 16 / (int)sizeof(VT);
+  constexpr int FULL = BB / V, REM = BB - FULL * V;
+#pragma unroll
+  for (int g = 0; g < FULL; ++g) {
+    using E = VT __attribute__((ext_vector_type(V)));
+    E e;
+#pragma unroll
+    for (int i = 0; i < V; ++i) e[i] = VT(v[g * V + i]);
+    *reinterpret_cast<E*>(region + g * 64 * V + lane * V) = e;
+  }
+#pragma unroll
+  for (int i = 0; i < REM; ++i) region[FULL * 64 * V + lane * REM + i] = VT(v[FULL * V + i]);
+}
+
 template <typename T> struct AccT { using type = T; };
 template <> struct AccT<_Float16> { using type = float; };  // FP16 storage, FP32 arithmetic
 

@@ -25,6 +25,7 @@ struct SellMatrix {
   int2* d_rinfo = nullptr;  // [n_slices * 64/lanes] {block row or -1, blocks in the row}
   int* d_col = nullptr;
   long long* d_slot = nullptr;  // standard block index -> slot
+  int* d_rstart = nullptr;      // [n_slices * 64/lanes] standard index of the row's first block
   double* d_v64 = nullptr;   // primary FP64 values (the assembled K)
   double* d_v64e = nullptr;  // optional FP64 equilibrated values S K S
   float* d_v32 = nullptr;    // FP32 values (equilibrated for the fine level)
@@ -283,13 +284,19 @@ int spmv_restrict_first(const SellMatrix& A, const T* x, T* y, const T* dinv, T*
 // standard block layout <-> sliced layout, and assembly
 int sell_from_std(SellMatrix& A, const double* vals_std, int to64, int to32, hipStream_t s, int to16 = 0);
 int sell_to_std(const SellMatrix& A, double* vals_std, hipStream_t s);
-int assemble_gather(SellMatrix& A, const int* d_rowidx, const int* d_colidx, const long long* cptr, const int* codes,
-                    const double* Ke, const unsigned char* node_fix, double* vals_std, hipStream_t s);
-// Square element matrices Ke[M][npe*b][npe*b] (b = block size of A) into A's
-// FP64 values through the contribution lists; sym != 0 assembles the
+// Square element matrices Ke[M][npe*b][npe*b] (b = block size of A, 3 or 6)
+// into A's FP64 values through the contribution lists; sym != 0 assembles the
 // symmetric part 0.5 (Ke + Ke^T); node_fix bit c marks DOF c of a node fixed.
-int assemble_elem(SellMatrix& A, int npe, int sym, const int* d_rowidx, const int* d_colidx, const long long* cptr,
-                  const int* codes, const double* Ke, const unsigned char* node_fix, double* vals_std, hipStream_t s);
+int assemble_elem(SellMatrix& A, int npe, int sym, const long long* cptr, const int* codes, const double* Ke,
+                  const unsigned char* node_fix, double* vals_std, hipStream_t s);
+// The C3D10 matrix of an affine mesh from its element records (16 doubles each)
+int affine_records(int M, const int* conn, const double* nodes, const double* E, const double* nu, double* rec,
+                   int* flags, hipStream_t s);
+int assemble_affine(SellMatrix& A, const long long* cptr, const int* codes, const double* rec,
+                    const unsigned char* node_fix, hipStream_t s);
+// one lane per slot, 3x3 and 6x6 (and 3x6, 6x3) blocks
+void launch_equilibrate_slots(const SellMatrix& A, const double* scale, double* v64e, hipStream_t s);
+void launch_to_std_slots(const SellMatrix& A, double* vals_std, hipStream_t s);
 int extract_diag(const SellMatrix& A, const long long* diag_block, double* diag, hipStream_t s);
 int equilibrate(SellMatrix& A, const int* d_rowidx, const int* d_colidx, const double* scale, int want64e,
                 hipStream_t s, int want16 = 0);

@@ -160,20 +160,10 @@ def assemble_c3d10_bsr(model: FEAModel, apply_bcs: bool = True, sigma: int = 163
     t_plan = time.perf_counter() - t0
     K = DeviceBSR(3, 3, n, n, rowptr, colidx, sigma)
     t_layout = time.perf_counter() - t0 - t_plan
-    stream = _lib.stream_of()
-    Ke = torch.empty((M, 30, 30), dtype=torch.float64, device=dev)
-    bad = torch.zeros(1, dtype=torch.int32, device=dev)
-    _lib.check(L.wnfea_c3d10_ke(M, _lib.dptr(mesh["conn"]), _lib.dptr(mesh["nodes"]), _lib.dptr(mesh["E"]),
-                                _lib.dptr(mesh["nu"]), _lib.dptr(Ke), _lib.dptr(bad), stream), "wnfea_c3d10_ke")
     d_cptr = torch.as_tensor(cptr, device=dev)
     d_codes = torch.as_tensor(codes[:nc].copy() if nc else codes[:1].copy(), device=dev)
     d_fix = torch.as_tensor(node_fix, device=dev)
-    _lib.check(L.wnfea_bsr_assemble(K.handle, _lib.dptr(K.d_rowidx), _lib.dptr(K.d_colidx), _lib.dptr(d_cptr),
-                                    _lib.dptr(d_codes), _lib.dptr(Ke), _lib.dptr(d_fix) if apply_bcs else None,
-                                    None, stream), "wnfea_bsr_assemble")
-    if int(bad.item()):
-        raise ValueError(f"Non-positive Jacobian determinant in C3D10 element {int(bad.item()) - 1}. "
-                         "Element is inverted, degenerate, or has bad node numbering.")
+    _assemble_values(K, mesh, d_cptr, d_codes, d_fix if apply_bcs else None)
     F = model.load_vector(3)
     if apply_bcs:
         F[fixed_mask] = 0.0
@@ -183,10 +173,41 @@ def assemble_c3d10_bsr(model: FEAModel, apply_bcs: bool = True, sigma: int = 163
     if keep_plan:
         mesh["plan"] = {"cptr": d_cptr, "codes": d_codes, "fix": d_fix if apply_bcs else None,
                         "want64e": bool(want_fp64_equilibrated)}
-    del Ke, d_cptr, d_codes
+    del d_cptr, d_codes
     torch.cuda.empty_cache()
     sys_.timings = {"plan_sec": t_plan, "layout_sec": t_layout, "assemble_total_sec": time.perf_counter() - t0}
     return sys_
+
+
+def _assemble_values(K: DeviceBSR, mesh: dict, cptr, codes, fix) -> None:
+    """FP64 values of K from the mesh's geometry and moduli through the device
+    contribution lists, supports applied.  A mesh of affine elements (told on
+    the device, each time) is assembled from one 128-byte record per element;
+    one with curved elements from its element matrices."""
+    import torch
+    L = _lib.load()
+    M, dev, stream = mesh["n_elements"], K.device, _lib.stream_of()
+    args = (M, _lib.dptr(mesh["conn"]), _lib.dptr(mesh["nodes"]), _lib.dptr(mesh["E"]), _lib.dptr(mesh["nu"]))
+    rec = torch.empty((max(M, 1), 16), dtype=torch.float64, device=dev)
+    flags = torch.zeros(2, dtype=torch.int32, device=dev)
+    _lib.check(L.wnfea_c3d10_affine_records(*args, _lib.dptr(rec), _lib.dptr(flags), stream),
+               "wnfea_c3d10_affine_records")
+    bad, curved = flags.tolist()
+    if not curved and not bad:
+        _lib.check(L.wnfea_bsr_assemble_affine(K.handle, _lib.dptr(cptr), _lib.dptr(codes), _lib.dptr(rec),
+                                               _lib.dptr(fix), stream), "wnfea_bsr_assemble_affine")
+        return
+    if curved:
+        Ke = torch.empty((M, 30, 30), dtype=torch.float64, device=dev)
+        flags.zero_()
+        _lib.check(L.wnfea_c3d10_ke(*args, _lib.dptr(Ke), _lib.dptr(flags), stream), "wnfea_c3d10_ke")
+        _lib.check(L.wnfea_bsr_assemble(K.handle, _lib.dptr(K.d_rowidx), _lib.dptr(K.d_colidx), _lib.dptr(cptr),
+                                        _lib.dptr(codes), _lib.dptr(Ke), _lib.dptr(fix), None, stream),
+                   "wnfea_bsr_assemble")
+        bad = int(flags[0].item())
+    if bad:
+        raise ValueError(f"Non-positive Jacobian determinant in C3D10 element {bad - 1}. "
+                         "Element is inverted, degenerate, or has bad node numbering.")
 
 
 def reassemble_c3d10_values(system: SolidSystem, E=None, nu=None) -> SolidSystem:
@@ -195,7 +216,6 @@ def reassemble_c3d10_values(system: SolidSystem, E=None, nu=None) -> SolidSystem
     stiffnesses, the deterministic gather, the diagonal, the scaling and the
     equilibrated copies are recomputed in place; the pattern is unchanged."""
     import torch
-    L = _lib.load()
     mesh = system.mesh
     plan = mesh.get("plan")
     if plan is None:
@@ -209,19 +229,7 @@ def reassemble_c3d10_values(system: SolidSystem, E=None, nu=None) -> SolidSystem
                 raise ValueError(f"{key} must have one value per element ({M})")
             # in place: matrix-free operators of this system read the same buffer
             mesh[key].copy_(t)
-    stream = _lib.stream_of()
-    Ke = torch.empty((M, 30, 30), dtype=torch.float64, device=dev)
-    bad = torch.zeros(1, dtype=torch.int32, device=dev)
-    _lib.check(L.wnfea_c3d10_ke(M, _lib.dptr(mesh["conn"]), _lib.dptr(mesh["nodes"]), _lib.dptr(mesh["E"]),
-                                _lib.dptr(mesh["nu"]), _lib.dptr(Ke), _lib.dptr(bad), stream), "wnfea_c3d10_ke")
-    K = system.K
-    _lib.check(L.wnfea_bsr_assemble(K.handle, _lib.dptr(K.d_rowidx), _lib.dptr(K.d_colidx), _lib.dptr(plan["cptr"]),
-                                    _lib.dptr(plan["codes"]), _lib.dptr(Ke),
-                                    _lib.dptr(plan["fix"]) if plan["fix"] is not None else None, None, stream),
-               "wnfea_bsr_assemble")
-    if int(bad.item()):
-        raise ValueError(f"Non-positive Jacobian determinant in C3D10 element {int(bad.item()) - 1}.")
-    del Ke
+    _assemble_values(system.K, mesh, plan["cptr"], plan["codes"], plan["fix"])
     refresh_scaling(system)
     return system
 
