@@ -1099,10 +1099,11 @@ __global__ __launch_bounds__(64 * kGatherWaves) void mf_gather_op_kernel(
 //  1. loads addressed by the patch index alone are issued first: each lane's
 //     four 16-bit local nodes (its vertex and that vertex's three edges, 8
 //     bytes), its part of the element's record, the patch's slot codes (into
-//     LDS) and its local nodes' global ids and list starts (fixed stride per
-//     patch); then those addressed through them: the scaled nodal values
-//     sc .* U of the local nodes (into LDS, four entries per node; up to NS
-//     nodes per lane, loads issued together) and, unfolded, the element moduli;
+//     LDS) and its local nodes' global ids, list starts and, where the stage
+//     sums partials, heads (fixed stride per patch); then those addressed
+//     through them: what Stage needs for the scaled nodal values of the local
+//     nodes (into LDS, four entries per node; up to NS nodes per lane, loads
+//     issued together) and, unfolded, the element moduli;
 //  2. each quad computes its element's forces (vertex_forces, lane v at vertex
 //     v, four nodal values per lane read from LDS) and keeps them in LDS;
 //  3. each local node adds its element forces in slot order (slot codes
@@ -1158,12 +1159,124 @@ __device__ __forceinline__ void lds_force(const double* fl, int i, double (&v)[3
   for (int c = 0; c < 3; ++c) v[c] = fl[3 * i + c];
 }
 
-template <typename T, int P, int NS, bool Folded>
+// What a patch stages for its local nodes.  load() issues the loads of node n
+// (clamped: in bounds for any lane), value() gives the scaled nodal values.
+template <typename T>
+struct StageScaled {  // sc .* U
+  static constexpr bool kHead = false;
+  const T* sc;
+  const T* U;
+  struct Pre { T u[3], s[3]; };
+  __device__ __forceinline__ void load(unsigned n, const int4&, Pre& p) const {
+    const T* u = U + 3 * (size_t)n;
+    const T* s = sc + 3 * (size_t)n;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      p.u[c] = u[c];
+      p.s[c] = s[c];
+    }
+  }
+  __device__ __forceinline__ void value(unsigned, bool, const int4&, const Pre& p, T (&x)[3]) const {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) x[c] = p.u[c] * p.s[c];
+  }
+};
+
+// A node's partial sums in patch order: head h (its first three slots and the
+// count, or an overflow list).
+template <typename T>
+__device__ __forceinline__ void load_partials(const int4& h, const T* __restrict__ part, T (&v)[3][3]) {
+  const int hi[3] = {h.x, h.y, h.z};
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[q][c] = part[(size_t)max(hi[q], 0) * 3 + c];
+}
+template <typename T>
+__device__ __forceinline__ void sum_partials(const int4& h, const int* __restrict__ novf, const T* __restrict__ part,
+                                             const T (&v)[3][3], T (&acc)[3]) {
+  const int hi[3] = {h.x, h.y, h.z};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) acc[c] = T(0);
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      if (hi[q] >= 0) acc[c] = q == 0 ? v[q][c] : acc[c] + v[q][c];
+  if (h.w < 0) {  // more than three partials
+    const int k = -h.w - 1, cnt = novf[k];
+    for (int q = 1; q <= cnt; ++q) {
+      const T* w = part + (size_t)novf[k + q] * 3;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) acc[c] += w[c];
+    }
+  }
+}
+
+// The Chebyshev step that completes the product before, as mf_node_kernel
+// with OpCheb would, formed by every patch that stages the node (2.1 times per
+// node on the I-beam); the patch of the node's first partial stores the step's
+// x and d.  Its inputs are read by other patches, so outputs, partial sums and
+// d go to buffers of their own.  One launch and one pass over the nodes fewer
+// per step; the same expressions and order, so the same bits.  On the first
+// step (c1 = 0) d is not read.
+template <typename T, bool Unit>
+struct StageCheb {
+  static constexpr bool kHead = true;
+  const T* part;  // partial sums of the product of x
+  const int* novf;
+  const unsigned char* fix;
+  const T* sc;    // the operator's scaling (true values on fixed DOFs)
+  const T* x;
+  const T* b;
+  const T* dinv;
+  const T* d;
+  T* x_out;
+  T* d_out;
+  T c1, c2;
+  struct Pre { T x[3], b[3], d[3], dv[3], s[3], v[3][3]; int m; };
+  __device__ __forceinline__ void load(unsigned n, const int4& h, Pre& p) const {
+    const size_t n3 = 3 * (size_t)n;
+    p.m = fix ? fix[n] : 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      p.x[c] = x[n3 + c];
+      p.b[c] = b[n3 + c];
+      p.s[c] = sc[n3 + c];
+      p.d[c] = c1 != T(0) ? d[n3 + c] : T(0);
+      if constexpr (Unit) {
+        p.dv[c] = T(1);
+      } else {
+        p.dv[c] = dinv[n3 + c];
+      }
+    }
+    load_partials(h, part, p.v);
+  }
+  __device__ __forceinline__ void value(unsigned n, bool store, const int4& h, const Pre& p, T (&out)[3]) const {
+    T acc[3];
+    sum_partials(h, novf, part, p.v, acc);
+    const size_t n3 = 3 * (size_t)n;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const bool fixed = (p.m >> c) & 1;
+      const T ku = fixed ? p.s[c] * p.x[c] : acc[c];
+      const T dn = c1 * p.d[c] + c2 * p.dv[c] * (p.b[c] - p.s[c] * ku);
+      const T xo = p.x[c] + dn;
+      if (store) {
+        d_out[n3 + c] = dn;
+        x_out[n3 + c] = xo;
+      }
+      out[c] = fixed ? T(0) : xo * p.s[c];
+    }
+  }
+};
+
+template <typename T, int P, int NS, bool Folded, class Stage>
 __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
     int n_patch, int M, int stride, const int* __restrict__ pnode, const ushort4* __restrict__ pconn,
     const unsigned short* __restrict__ poff, const uint2* __restrict__ pslot, const int* __restrict__ pe,
     const T* __restrict__ qdp, const double* __restrict__ E, const double* __restrict__ nu,
-    const T* __restrict__ sc, const T* __restrict__ U, T* __restrict__ part, const int* skip) {
+    const int4* __restrict__ phead, Stage stage, T* __restrict__ part, const int* skip) {
   constexpr int NT = 4 * P, FS = force_stride<T>(), NC = 10 * P / 4;  // NC: 8-byte runs of slot codes
   if (skip && *skip) return;
   extern __shared__ __align__(16) unsigned char patch_lds[];
@@ -1198,11 +1311,13 @@ __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
   const unsigned short* po = poff + pb;
   int gn[NS];
   unsigned short off[NS];
+  int4 head[NS];
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
     const unsigned j = (unsigned)min(t + k * NT, stride - 1);
     gn[k] = pn[j];
     off[k] = po[j];
+    if constexpr (Stage::kHead) head[k] = phead[pb + j];
   }
   // second round: addressed through the first
   double Ev = 0.0, nv = 0.0;
@@ -1210,22 +1325,20 @@ __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
     Ev = E[ee];
     nv = nu[ee];
   }
-  T xv[NS][3];
+  typename Stage::Pre pre[NS];
 #pragma unroll
-  for (int k = 0; k < NS; ++k) {
-    const size_t n3 = 3 * (size_t)max(gn[k], 0);
-    const T* uk = U + n3;
-    const T* sk = sc + n3;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) xv[k][c] = uk[c] * sk[c];
-  }
+  for (int k = 0; k < NS; ++k) stage.load((unsigned)max(gn[k], 0), head[k], pre[k]);
   if (t < NC) reinterpret_cast<uint2*>(ls)[t] = code;
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
     const int j = t + k * NT;
     if (j < stride) {
+      T xv[3];
+      // the node's first partial is this patch's: this patch stores for it
+      const bool first = Stage::kHead && gn[k] >= 0 && head[k].x == (int)(pb + j);
+      stage.value((unsigned)max(gn[k], 0), first, head[k], pre[k], xv);
       lo[j] = off[k];
-      lds_store_node(xs, j, xv[k]);
+      lds_store_node(xs, j, xv);
     }
   }
   __syncthreads();
@@ -1336,27 +1449,9 @@ __global__ __launch_bounds__(kNodeThreads) void mf_node_kernel(int n_nodes, cons
     if (sc) s3[c] = sc[k];
     xr[c] = x[k];
   }
-  const int hi[3] = {h.x, h.y, h.z};
-  T v[3][3];
-#pragma unroll
-  for (int q = 0; q < 3; ++q)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) v[q][c] = part[(size_t)max(hi[q], 0) * 3 + c];
-  T acc[3] = {T(0), T(0), T(0)};
-#pragma unroll
-  for (int q = 0; q < 3; ++q)
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      if (hi[q] >= 0) acc[c] = q == 0 ? v[q][c] : acc[c] + v[q][c];
-  if (h.w < 0) {  // more than three partials
-    const int k = -h.w - 1, cnt = novf[k];
-    for (int q = 1; q <= cnt; ++q) {
-      const T* w = part + (size_t)novf[k + q] * 3;
-      acc[0] += w[0];
-      acc[1] += w[1];
-      acc[2] += w[2];
-    }
-  }
+  T v[3][3], acc[3];
+  load_partials(h, part, v);
+  sum_partials(h, novf, part, v, acc);
   double dots[2] = {0.0, 0.0};
   if (has) {
     const int m = mraw;
@@ -1484,12 +1579,14 @@ std::vector<int> mf_chunks(const std::vector<int>& ptr) {  // first node of each
 // ---------------------------------------------------------------- patch layout (host set-up)
 static void mf_patch_release(MfOp& op) {
   for (void* p : {(void*)op.pe, (void*)op.pnode, (void*)op.pconn, (void*)op.poff, (void*)op.pslot, (void*)op.nhead,
-                  (void*)op.novf, (void*)op.qdp, (void*)op.part})
+                  (void*)op.novf, (void*)op.qdp, (void*)op.part, (void*)op.part2, (void*)op.phead})
     if (p) (void)hipFree(p);
   op.pe = op.pnode = op.novf = nullptr;
   op.nhead = nullptr;
   op.pconn = op.poff = op.pslot = nullptr;
-  op.qdp = op.part = nullptr;
+  op.qdp = op.part = op.part2 = nullptr;
+  op.phead = nullptr;
+  op.orphans = 0;
   op.patch = op.n_patch = op.lmax = op.stride = op.n_local = 0;
   ++op.gen;
 }
@@ -1502,6 +1599,20 @@ static size_t patch_lds_bytes(const MfOp& op, size_t elem) {
 constexpr size_t kPatchLdsMax = 64 * 1024;
 constexpr int kDefaultPatch = 64;
 constexpr int kStageSlots = 3;  // most local nodes a lane stages: 3 * 4 P >= the stride
+
+// Where the smoothing chain pays: while a product has few patches for the
+// chip, its kernels are bound by their chains of dependent loads and by the
+// launches between them, and staging a step's completion drops a launch per
+// step; with more, the nodes that several patches form (twice on average)
+// cost more than the launch.  A whole solve without and with the chain: FP32,
+// box of 60 patches 1850 -> 1690 us, of 203 2135 -> 2069, I-beam of 490
+// 5366 -> 5282, of 653 6496 -> 6470, of 1632 9492 -> 9700.  FP64, whose chain
+// keeps 4 wavefronts per SIMD and not 8: box of 60 patches 1858 -> 1805 us, of
+// 203 2498 -> 2470, I-beam of 326 6252 -> 6293.
+template <typename T>
+static bool mf_chain_rule(const MfOp& op) {
+  return op.patch && !op.orphans && op.n_patch <= (sizeof(T) == 4 ? 512 : 256);
+}
 
 int mf_set_patch(MfOp& op, int elems, hipStream_t s) {
   if (elems < 0 || elems > 256 || elems % 64) return kBadArg;
@@ -1546,6 +1657,15 @@ int mf_set_patch(MfOp& op, int elems, hipStream_t s) {
       o[0] = c[v];
       for (int m = 0; m < 3; ++m) o[1 + m] = c[kEdgeOf[v][m]];
     }
+  // the node heads per local node, for the patches that sum partials themselves
+  std::vector<int4> phead(cap, make_int4(-1, -1, -1, 0));
+  for (size_t k = 0; k < cap; ++k)
+    if (pnode[k] >= 0) {
+      const int* h = nhead.data() + 4 * (size_t)pnode[k];
+      phead[k] = make_int4(h[0], h[1], h[2], h[3]);
+    }
+  for (int i = 0; i < N; ++i)
+    if (nhead[4 * (size_t)i + 3] == 0) op.orphans = 1;  // a node of no element
   pslot.resize((size_t)op.n_patch * P * 10, 0);  // whole patches: the last one's codes are read in full
   auto up = [&](auto*& dst, const auto& v) -> int {
     using E = typename std::decay_t<decltype(v)>::value_type;
@@ -1555,12 +1675,13 @@ int mf_set_patch(MfOp& op, int elems, hipStream_t s) {
   };
   int r;
   if ((r = up(op.pe, order)) || (r = up(op.pnode, pnode)) || (r = up(op.pconn, lconn)) || (r = up(op.poff, poff)) ||
-      (r = up(op.pslot, pslot)) || (r = up(op.nhead, nhead)) || (r = up(op.novf, novf))) {
+      (r = up(op.pslot, pslot)) || (r = up(op.nhead, nhead)) || (r = up(op.novf, novf)) || (r = up(op.phead, phead))) {
     mf_patch_release(op);
     return r;
   }
   hipError_t e = hipMalloc(&op.qdp, sizeof(double) * 10 * (size_t)M);
   if (e == hipSuccess) e = hipMalloc(&op.part, sizeof(double) * 3 * cap);
+  if (e == hipSuccess && mf_chain_rule<double>(op)) e = hipMalloc(&op.part2, sizeof(double) * 3 * cap);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(qdata_permute_kernel, dim3(vec_grid(10LL * M)), dim3(256), 0, s, M, op.pe, op.qd, op.qdp);
     e = hipGetLastError();
@@ -1649,15 +1770,14 @@ static int node_grid(int n_nodes) { return 8 * ceil_div(std::max(1, ceil_div(n_n
 static int patch_grid(int n_patch) { return 8 * ceil_div(std::max(1, n_patch), 8); }
 
 // the patch kernel for the layout's patch size
-template <typename T, bool Folded>
-static void launch_patch(const MfOp& op, const T* qdp, const T* sc, const T* U, T* part, const int* skip,
-                         hipStream_t s) {
+template <typename T, bool Folded, class Stage>
+static void launch_patch(const MfOp& op, const T* qdp, const Stage& st, T* part, const int* skip, hipStream_t s) {
   const dim3 grid(patch_grid(op.n_patch));
   const size_t lds = patch_lds_bytes(op, sizeof(T));
 #define WN_PATCH_LAUNCH1(PP, NS)                                                                                    \
-  hipLaunchKernelGGL((mf_patch_kernel<T, PP, NS, Folded>), grid, dim3(4 * (PP)), lds, s, op.n_patch, op.M,          \
+  hipLaunchKernelGGL((mf_patch_kernel<T, PP, NS, Folded, Stage>), grid, dim3(4 * (PP)), lds, s, op.n_patch, op.M,   \
                      op.stride, op.pnode, reinterpret_cast<const ushort4*>(op.pconn), op.poff,                      \
-                     reinterpret_cast<const uint2*>(op.pslot), op.pe, qdp, op.E, op.nu, sc, U, part, skip)
+                     reinterpret_cast<const uint2*>(op.pslot), op.pe, qdp, op.E, op.nu, op.phead, st, part, skip)
 #define WN_PATCH_LAUNCH(PP)                                                                                         \
   if (op.stride <= 8 * (PP)) WN_PATCH_LAUNCH1(PP, 2); else WN_PATCH_LAUNCH1(PP, kStageSlots)
   switch (op.patch) {
@@ -1684,7 +1804,7 @@ int mf_apply(const MfOp& op, const double* u, const double* f, double* y, double
   if (op.patch) {
     if (!op.mask) return kNotReady;
     const int* skip = guard ? flags : nullptr;
-    launch_patch<double, false>(op, op.qdp, op.mask, u, op.part, skip, s);
+    launch_patch<double, false>(op, op.qdp, StageScaled<double>{op.mask, u}, op.part, skip, s);
     const OpMfMode o{u, f, y, mode, mode ? partials : nullptr};
     hipLaunchKernelGGL((mf_node_kernel<double, OpMfMode>), dim3(node_grid(op.n_nodes)), dim3(kNodeThreads), 0, s,
                        op.n_nodes, op.nhead, op.novf, op.part, op.fix, nullptr, u, o, skip);
@@ -1732,12 +1852,12 @@ int launch_adjoint_dot(int M, const int* conn, const double* E, const double* fe
 // ---------------------------------------------------------------- V-cycle smoothing on the matrix-free operator
 void mf_smooth_release(MfSmooth& m) {
   for (void* p : {(void*)m.s64e, (void*)m.s32, (void*)m.s32e, (void*)m.qd32, (void*)m.fe32, (void*)m.qdp32,
-                  (void*)m.part32})
+                  (void*)m.part32, (void*)m.part32b, (void*)m.d32b, (void*)m.d64b})
     if (p) (void)hipFree(p);
   m = MfSmooth{};
 }
 
-int mf_smooth_attach(MfSmooth& m, const MfOp* op, const double* scale, int want32, hipStream_t s) {
+int mf_smooth_attach(MfSmooth& m, const MfOp* op, const double* scale, int want64, int want32, hipStream_t s) {
   mf_smooth_release(m);
   if (!op) return kOk;  // detach
   if (!op->chunk || (op->M > 0 && (!op->qd || !op->fe)) || !scale) return kBadArg;
@@ -1745,6 +1865,8 @@ int mf_smooth_attach(MfSmooth& m, const MfOp* op, const double* scale, int want3
   const size_t nv = (size_t)std::max<long long>(n, 1);
   WN_HIP(hipMalloc(&m.s64e, sizeof(double) * nv));
   hipLaunchKernelGGL(dof_scale_kernel<double>, dim3(vec_grid(n)), dim3(256), 0, s, n, scale, op->fix, m.s64e);
+  // second d of the smoothing chain (its patches read the first while one stores)
+  if (want64 && mf_chain_rule<double>(*op)) WN_HIP(hipMalloc(&m.d64b, sizeof(double) * nv));
   if (want32) {
     WN_HIP(hipMalloc(&m.s32, sizeof(float) * nv));
     WN_HIP(hipMalloc(&m.s32e, sizeof(float) * nv));
@@ -1758,6 +1880,10 @@ int mf_smooth_attach(MfSmooth& m, const MfOp* op, const double* scale, int want3
     if (op->patch) {
       WN_HIP(hipMalloc(&m.qdp32, sizeof(float) * 12 * (size_t)op->M));
       WN_HIP(hipMalloc(&m.part32, sizeof(float) * 3 * (size_t)op->n_patch * op->stride));
+      if (mf_chain_rule<float>(*op)) {
+        WN_HIP(hipMalloc(&m.part32b, sizeof(float) * 3 * (size_t)op->n_patch * op->stride));
+        WN_HIP(hipMalloc(&m.d32b, sizeof(float) * nv));
+      }
       hipLaunchKernelGGL(qdata_fold_kernel, dim3(vec_grid(op->M)), dim3(256), 0, s, op->M, op->pe, op->qdp, op->E,
                          op->nu, m.qdp32);
     }
@@ -1804,7 +1930,7 @@ static int mf_smooth_run(const MfSmooth& m, const T* x, const Op& o, const int* 
   const T* sc = mf_scale<T>(m);
   if (const T* qdp = mf_qdp<T>(m)) {
     T* part = mf_part<T>(m);
-    launch_patch<T, std::is_same<T, float>::value>(op, qdp, mf_scale_in<T>(m), x, part, skip, s);
+    launch_patch<T, std::is_same<T, float>::value>(op, qdp, StageScaled<T>{mf_scale_in<T>(m), x}, part, skip, s);
     hipLaunchKernelGGL((mf_node_kernel<T, Op>), dim3(node_grid(op.n_nodes)), dim3(kNodeThreads), 0, s, op.n_nodes,
                        op.nhead, op.novf, part, op.fix, sc, x, o, skip);
     return static_cast<int>(hipGetLastError());
@@ -1866,6 +1992,81 @@ struct OpChebRho {
   }
 };
 
+// The smoothing chain of the patch layout: a product (mf_smooth_product),
+// steps that complete one product and form the next (mf_smooth_step), and a
+// node kernel that completes the last (mf_smooth_end_*).  `from` names the
+// partial-sum buffer, 0 or 1, that holds the product to complete.
+template <typename T> static T* mf_parts(const MfSmooth& m, int k);
+template <> double* mf_parts<double>(const MfSmooth& m, int k) { return k ? m.op->part2 : m.op->part; }
+template <> float* mf_parts<float>(const MfSmooth& m, int k) { return k ? m.part32b : m.part32; }
+template <> double* mf_smooth_d2<double>(const MfSmooth& m) { return m.d64b; }
+template <> float* mf_smooth_d2<float>(const MfSmooth& m) { return m.d32b; }
+
+template <typename T>
+bool mf_smooth_chain(const MfSmooth& m) {
+  // (a relayout since the attachment may have dropped the second partial sums)
+  return mf_smooth_ready<T>(m) && mf_qdp<T>(m) && mf_smooth_d2<T>(m) && mf_parts<T>(m, 1);
+}
+
+template <typename T>
+int mf_smooth_product(const MfSmooth& m, const T* x, const int* skip, hipStream_t s) {
+  launch_patch<T, std::is_same<T, float>::value>(*m.op, mf_qdp<T>(m), StageScaled<T>{mf_scale_in<T>(m), x},
+                                                 mf_parts<T>(m, 0), skip, s);
+  return static_cast<int>(hipGetLastError());
+}
+
+template <typename T>
+int mf_smooth_step(const MfSmooth& m, int from, const T* x, T* x_out, const T* b, const T* dinv, const T* d, T* d_out,
+                   T c1, T c2, const int* skip, hipStream_t s) {
+  const MfOp& op = *m.op;
+  constexpr bool F = std::is_same<T, float>::value;
+  T* to = mf_parts<T>(m, 1 - from);
+  if (!dinv)
+    launch_patch<T, F>(op, mf_qdp<T>(m), StageCheb<T, true>{mf_parts<T>(m, from), op.novf, op.fix, mf_scale<T>(m), x, b,
+                                                            nullptr, d, x_out, d_out, c1, c2}, to, skip, s);
+  else
+    launch_patch<T, F>(op, mf_qdp<T>(m), StageCheb<T, false>{mf_parts<T>(m, from), op.novf, op.fix, mf_scale<T>(m), x,
+                                                             b, dinv, d, x_out, d_out, c1, c2}, to, skip, s);
+  return static_cast<int>(hipGetLastError());
+}
+
+template <typename T, class Op>
+static int mf_smooth_end(const MfSmooth& m, int from, const T* x, const Op& o, const int* skip, hipStream_t s) {
+  const MfOp& op = *m.op;
+  hipLaunchKernelGGL((mf_node_kernel<T, Op>), dim3(node_grid(op.n_nodes)), dim3(kNodeThreads), 0, s, op.n_nodes,
+                     op.nhead, op.novf, mf_parts<T>(m, from), op.fix, mf_scale<T>(m), x, o, skip);
+  return static_cast<int>(hipGetLastError());
+}
+
+template <typename T>
+int mf_smooth_end_defect(const MfSmooth& m, int from, const T* x, const T* b, T* res, const int* skip,
+                         hipStream_t s) {
+  return mf_smooth_end<T>(m, from, x, OpDefect<3, T>{b, res}, skip, s);
+}
+
+// the last step of a smoother; with rq also the partials of rho = r . (S x_out)
+template <typename T>
+int mf_smooth_end_cheb(const MfSmooth& m, int from, const T* x, T* x_out, const T* b, const T* dinv, T* d, T c1, T c2,
+                       const RhoReq* rq, const int* skip, hipStream_t s) {
+  const OpCheb<3, T> o{b, dinv, x, x_out, d, c1, c2};
+  const OpCheb<3, T, true> u{b, nullptr, x, x_out, d, c1, c2};
+  if (rq && !dinv) return mf_smooth_end<T>(m, from, x, OpChebRho<T, true>{u, rq->r, rq->scale, rq->partials}, skip, s);
+  if (rq) return mf_smooth_end<T>(m, from, x, OpChebRho<T>{o, rq->r, rq->scale, rq->partials}, skip, s);
+  return dinv ? mf_smooth_end<T>(m, from, x, o, skip, s) : mf_smooth_end<T>(m, from, x, u, skip, s);
+}
+
+#define WN_CHAIN_INST(T)                                                                                          \
+  template bool mf_smooth_chain<T>(const MfSmooth&);                                                             \
+  template int mf_smooth_product<T>(const MfSmooth&, const T*, const int*, hipStream_t);                         \
+  template int mf_smooth_step<T>(const MfSmooth&, int, const T*, T*, const T*, const T*, const T*, T*, T, T,     \
+                                 const int*, hipStream_t);                                                       \
+  template int mf_smooth_end_defect<T>(const MfSmooth&, int, const T*, const T*, T*, const int*, hipStream_t);   \
+  template int mf_smooth_end_cheb<T>(const MfSmooth&, int, const T*, T*, const T*, const T*, T*, T, T,           \
+                                     const RhoReq*, const int*, hipStream_t);
+WN_CHAIN_INST(float)
+WN_CHAIN_INST(double)
+#undef WN_CHAIN_INST
+
 template <typename T>
 int mf_smooth_rho_blocks(const MfSmooth& m) {
   return mf_smooth_ready<T>(m) && mf_qdp<T>(m) ? node_grid(m.op->n_nodes) : 0;
@@ -1878,7 +2079,7 @@ int mf_smooth_cheb_rho(const MfSmooth& m, const T* x_in, T* x_out, const T* b, c
   if (!qdp || !rq.r || !rq.partials) return kBadMode;
   const MfOp& op = *m.op;
   T* part = mf_part<T>(m);
-  launch_patch<T, std::is_same<T, float>::value>(op, qdp, mf_scale_in<T>(m), x_in, part, skip, s);
+  launch_patch<T, std::is_same<T, float>::value>(op, qdp, StageScaled<T>{mf_scale_in<T>(m), x_in}, part, skip, s);
   const dim3 grid(node_grid(op.n_nodes));
   if (!dinv) {
     const OpChebRho<T, true> o{{b, nullptr, x_in, x_out, d, c1, c2}, rq.r, rq.scale, rq.partials};

@@ -313,12 +313,27 @@ static int vcycle(Amg& g, int l, const T* b, T* x, const int* skip, hipStream_t 
                        skip);
     if ((r = static_cast<int>(hipGetLastError()))) return r;
   }
-  for (int k = 1; k < deg; ++k) {
-    if ((r = cheb(cur, oth, k))) return r;
-    std::swap(cur, oth);
+  // in the patch layout each step's completion is staged by the next product
+  const bool chain = mf && mf_smooth_chain<T>(g.mfs);
+  T* d2 = chain ? mf_smooth_d2<T>(g.mfs) : nullptr;
+  if (chain) {
+    if ((r = mf_smooth_product<T>(g.mfs, cur, skip, s))) return r;
+    int from = 0;
+    for (int k = 1; k < deg; ++k, from = 1 - from) {
+      if ((r = mf_smooth_step<T>(g.mfs, from, cur, oth, b, dinv_mf, d, d2, T(c.c1[k]), T(c.c2[k]), skip, s))) return r;
+      std::swap(cur, oth);
+      std::swap(d, d2);
+    }
+    if ((r = mf_smooth_end_defect<T>(g.mfs, from, cur, b, res, skip, s))) return r;
+  } else {
+    for (int k = 1; k < deg; ++k) {
+      if ((r = cheb(cur, oth, k))) return r;
+      std::swap(cur, oth);
+    }
+    // defect and restriction
+    r = mf ? mf_smooth_defect<T>(g.mfs, cur, b, res, skip, s) : spmv_defect<VT, T>(A, cur, b, res, t, s);
+    if (r) return r;
   }
-  // defect and restriction
-  if ((r = mf ? mf_smooth_defect<T>(g.mfs, cur, b, res, skip, s) : spmv_defect<VT, T>(A, cur, b, res, t, s))) return r;
   AmgLevel& N = *g.L[l + 1];
   T** nv = level_vecs<T>(N);
   // a smoothed coarser level gets its first Chebyshev iterate from the
@@ -337,6 +352,16 @@ static int vcycle(Amg& g, int l, const T* b, T* x, const int* skip, hipStream_t 
   if ((r = vcycle<VTC, VTC, T, VSC, VSC>(g, l + 1, nv[0], nv[1], skip, s, nullptr, fuse_first))) return r;
   if ((r = spmv_addto<VT, T>(L.P, nv[1], cur, t, s))) return r;  // cur == post here
   oth = (cur == x) ? tmp : x;
+  if (chain) {
+    if ((r = mf_smooth_product<T>(g.mfs, cur, skip, s))) return r;
+    int from = 0;
+    for (int k = 0; k < deg - 1; ++k, from = 1 - from) {
+      if ((r = mf_smooth_step<T>(g.mfs, from, cur, oth, b, dinv_mf, d, d2, T(c.c1[k]), T(c.c2[k]), skip, s))) return r;
+      std::swap(cur, oth);
+      std::swap(d, d2);
+    }
+    return mf_smooth_end_cheb<T>(g.mfs, from, cur, oth, b, dinv_mf, d, T(c.c1[deg - 1]), T(c.c2[deg - 1]), rq, skip, s);
+  }
   for (int k = 0; k < deg; ++k) {
     if ((r = cheb(cur, oth, k, k == deg - 1 ? rq : nullptr))) return r;
     std::swap(cur, oth);
@@ -929,7 +954,7 @@ int amg_set_coarse(Amg& g, int n, const double* inv) {
 
 int amg_attach_mf(Amg& g, const MfOp* op, const double* scale, hipStream_t s) {
   if (op && (g.L.empty() || 3LL * op->n_nodes != g.L[0]->n)) return kBadArg;
-  return mf_smooth_attach(g.mfs, op, scale, (g.store & 2) ? 1 : 0, s);
+  return mf_smooth_attach(g.mfs, op, scale, g.store & 1, (g.store & 2) ? 1 : 0, s);
 }
 
 int amg_set_tune(Amg& g, int prec, int waves, int xcd_remap, int unroll) {

@@ -120,6 +120,9 @@ struct MfOp {
   int* novf = nullptr;                   // overflow lists of nodes with more than three partials
   double* qdp = nullptr;                 // [M][10] per slot det J / 24 and the gradients of L_1, L_2, L_3
   double* part = nullptr;                // [n_patch * stride][3]
+  double* part2 = nullptr;               // a second one: FP64 smoothing steps read one and write the other
+  int4* phead = nullptr;                 // [n_patch * stride] nhead of each local node
+  int orphans = 0;                       // some node belongs to no element (and so to no patch)
   std::vector<int> order;                // host: elements in Morton order of their centroids
 };
 // The finest level's smoothing and defect products of a V-cycle run
@@ -137,9 +140,12 @@ struct MfSmooth {
   float* fe32 = nullptr;  // [10][M][3]
   float* qdp32 = nullptr;   // [M][12] patch layout: weighted lambda, mu, a pad and the rounded gradients
   float* part32 = nullptr;  // [n_patch * stride][3]
+  float* part32b = nullptr;
+  float* d32b = nullptr;    // second d of the smoothing chain, per precision
+  double* d64b = nullptr;
   int gen = -1;             // the operator's layout generation the copies were made for
 };
-int mf_smooth_attach(MfSmooth& m, const MfOp* op, const double* scale, int want32, hipStream_t s);
+int mf_smooth_attach(MfSmooth& m, const MfOp* op, const double* scale, int want64, int want32, hipStream_t s);
 void mf_smooth_release(MfSmooth& m);
 template <typename T> bool mf_smooth_ready(const MfSmooth& m);
 template <> bool mf_smooth_ready<double>(const MfSmooth& m);
@@ -165,6 +171,25 @@ struct RhoReq {
 template <typename T>
 int mf_smooth_cheb_rho(const MfSmooth& m, const T* x_in, T* x_out, const T* b, const T* dinv, T* d, T c1, T c2,
                        const RhoReq& rq, const int* skip, hipStream_t s);
+// The smoothing chain of the patch layout (mf_smooth_chain: whether it can
+// run): a product of x, steps that complete the product in buffer `from` (0
+// or 1, the product's is 0) as a Chebyshev step and form the product of its
+// result in the other buffer, and the node kernel that completes the last.  A
+// step's x_out, d_out are buffers of their own (mf_smooth_d2: a second d);
+// dinv null: the unit diagonal.
+template <typename T> T* mf_smooth_d2(const MfSmooth& m);
+template <> double* mf_smooth_d2<double>(const MfSmooth& m);
+template <> float* mf_smooth_d2<float>(const MfSmooth& m);
+template <typename T> bool mf_smooth_chain(const MfSmooth& m);
+template <typename T> int mf_smooth_product(const MfSmooth& m, const T* x, const int* skip, hipStream_t s);
+template <typename T>
+int mf_smooth_step(const MfSmooth& m, int from, const T* x, T* x_out, const T* b, const T* dinv, const T* d, T* d_out,
+                   T c1, T c2, const int* skip, hipStream_t s);
+template <typename T>
+int mf_smooth_end_defect(const MfSmooth& m, int from, const T* x, const T* b, T* res, const int* skip, hipStream_t s);
+template <typename T>
+int mf_smooth_end_cheb(const MfSmooth& m, int from, const T* x, T* x_out, const T* b, const T* dinv, T* d, T c1, T c2,
+                       const RhoReq* rq, const int* skip, hipStream_t s);
 // Partials mf_smooth_cheb_rho writes in precision T (0: it cannot run).
 template <typename T>
 int mf_smooth_rho_blocks(const MfSmooth& m);
