@@ -1963,35 +1963,6 @@ int mf_smooth_defect(const MfSmooth& m, const T* x, const T* b, T* res, const in
   return mf_smooth_run<T>(m, x, o, skip, s);
 }
 
-// A Chebyshev step (as OpCheb) that also forms the partials of
-// rho = r . (S z), z = the step's x_out as stored: the V-cycle's last step
-// hands the CG iteration its rho without a pass over r, S and z of its own.
-// Per DOF the same product as the separate rho kernel, r (S z).
-template <typename T, bool Unit = false>
-struct OpChebRho {
-  static constexpr int kDots = 1;
-  OpCheb<3, T, Unit> c;
-  const double* r;
-  const double* scale;
-  double* partials;
-  struct Pre {
-    typename OpCheb<3, T, Unit>::Pre c;
-    double r, s;
-  };
-  __device__ __forceinline__ void load(long long k, Pre& p) const {
-    c.load(k, p.c);
-    p.r = r[k];
-    p.s = scale ? scale[k] : 1.0;
-  }
-  __device__ __forceinline__ void out(long long k, T a, double (&dots)[2], const Pre& p) const {
-    const T dn = c.c1 * p.c.d + c.c2 * p.c.dinv * (p.c.b - a);
-    const T xo = p.c.x + dn;
-    c.d[k] = dn;
-    c.x_out[k] = xo;
-    dots[0] += p.r * (double(xo) * p.s);
-  }
-};
-
 // The smoothing chain of the patch layout: a product (mf_smooth_product),
 // steps that complete one product and form the next (mf_smooth_step), and a
 // node kernel that completes the last (mf_smooth_end_*).  `from` names the
@@ -2050,8 +2021,8 @@ int mf_smooth_end_cheb(const MfSmooth& m, int from, const T* x, T* x_out, const 
                        const RhoReq* rq, const int* skip, hipStream_t s) {
   const OpCheb<3, T> o{b, dinv, x, x_out, d, c1, c2};
   const OpCheb<3, T, true> u{b, nullptr, x, x_out, d, c1, c2};
-  if (rq && !dinv) return mf_smooth_end<T>(m, from, x, OpChebRho<T, true>{u, rq->r, rq->scale, rq->partials}, skip, s);
-  if (rq) return mf_smooth_end<T>(m, from, x, OpChebRho<T>{o, rq->r, rq->scale, rq->partials}, skip, s);
+  if (rq && !dinv) return mf_smooth_end<T>(m, from, x, OpChebRho<3, T, true>{u, rq->r, rq->scale, rq->partials}, skip, s);
+  if (rq) return mf_smooth_end<T>(m, from, x, OpChebRho<3, T>{o, rq->r, rq->scale, rq->partials}, skip, s);
   return dinv ? mf_smooth_end<T>(m, from, x, o, skip, s) : mf_smooth_end<T>(m, from, x, u, skip, s);
 }
 
@@ -2082,12 +2053,12 @@ int mf_smooth_cheb_rho(const MfSmooth& m, const T* x_in, T* x_out, const T* b, c
   launch_patch<T, std::is_same<T, float>::value>(op, qdp, StageScaled<T>{mf_scale_in<T>(m), x_in}, part, skip, s);
   const dim3 grid(node_grid(op.n_nodes));
   if (!dinv) {
-    const OpChebRho<T, true> o{{b, nullptr, x_in, x_out, d, c1, c2}, rq.r, rq.scale, rq.partials};
-    hipLaunchKernelGGL((mf_node_kernel<T, OpChebRho<T, true>>), grid, dim3(kNodeThreads), 0, s, op.n_nodes,
+    const OpChebRho<3, T, true> o{{b, nullptr, x_in, x_out, d, c1, c2}, rq.r, rq.scale, rq.partials};
+    hipLaunchKernelGGL((mf_node_kernel<T, OpChebRho<3, T, true>>), grid, dim3(kNodeThreads), 0, s, op.n_nodes,
                        op.nhead, op.novf, part, op.fix, mf_scale<T>(m), x_in, o, skip);
   } else {
-    const OpChebRho<T> o{{b, dinv, x_in, x_out, d, c1, c2}, rq.r, rq.scale, rq.partials};
-    hipLaunchKernelGGL((mf_node_kernel<T, OpChebRho<T>>), grid, dim3(kNodeThreads), 0, s, op.n_nodes, op.nhead,
+    const OpChebRho<3, T> o{{b, dinv, x_in, x_out, d, c1, c2}, rq.r, rq.scale, rq.partials};
+    hipLaunchKernelGGL((mf_node_kernel<T, OpChebRho<3, T>>), grid, dim3(kNodeThreads), 0, s, op.n_nodes, op.nhead,
                        op.novf, part, op.fix, mf_scale<T>(m), x_in, o, skip);
   }
   return static_cast<int>(hipGetLastError());

@@ -390,12 +390,17 @@ int spmv_residual64(const SellMatrix& A, const double* x, const double* b, doubl
 
 template <typename VT, typename T>
 int spmv_cheb(const SellMatrix& A, const T* x_in, T* x_out, const T* b, const T* dinv, T* d, double c1, double c2,
-              const SpmvTune& t, hipStream_t s) {
+              const SpmvTune& t, hipStream_t s, const RhoReq* rq) {
   if (A.br != A.bc) return kBadArg;
-#define CALL(R, C)                                                  \
-  {                                                                 \
-    OpCheb<R, T> op{b, dinv, x_in, x_out, d, T(c1), T(c2)};         \
-    return launch_sell<R, C, VT, T>(A, x_in, op, t, s);             \
+#define CALL(R, C)                                                                                          \
+  {                                                                                                         \
+    OpCheb<R, T> op{b, dinv, x_in, x_out, d, T(c1), T(c2)};                                                 \
+    if constexpr (std::is_same<VT, T>::value) {                                                             \
+      if (rq) {                                                                                             \
+        return launch_sell<R, C, VT, T>(A, x_in, OpChebRho<R, T>{op, rq->r, rq->scale, rq->partials}, t, s); \
+      }                                                                                                     \
+    }                                                                                                       \
+    return rq ? (int)kBadMode : launch_sell<R, C, VT, T>(A, x_in, op, t, s);                                \
   }
   if (A.br == 3) CALL(3, 3) else if (A.br == 6) CALL(6, 6) else return kBadArg;
 #undef CALL
@@ -451,7 +456,7 @@ int spmv_restrict_first(const SellMatrix& A, const T* x, T* y, const T* dinv, T*
 
 #define WN_VINST(VT, T)                                                                                          \
   template int spmv_cheb<VT, T>(const SellMatrix&, const T*, T*, const T*, const T*, T*, double, double,       \
-                                const SpmvTune&, hipStream_t);                                                 \
+                                const SpmvTune&, hipStream_t, const RhoReq*);                                \
   template int spmv_defect<VT, T>(const SellMatrix&, const T*, const T*, T*, const SpmvTune&, hipStream_t);   \
   template int spmv_addto<VT, T>(const SellMatrix&, const T*, T*, const SpmvTune&, hipStream_t);              \
   template int spmv_restrict<VT, T>(const SellMatrix&, const T*, T*, const SpmvTune&, hipStream_t);           \

@@ -433,6 +433,44 @@ struct OpCheb {
   }
 };
 
+// OpCheb, also writing the partials of rho = r . (S x_out), S a per-DOF scale
+// (may be null): the last smoothing step of a preconditioner cycle hands the
+// CG iteration its rho without a pass over r, S and z of its own.  Per DOF the
+// same product as the separate rho kernel, r (S z).
+template <int BR, typename T, bool Unit = false>
+struct OpChebRho {
+  static constexpr int kDots = 1;
+  OpCheb<BR, T, Unit> c;
+  const double* r;
+  const double* scale;
+  double* partials;
+  struct Pre {
+    typename OpCheb<BR, T, Unit>::Pre c;
+    double r, s;
+  };
+  __device__ __forceinline__ void load(long long k, Pre& p) const {
+    c.load(k, p.c);
+    p.r = r[k];
+    p.s = scale ? scale[k] : 1.0;
+  }
+  __device__ __forceinline__ void out(long long k, T a, double (&dots)[2], const Pre& p) const {
+    const T dn = c.c1 * p.c.d + c.c2 * p.c.dinv * (p.c.b - a);
+    const T xo = p.c.x + dn;
+    c.d[k] = dn;
+    c.x_out[k] = xo;
+    dots[0] += p.r * (double(xo) * p.s);
+  }
+  __device__ __forceinline__ void row(int i, const T (&acc)[BR], double (&dots)[2], int q, int L) const {
+#pragma unroll
+    for (int j = 0; j < BR; ++j) {
+      if ((j & (L - 1)) != q) continue;
+      Pre p;
+      load((long long)i * BR + j, p);
+      out((long long)i * BR + j, acc[j], dots, p);
+    }
+  }
+};
+
 // res = b - A x (working precision), written to `res`.
 template <int BR, typename T>
 struct OpDefect {

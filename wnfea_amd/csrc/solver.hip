@@ -298,15 +298,14 @@ static int vcycle(Amg& g, int l, const T* b, T* x, const int* skip, hipStream_t 
   T* oth = (cur == x) ? tmp : x;
   // the finest level of an FP32 / FP64 cycle may run its products matrix-free
   const bool mf = l == 0 && std::is_same<VT, T>::value && mf_smooth_ready<T>(g.mfs);
-  // rq: the last post-smoothing step (matrix-free, patch layout) also writes
-  // the partials of rho = r . (S x) for the Krylov loop
-  if (rq && !mf) return kBadMode;
+  // rq: the last post-smoothing step also writes the partials of
+  // rho = r . (S x) for the Krylov loop (see amg_rho_blocks)
   // a unit inverse diagonal is passed to the matrix-free steps as null
   const T* dinv_mf = level_unit<T>(L) ? nullptr : dinv;
   auto cheb = [&](const T* xi, T* xo, int k, const RhoReq* q = nullptr) -> int {
     if (mf && q) return mf_smooth_cheb_rho<T>(g.mfs, xi, xo, b, dinv_mf, d, T(c.c1[k]), T(c.c2[k]), *q, skip, s);
     if (mf) return mf_smooth_cheb<T>(g.mfs, xi, xo, b, dinv_mf, d, T(c.c1[k]), T(c.c2[k]), skip, s);
-    return spmv_cheb<VS, T>(A, xi, xo, b, dinv, d, c.c1[k], c.c2[k], t, s);
+    return spmv_cheb<VS, T>(A, xi, xo, b, dinv, d, c.c1[k], c.c2[k], t, s, q);
   };
   if (!first_done) {
     hipLaunchKernelGGL(cheb_first_kernel<T>, dim3(vec_grid(n)), dim3(256), 0, s, n, b, dinv, d, cur, T(c.c2[0]),
@@ -398,12 +397,16 @@ template int amg_first_launch<double>(const FirstIter<double>&, long long, const
 template int amg_first_launch<float>(const FirstIter<float>&, long long, const float*, const int*, hipStream_t);
 
 // Partials the cycle of kind vt writes for a RhoReq (0: that cycle cannot
-// form rho: its finest level is not smoothed matrix-free in the patch layout,
-// or vt is not 0 or 1).
+// form rho: its values and vectors differ in type, or its finest level is
+// smoothed matrix-free element by element).
+template <typename T>
+static int rho_blocks(const Amg& g) {
+  return mf_smooth_ready<T>(g.mfs) ? mf_smooth_rho_blocks<T>(g.mfs) : spmv_partials<T>(*g.L[0]->A, g.tune);
+}
 int amg_rho_blocks(const Amg& g, int vt) {
   if (g.L.size() < 2) return 0;
-  if (vt == 0) return (g.store & 1) ? mf_smooth_rho_blocks<double>(g.mfs) : 0;
-  if (vt == 1) return (g.store & 2) ? mf_smooth_rho_blocks<float>(g.mfs) : 0;
+  if (vt == 0) return (g.store & 1) ? rho_blocks<double>(g) : 0;
+  if (vt == 1) return (g.store & 2) ? rho_blocks<float>(g) : 0;
   return 0;
 }
 
@@ -522,7 +525,8 @@ static void key_mf(std::vector<uint64_t>& k, const MfOp& m) {
                         (const void*)m.fix, (const void*)m.E, (const void*)m.nu, (const void*)m.n2e,
                         (const void*)m.n2e_ptr, (const void*)m.chunk, (const void*)m.pe, (const void*)m.pnode,
                         (const void*)m.pconn, (const void*)m.poff, (const void*)m.pslot, (const void*)m.nhead,
-                        (const void*)m.novf, (const void*)m.qdp, (const void*)m.part})
+                        (const void*)m.novf, (const void*)m.qdp, (const void*)m.part, (const void*)m.part2,
+                        (const void*)m.phead})
     key_push(k, p);
   for (int v : {m.M, m.n_nodes, m.n_chunks, m.affine, m.patch, m.n_patch, m.stride, m.n_local, m.gen}) key_push(k, v);
 }
@@ -535,7 +539,8 @@ static void key_amg(std::vector<uint64_t>& k, const Amg* g) {
                         (const void*)g->tij, (const void*)g->tpart, (const void*)g->mfs.op,
                         (const void*)g->mfs.s64, (const void*)g->mfs.s64e, (const void*)g->mfs.s32,
                         (const void*)g->mfs.s32e, (const void*)g->mfs.qd32, (const void*)g->mfs.fe32,
-                        (const void*)g->mfs.qdp32, (const void*)g->mfs.part32})
+                        (const void*)g->mfs.qdp32, (const void*)g->mfs.part32, (const void*)g->mfs.part32b,
+                        (const void*)g->mfs.d32b, (const void*)g->mfs.d64b})
     key_push(k, p);
   key_push(k, g->mfs.gen);
   if (g->mfs.op) key_mf(k, *g->mfs.op);
@@ -599,8 +604,10 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
   // q = A p of the previous iteration in the rho kernel
   const bool flexible = pkind == 2 && amg_vt == 5;
   // rho from the cycle's last smoothing step (FP64 Krylov vectors, a
-  // symmetric cycle whose finest level is smoothed matrix-free in the patch
-  // layout): that step writes the rho partials, the rho pass is skipped
+  // symmetric cycle): that step writes the rho partials, which costs it a read
+  // of r and S it does not otherwise need but saves the rho pass and its
+  // launch (lattice of 35 937 6-DOF nodes, assembled: 2 of 5.6 us per
+  // iteration; 144k-row FP64 solid 1.8 of 5.7)
   const int nb_cycle_rho =
       (pkind == 2 && amg && !flexible && std::is_same<T, double>::value) ? amg_rho_blocks(*amg, amg_vt) : 0;
   if ((r = S.ws.alloc(std::max((mf ? mf_grid(*mf) : A.n_slices), nb_cycle_rho) + 8))) return r;

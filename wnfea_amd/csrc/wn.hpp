@@ -160,7 +160,8 @@ template <typename T>
 int mf_smooth_defect(const MfSmooth& m, const T* x, const T* b, T* res, const int* skip, hipStream_t s);
 // Partials of rho = r . (S z) requested from the Chebyshev step that writes
 // a V-cycle's output z (scale null: S = I); nb partials, see
-// mf_smooth_rho_blocks.
+// mf_smooth_rho_blocks and spmv_partials.  spmv_cheb takes it with values of
+// the vectors' type only.
 struct RhoReq {
   const double* r;
   const double* scale;
@@ -294,7 +295,7 @@ int spmv_residual64(const SellMatrix& A, const double* x, const double* b, doubl
 // T the vector/arithmetic type (double for VT = double, float otherwise).
 template <typename VT, typename T>
 int spmv_cheb(const SellMatrix& A, const T* x_in, T* x_out, const T* b, const T* dinv, T* d, double c1, double c2,
-              const SpmvTune& t, hipStream_t s);
+              const SpmvTune& t, hipStream_t s, const RhoReq* rq = nullptr);
 template <typename VT, typename T>
 int spmv_defect(const SellMatrix& A, const T* x, const T* b, T* res, const SpmvTune& t, hipStream_t s);
 template <typename VT, typename T> int spmv_addto(const SellMatrix& A, const T* e, T* x, const SpmvTune& t,
