@@ -275,21 +275,37 @@ int equilibrate(SellMatrix& A, const int* d_rowidx, const int* d_colidx, const d
 }
 
 // ---------------------------------------------------------------- SpMV dispatch
-template <int BR, int BC, typename VT, typename XT, int W, class Op>
-static void launch_w(const SellView<VT>& v, const XT* x, const Op& op, int grid, int unroll, int xcd, const int* flags,
+template <int BR, int BC, typename VT, typename XT, int W, int K, class Op>
+static void launch_k(const SellView<VT>& v, const XT* x, const Op& op, int grid, int unroll, int xcd, const int* flags,
                      int guard, hipStream_t s) {
   // keep the unrolled value registers within budget: U*BB values of VT
   constexpr int kMaxU = (BR * BC * (int)sizeof(VT) <= 48) ? 4 : ((BR * BC * (int)sizeof(VT) <= 160) ? 2 : 1);
   const int u = std::min(unroll, kMaxU);
   if (u >= 4 && kMaxU >= 4)
-    hipLaunchKernelGGL((sell_spmv_kernel<BR, BC, VT, XT, W, (kMaxU >= 4 ? 4 : 1), Op>), dim3(grid), dim3(64 * W), 0,
+    hipLaunchKernelGGL((sell_spmv_kernel<BR, BC, VT, XT, W, (kMaxU >= 4 ? 4 : 1), K, Op>), dim3(grid), dim3(64 * W), 0,
                        s, v, x, op, xcd, flags, guard);
   else if (u >= 2 && kMaxU >= 2)
-    hipLaunchKernelGGL((sell_spmv_kernel<BR, BC, VT, XT, W, (kMaxU >= 2 ? 2 : 1), Op>), dim3(grid), dim3(64 * W), 0,
+    hipLaunchKernelGGL((sell_spmv_kernel<BR, BC, VT, XT, W, (kMaxU >= 2 ? 2 : 1), K, Op>), dim3(grid), dim3(64 * W), 0,
                        s, v, x, op, xcd, flags, guard);
   else
-    hipLaunchKernelGGL((sell_spmv_kernel<BR, BC, VT, XT, W, 1, Op>), dim3(grid), dim3(64 * W), 0, s, v, x, op, xcd,
+    hipLaunchKernelGGL((sell_spmv_kernel<BR, BC, VT, XT, W, 1, K, Op>), dim3(grid), dim3(64 * W), 0, s, v, x, op, xcd,
                        flags, guard);
+}
+
+// K, the outputs whose epilogue operands a lane holds: one where a row has a
+// lane per output, else up to BR (short rows, two or four lanes a row).
+// Loading them before the block stream, as the first case does, takes a
+// trailing latency off each of the beam lattice's products, seven blocks a row
+// (its tangent solve 18.58 -> 18.05 ms), and of the I-beam's transfers (its
+// solve 18.41 -> 18.23 ms); held by every kernel they would cost the long rows
+// registers they have no use for.
+template <int BR, int BC, typename VT, typename XT, int W, class Op>
+static void launch_w(const SellView<VT>& v, const XT* x, const Op& op, int grid, int unroll, int xcd, const int* flags,
+                     int guard, hipStream_t s) {
+  if (v.lanes >= BR)
+    launch_k<BR, BC, VT, XT, W, 1>(v, x, op, grid, unroll, xcd, flags, guard, s);
+  else
+    launch_k<BR, BC, VT, XT, W, BR>(v, x, op, grid, unroll, xcd, flags, guard, s);
 }
 
 template <typename VT>

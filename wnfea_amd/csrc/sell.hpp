@@ -151,7 +151,7 @@ __device__ __forceinline__ bool guard_skip(const int* flags, int mode) {
 // gathers, then the FMAs) to cover memory latency.  `Op` receives (block row,
 // accumulated BR values) for every real row and may add to up to two fused
 // dot products, reduced deterministically.
-template <int BR, int BC, typename VT, typename XT, int W, int U, class Op>
+template <int BR, int BC, typename VT, typename XT, int W, int U, int K, class Op>
 __global__ __launch_bounds__(64 * W) void sell_spmv_kernel(SellView<VT> A, const XT* __restrict__ x, Op op,
                                                            int xcd_remap, const int* flags, int guard) {
   if (guard_skip(flags, guard)) return;
@@ -176,13 +176,15 @@ __global__ __launch_bounds__(64 * W) void sell_spmv_kernel(SellView<VT> A, const
     const int q = lane / rps;
     const int len = lane_steps(ri.y, q, A.lanes);  // steps of this lane
     const long long base = A.off[s];
-    // With at least BR lanes per row each output has its own lane (output q
-    // on sub-lane q): its epilogue operands are loaded now, so that their
-    // latency hides behind the block stream instead of trailing it.
-    const bool one_out = A.lanes >= BR;
-    const bool has_out = wave == 0 && ri.x >= 0 && q < BR;
-    typename Op::Pre pre{};
-    if (one_out && has_out) op.load((long long)ri.x * BR + q, pre);
+    // The row's L lanes share its BR outputs: outputs q, q + L, ... on sub-lane
+    // q, K of them at most (1 where L >= BR).  Their epilogue operands are
+    // loaded now, so that their latency hides behind the block stream instead
+    // of trailing it.
+    const bool has_row = wave == 0 && ri.x >= 0;
+    typename Op::Pre pre[K] = {};
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (has_row && q + k * A.lanes < BR) op.load((long long)ri.x * BR + q + k * A.lanes, pre[k]);
     AT acc[BR];
 #pragma unroll
     for (int r = 0; r < BR; ++r) acc[r] = AT(0);
@@ -249,19 +251,17 @@ __global__ __launch_bounds__(64 * W) void sell_spmv_kernel(SellView<VT> A, const
     for (int off = 32; off >= rps; off >>= 1)
 #pragma unroll
       for (int r = 0; r < BR; ++r) acc[r] += __shfl_xor(acc[r], off, 64);
-    const int row = ri.x;
-    // every lane of the row holds the full sums after the butterfly: the row's
-    // L lanes share its BR outputs (output r on sub-lane r mod L)
-    if (one_out) {
-      if (has_out) {
+    // every lane of the row holds the full sums after the butterfly
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int o = q + k * A.lanes;
+      if (has_row && o < BR) {
         AT a = acc[0];
 #pragma unroll
         for (int r = 1; r < BR; ++r)
-          if (q == r) a = acc[r];
-        op.out((long long)row * BR + q, a, dot, pre);
+          if (o == r) a = acc[r];
+        op.out((long long)ri.x * BR + o, a, dot, pre[k]);
       }
-    } else if (wave == 0 && row >= 0) {
-      op.row(row, acc, dot, q, A.lanes);
     }
   }
   if constexpr (Op::kDots > 0) {
@@ -286,16 +286,6 @@ struct OpAxpby {
   __device__ __forceinline__ void out(long long k, AT a, double (&)[2], const Pre& p) const {
     y[k] = YT(alpha * a + beta * p.y);
   }
-  __device__ __forceinline__ void row(int i, const AT (&acc)[BR], double (&)[2], int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r) {
-      if ((r & (L - 1)) != q) continue;
-      const long long k = (long long)i * BR + r;
-      AT v = alpha * acc[r];
-      if (beta != AT(0)) v += beta * AT(y[k]);
-      y[k] = YT(v);
-    }
-  }
 };
 
 // y = R x (restriction) and, from it, the coarse level's first Chebyshev
@@ -319,14 +309,6 @@ struct OpRestrictFirst {
     x1[k] = v;
   }
   __device__ __forceinline__ void out(long long k, AT a, double (&)[2], const Pre& p) const { put(k, T(a), p.dinv); }
-  __device__ __forceinline__ void row(int i, const AT (&acc)[BR], double (&)[2], int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r) {
-      if ((r & (L - 1)) != q) continue;
-      const long long k = (long long)i * BR + r;
-      put(k, T(acc[r]), dinv[k]);
-    }
-  }
 };
 
 // y = A p and gamma = p . (A p) (block partials; the finaliser forms alpha = rho / gamma).
@@ -341,15 +323,6 @@ struct OpSpmvDot {
   __device__ __forceinline__ void out(long long k, AT a, double (&d)[2], const Pre& pr) const {
     y[k] = YT(a);
     d[0] += pr.p * double(a);
-  }
-  __device__ __forceinline__ void row(int i, const AT (&acc)[BR], double (&d)[2], int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r) {
-      if ((r & (L - 1)) != q) continue;
-      const long long k = (long long)i * BR + r;
-      y[k] = YT(acc[r]);
-      d[0] += double(p[k]) * double(acc[r]);
-    }
   }
 };
 
@@ -375,19 +348,6 @@ struct OpResidual {
     if (rs) rs[k] = float(vs);
     d[0] += v * v;
     d[1] += vs * vs;
-  }
-  __device__ __forceinline__ void row(int i, const AT (&acc)[BR], double (&d)[2], int q, int L) const {
-#pragma unroll
-    for (int r0 = 0; r0 < BR; ++r0) {
-      if ((r0 & (L - 1)) != q) continue;
-      const long long k = (long long)i * BR + r0;
-      const double v = b[k] - double(acc[r0]);
-      const double vs = scale ? scale[k] * v : v;
-      if (r) r[k] = v;
-      if (rs) rs[k] = float(vs);
-      d[0] += v * v;
-      d[1] += vs * vs;
-    }
   }
 };
 
@@ -420,17 +380,6 @@ struct OpCheb {
     d[k] = dn;
     x_out[k] = p.x + dn;
   }
-  __device__ __forceinline__ void row(int i, const T (&acc)[BR], double (&)[2], int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r) {
-      if ((r & (L - 1)) != q) continue;
-      const long long k = (long long)i * BR + r;
-      const T res = b[k] - acc[r];
-      const T dn = c1 * d[k] + c2 * (Unit ? T(1) : dinv[k]) * res;
-      d[k] = dn;
-      x_out[k] = x_in[k] + dn;
-    }
-  }
 };
 
 // OpCheb, also writing the partials of rho = r . (S x_out), S a per-DOF scale
@@ -460,15 +409,6 @@ struct OpChebRho {
     c.x_out[k] = xo;
     dots[0] += p.r * (double(xo) * p.s);
   }
-  __device__ __forceinline__ void row(int i, const T (&acc)[BR], double (&dots)[2], int q, int L) const {
-#pragma unroll
-    for (int j = 0; j < BR; ++j) {
-      if ((j & (L - 1)) != q) continue;
-      Pre p;
-      load((long long)i * BR + j, p);
-      out((long long)i * BR + j, acc[j], dots, p);
-    }
-  }
 };
 
 // res = b - A x (working precision), written to `res`.
@@ -481,14 +421,6 @@ struct OpDefect {
   struct Pre { T b; };
   __device__ __forceinline__ void load(long long k, Pre& p) const { p.b = b[k]; }
   __device__ __forceinline__ void out(long long k, T a, double (&)[2], const Pre& p) const { res[k] = p.b - a; }
-  __device__ __forceinline__ void row(int i, const T (&acc)[BR], double (&)[2], int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r) {
-      if ((r & (L - 1)) != q) continue;
-      const long long k = (long long)i * BR + r;
-      res[k] = b[k] - acc[r];
-    }
-  }
 };
 
 // x += A e (prolongation: the gathered vector is the coarse correction).
@@ -500,11 +432,6 @@ struct OpAddTo {
   struct Pre { T x; };
   __device__ __forceinline__ void load(long long k, Pre& p) const { p.x = x[k]; }
   __device__ __forceinline__ void out(long long k, T a, double (&)[2], const Pre& p) const { x[k] = p.x + a; }
-  __device__ __forceinline__ void row(int i, const T (&acc)[BR], double (&)[2], int q, int L) const {
-#pragma unroll
-    for (int r = 0; r < BR; ++r)
-      if ((r & (L - 1)) == q) x[(long long)i * BR + r] += acc[r];
-  }
 };
 
 }  // namespace wn
