@@ -1,0 +1,33 @@
+"""Dense coarsest product: by rows up to 32 MB of inverse, by packed symmetric
+64 x 64 tiles beyond.  Hierarchies of one level on both sides of the line in
+FP64 (2 048 rows) and FP32 (2 896), at sizes that leave a partial last tile and
+a partial last round of a row; the cycle must be inv @ r, in FP32 of the
+inverse rounded to FP32 with the sum in FP64 and the result rounded once."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cells,rows", [((1, 1, 1), 81), ((16, 2, 2), 2475), ((20, 2, 2), 3075)])
+def test_cycle_is_the_inverse_product(cells, rows):
+    import torch
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr, build_amg
+    print(f"coarsest product of {rows} rows", flush=True)
+    m, _ = generate_c3d10_structured_block(1.0, 0.1, 0.1, *cells, tip_load_total=-1000.0, tets_per_hex=6,
+                                           load_direction="z")
+    amg = build_amg(assemble_c3d10_bsr(m, want_fp64_equilibrated=True), storage=("fp64", "fp32"), autotune=False)
+    inv = amg.coarse_inv
+    assert len(amg.levels) == 1 and inv.shape[0] == rows
+    r = np.random.default_rng(rows).standard_normal(rows)
+    z = amg.vcycle(torch.as_tensor(r, device="cuda")).cpu().numpy()
+    # a sum of `rows` products in another order: rows * eps of the sum of magnitudes
+    assert np.all(np.abs(z - inv @ r) <= rows * 2.3e-16 * (np.abs(inv) @ np.abs(r)))
+    r32, inv32 = r.astype(np.float32), inv.astype(np.float32).astype(np.float64)
+    z32 = amg.vcycle(torch.as_tensor(r32, device="cuda")).double().cpu().numpy()
+    ref = inv32 @ r32.astype(np.float64)
+    # one rounding of the result to FP32, plus the FP64 sum's as above
+    mag = np.abs(inv32) @ np.abs(r32.astype(np.float64))
+    assert np.all(np.abs(z32 - ref) <= 6.0e-8 * np.abs(ref) + rows * 2.3e-16 * mag)
+    amg.close()

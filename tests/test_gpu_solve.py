@@ -301,10 +301,10 @@ def test_vcycle_low_precision_matches_rounded_mirror(c0_amg, storage):
 @pytest.mark.parametrize("storage", ["fp64", "fp32"])
 def test_coarse_only_cycle_is_inverse_product(storage):
     """A hierarchy of one level (1 575 DOF, below the coarse size): the cycle
-    is the packed symmetric tile product of the exact inverse, so it must equal
-    inv @ r (FP64: to round-off; FP32: against the inverse rounded to FP32,
-    the result rounded once).  1 575 = 24 * 64 + 39 exercises a partial last
-    tile and off-diagonal tiles on both sides."""
+    is the dense product with the exact inverse (by rows at this size), so it
+    must equal inv @ r (FP64: to round-off; FP32: against the inverse rounded
+    to FP32, the result rounded once).  1 575 is no multiple of a row's 256
+    threads."""
     import torch
     from wnfea_amd.mesh.rcm import apply_rcm_to_model
     from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block

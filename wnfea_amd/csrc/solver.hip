@@ -55,18 +55,33 @@ __global__ void cheb_first_kernel(long long n, const T* __restrict__ b, const T*
 
 // x = inv * b on the coarsest level: one 256-thread block per row; the
 // inverse is stored in the cycle's type T (its bytes dominate), the dot
-// product accumulates in FP64.
-template <typename T>
+// product accumulates in FP64.  Bound by latency at the sizes that take it
+// (see coarse_apply), so up to 2048 columns are one round of loads in flight
+// (clamped, so that no branch splits the round).
+template <typename T, typename XT = T>
 __global__ __launch_bounds__(256) void coarse_gemv_kernel(int n, const T* __restrict__ inv,
-                                                          const T* __restrict__ b, T* __restrict__ x,
+                                                          const XT* __restrict__ b, XT* __restrict__ x,
                                                           const int* skip) {
   if (skip && *skip) return;
-  const int i = blockIdx.x;
+  constexpr int U = 8;
+  const T* row = inv + (size_t)blockIdx.x * n;
   double s = 0.0;
-  for (int j = threadIdx.x; j < n; j += blockDim.x) s += double(inv[(size_t)i * n + j]) * double(b[j]);
+  for (int base = threadIdx.x; base < n; base += 256 * U) {
+    T a[U];
+    XT v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = min(base + 256 * u, n - 1);
+      a[u] = row[j];
+      v[u] = b[j];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (base + 256 * u < n) s += double(a[u]) * double(v[u]);
+  }
   __shared__ double sm[4];
   s = block_sum(s, sm);
-  if (threadIdx.x == 0) x[i] = T(s);
+  if (threadIdx.x == 0) x[blockIdx.x] = XT(s);
 }
 
 // ---- packed symmetric coarse inverse ----------------------------------------
@@ -228,30 +243,38 @@ __global__ __launch_bounds__(kTile * kRedGroups) void sym_tile_reduce_kernel(int
   }
 }
 
+// Inverses up to this many bytes are applied by rows, in one kernel; larger
+// ones by symmetric tiles, which read half as much but take a second kernel
+// for the tiles' partial sums.  The line is what the eight L2s hold together
+// (32 MB).  A cycle that is this product alone, tiles against rows: FP32 567
+// rows 10.3 against 8.2 us, 2475 10.5 / 8.3, 3675 10.5 / 10.2, 4851 13.1 /
+// 16.2; FP64 1275 rows 10.9 / 8.5, 2475 10.6 / 11.6, 3675 13.4 / 17.5.
+constexpr size_t kCoarseRowBytes = size_t(32) << 20;
+
+// M: the inverse's type, T: the vectors'
+template <typename M, typename T>
+static int coarse_apply_as(const Amg& g, const T* b, T* x, const int* skip, hipStream_t s) {
+  const M* inv = coarse_inv<M>(g);
+  const M* tiles = coarse_tiles<M>(g);
+  const size_t bytes = sizeof(M) * (size_t)g.n_coarse * g.n_coarse;
+  if (inv && (bytes <= kCoarseRowBytes || !tiles || !g.tpart || !g.tij)) {
+    hipLaunchKernelGGL((coarse_gemv_kernel<M, T>), dim3(std::max(g.n_coarse, 1)), dim3(256), 0, s, g.n_coarse, inv, b,
+                       x, skip);
+    return static_cast<int>(hipGetLastError());
+  }
+  if (!tiles) return kNotReady;
+  hipLaunchKernelGGL((sym_tile_gemv_kernel<M, T>), dim3((unsigned)g.ntiles), dim3(256), 0, s, g.n_coarse, tiles, g.tij,
+                     b, g.tpart, skip);
+  hipLaunchKernelGGL(sym_tile_reduce_kernel<T>, dim3(g.nt), dim3(kTile * kRedGroups), 0, s, g.n_coarse, g.nt, g.tpart,
+                     x, skip);
+  return static_cast<int>(hipGetLastError());
+}
 template <typename T>
 static int coarse_apply(const Amg& g, const T* b, T* x, const int* skip, hipStream_t s) {
   // an FP32 cycle with coarse_fp64 set applies the FP64 inverse (FP64
   // products and partial sums; only the vectors stay FP32)
-  if (std::is_same<T, float>::value && g.coarse_fp64 && g.tiles64 && g.tpart && g.tij) {
-    hipLaunchKernelGGL((sym_tile_gemv_kernel<double, T>), dim3((unsigned)g.ntiles), dim3(256), 0, s, g.n_coarse,
-                       g.tiles64, g.tij, b, g.tpart, skip);
-    hipLaunchKernelGGL(sym_tile_reduce_kernel<T>, dim3(g.nt), dim3(kTile * kRedGroups), 0, s, g.n_coarse, g.nt,
-                       g.tpart, x, skip);
-    return static_cast<int>(hipGetLastError());
-  }
-  const T* tiles = coarse_tiles<T>(g);
-  if (tiles && g.tpart && g.tij) {
-    hipLaunchKernelGGL(sym_tile_gemv_kernel<T>, dim3((unsigned)g.ntiles), dim3(256), 0, s, g.n_coarse, tiles, g.tij,
-                       b, g.tpart, skip);
-    hipLaunchKernelGGL(sym_tile_reduce_kernel<T>, dim3(g.nt), dim3(kTile * kRedGroups), 0, s, g.n_coarse, g.nt,
-                       g.tpart, x, skip);
-    return static_cast<int>(hipGetLastError());
-  }
-  const T* inv = coarse_inv<T>(g);
-  if (!inv) return kNotReady;
-  hipLaunchKernelGGL(coarse_gemv_kernel<T>, dim3(std::max(g.n_coarse, 1)), dim3(256), 0, s, g.n_coarse, inv, b, x,
-                     skip);
-  return static_cast<int>(hipGetLastError());
+  if (std::is_same<T, float>::value && g.coarse_fp64 && g.tiles64) return coarse_apply_as<double, T>(g, b, x, skip, s);
+  return coarse_apply_as<T, T>(g, b, x, skip, s);
 }
 
 // One V-cycle from level l.  VT: values of this level; VTC: values of every
