@@ -57,3 +57,42 @@ def test_cg_iterates(dpn, nx, precision, cycle):
     assert err <= (1e-11 if cycle == "fp64" else 1e-5), err
     amg.close()
     system.K.close()
+
+
+@pytest.mark.parametrize("dpn,cycle", [(3, "fp64"), (3, "fp32"), (6, "fp64"), (6, "fp32")])
+def test_carried_finalisation_changes_nothing(dpn, cycle):
+    """Chunks of one iteration finalise ||r||^2 in a launch of their own, longer
+    ones in the next iteration's first kernel: the same sums in the same order,
+    so the same bits and the same last iteration."""
+    import torch
+    from wnfea_amd.solver.solid_solver import build_amg, pcg_device
+    print(f"carried finalisation: {dpn}-blocks, {cycle} cycle", flush=True)
+    _, _, system = _system(dpn, 41)
+    amg = build_amg(system, storage=("fp64", "fp32"), autotune=False, coarse_size=150)
+    runs = [pcg_device(system, rtol=1e-9, preconditioner="amg", amg=amg, amg_precision=cycle, check_every=k)
+            for k in (1, 2, 5, 16)]
+    assert 5 < runs[0][1] < 200 and runs[0][2] <= 1e-9
+    for x, it, rel, _ in runs[1:]:
+        assert it == runs[0][1] and rel == runs[0][2] and torch.equal(x, runs[0][0])
+    amg.close()
+    system.K.close()
+
+
+@pytest.mark.parametrize("cells,cycle", [((9, 1, 1), "fp64"), ((20, 4, 4), "fp32"), ((57, 12, 8), "fp32")])
+def test_carried_finalisation_matrix_free(cells, cycle):
+    import torch
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block
+    from wnfea_amd.solver.solid_solver import MatrixFreeOperator, assemble_c3d10_bsr, build_amg, solve_mixed
+    print(f"carried finalisation on a box of {cells} cells, {cycle} cycle", flush=True)
+    nx, ny, nz = cells
+    m, _ = generate_c3d10_structured_block(0.025 * nx, 0.02 * ny, 0.02 * nz, nx, ny, nz, tip_load_total=-1000.0,
+                                           tets_per_hex=6, load_direction="z")
+    system = assemble_c3d10_bsr(m, want_fp64_equilibrated=True)
+    amg = build_amg(system, storage=("fp64", "fp32"), autotune=False, coarse_size=200)
+    op = MatrixFreeOperator(system)
+    op.attach_smoother(amg)
+    runs = [solve_mixed(system, amg, tol=1e-8, amg_precision=cycle, operator=op, check_every=k) for k in (1, 3, 16)]
+    for u, it, _, rel, _ in runs:
+        assert it == runs[0][1] and rel == runs[0][3] <= 1e-8 and torch.equal(u, runs[0][0])
+    op.close()
+    amg.close()

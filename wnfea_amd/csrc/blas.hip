@@ -140,10 +140,11 @@ template <typename T, typename RT>
 __global__ __launch_bounds__(kVecBlock) void update_xr_kernel(long long n, T* __restrict__ x, T* __restrict__ r,
                                                               const T* __restrict__ p, const T* __restrict__ q,
                                                               RT* __restrict__ rp, const double* __restrict__ scale,
-                                                              double* partials, double* sc, const int* flags,
+                                                              double* partials, double* sc, int* flags,
                                                               const double* __restrict__ gam_part, int nb_gam,
                                                               const RT* __restrict__ fdinv, RT* __restrict__ fx1,
                                                               RT* __restrict__ fd1, RT fc2) {
+  if (flags && blockIdx.x == 0 && threadIdx.x == 0) flags[2] = flags[0];  // see FinRR
   if (flags && flags[0]) return;
   double alpha_d = sc[kScAlpha];
   if (gam_part) {
@@ -219,19 +220,7 @@ __global__ __launch_bounds__(1024) void dot_finalize_kernel(const double* __rest
   __shared__ double red[2][16];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   for (int k = 0; k < K; ++k) {
-    // four independent accumulators keep several loads in flight per thread
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    const double* p = partials + (size_t)k * nb;
-    const int stride = blockDim.x;
-    int i = threadIdx.x;
-    for (; i + 3 * stride < nb; i += 4 * stride) {
-      a0 += p[i];
-      a1 += p[i + stride];
-      a2 += p[i + 2 * stride];
-      a3 += p[i + 3 * stride];
-    }
-    for (; i < nb; i += stride) a0 += p[i];
-    double s = (a0 + a1) + (a2 + a3);
+    double s = partial_sum4(partials + (size_t)k * nb, nb, threadIdx.x, blockDim.x);
     s = wave_sum(s);
     if (lane == 0) red[k][wid] = s;
   }
@@ -263,11 +252,7 @@ __global__ __launch_bounds__(1024) void dot_finalize_kernel(const double* __rest
       sc[kScAlpha] = v[0] != 0.0 ? sc[kScRho] / v[0] : 0.0;
       break;
     case kFinRR:
-      sc[kScRR] = v[0];
-      if (flags) {
-        flags[1] += 1;
-        if (v[0] <= sc[kScTol2] || !(v[0] == v[0])) flags[0] = 1;
-      }
+      fin_rr(sc, flags, v[0]);
       break;
     default:
       for (int k = 0; k < K; ++k) out[k] = v[k];
@@ -382,7 +367,8 @@ int launch_update_p(long long n, const ZT* z, const double* scale, T* p, Workspa
 }
 template <typename T, typename RT>
 int launch_update_xr(long long n, T* x, T* r, const T* p, const T* q, RT* rp, const double* scale, Workspace& w,
-                     int* flags, hipStream_t s, const double* gam_part, int nb_gam, const FirstIter<RT>* fi) {
+                     int* flags, hipStream_t s, const double* gam_part, int nb_gam, const FirstIter<RT>* fi,
+                     FinRR* later) {
   const int g = vec_grid(n);
   // the rr partials go past the region the gamma partials may occupy
   double* rr_part = gam_part ? w.partials + 2 * (size_t)w.max_blocks : w.partials;
@@ -391,6 +377,10 @@ int launch_update_xr(long long n, T* x, T* r, const T* p, const T* q, RT* rp, co
                      w.sc, flags, gam_part, nb_gam, f && !fi->unit ? fi->dinv : nullptr, f ? fi->x1 : nullptr,
                      f ? fi->d1 : nullptr, f ? fi->c2 : RT(0));
   int e = static_cast<int>(hipGetLastError());
+  if (later) {
+    *later = FinRR{rr_part, g, w.sc, flags};
+    return e;
+  }
   return e ? e : launch_finalize(rr_part, g, 1, kFinRR, nullptr, w.sc, flags, 0, flags, s);
 }
 template <typename T>
@@ -459,7 +449,7 @@ WN_INST(double)
   template int launch_update_p<T, U>(long long, const U*, const double*, T*, Workspace&, int, const int*,      \
                                      hipStream_t, const double*, int);                                         \
   template int launch_update_xr<T, U>(long long, T*, T*, const T*, const T*, U*, const double*, Workspace&,    \
-                                      int*, hipStream_t, const double*, int, const FirstIter<U>*);
+                                      int*, hipStream_t, const double*, int, const FirstIter<U>*, FinRR*);
 WN_INST2(double, double)
 WN_INST2(double, float)
 WN_INST2(float, float)

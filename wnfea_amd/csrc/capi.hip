@@ -37,7 +37,7 @@ struct Amg;
 struct AmgLevel;
 struct Solver;
 int amg_apply(Amg& g, int vt, const void* r, void* z, const int* skip, hipStream_t s, const RhoReq* rq,
-              bool first_done);
+              bool first_done, const FinRR* fin);
 int amg_level_cheb(Amg& g, int l, int vt, int reps, hipStream_t s);
 int amg_set_coarse_fp64(Amg& g, int fp64);
 template <typename T>
@@ -459,7 +459,7 @@ int wnfea_amg_tune_precision(void* h, int prec, int waves, int xcd_remap, int un
 // finest level and FP32 below, 4 = FP32 finest and FP16 below (vt >= 1: FP32 vectors)
 int wnfea_amg_vcycle(void* h, int vt, const void* r, void* z, void* stream) {
   if (!h || !r || !z) return kBadArg;
-  return amg_apply(*static_cast<Amg*>(h), vt, r, z, nullptr, S(stream), nullptr, false);
+  return amg_apply(*static_cast<Amg*>(h), vt, r, z, nullptr, S(stream), nullptr, false, nullptr);
 }
 
 // FP32 cycles: coarsest solve with the FP64 inverse (fp64 != 0) or its FP32 copy

@@ -96,4 +96,59 @@ enum FinMode : int {
   kFinRhoFlex = 4,  // rho and z.q_old: flexible (Polak-Ribiere) beta = -alpha (z.q_old) / rho_prev
 };
 
+// kFinRR carried by another kernel: the next iteration's first kernel launches
+// one block more, which finalises ||r||^2 beside that kernel's own work
+// instead of in a launch between the two.  The kernel's other blocks must not
+// read flags[0], which that block may set: they look at flags[2], the done
+// flag as the last update of x and r found it.  part null: nothing to do.
+// Saves that launch, 2.5 to 4.7 us of an iteration: box of 19 683 DOF
+// 1625 -> 1550 us a solve, 32-cell lattice 18.2 -> 17.75 ms, 144k-row FP64
+// solid 8.84 -> 8.72 ms.
+struct FinRR {
+  const double* part = nullptr;  // nb <= kFinRRMax partials
+  int nb = 0;
+  double* sc = nullptr;
+  int* flags = nullptr;
+};
+constexpr int kFinRRMax = 4096;
+
+__device__ __forceinline__ void fin_rr(double* sc, int* flags, double rr) {
+  sc[kScRR] = rr;
+  if (flags) {
+    flags[1] += 1;
+    if (rr <= sc[kScTol2] || !(rr == rr)) flags[0] = 1;
+  }
+}
+
+// thread t of `threads` of a finalising block: four independent accumulators
+// keep several loads in flight
+__device__ __forceinline__ double partial_sum4(const double* __restrict__ p, int nb, int t, int threads) {
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  int i = t;
+  for (; i + 3 * threads < nb; i += 4 * threads) {
+    a0 += p[i];
+    a1 += p[i + threads];
+    a2 += p[i + 2 * threads];
+    a3 += p[i + 3 * threads];
+  }
+  for (; i < nb; i += threads) a0 += p[i];
+  return (a0 + a1) + (a2 + a3);
+}
+
+// the extra block's work, whatever its size: the sums of a finalise launch's
+// 256 threads in the same order, so the same bits.  red: four doubles of LDS.
+__device__ __forceinline__ void fin_rr_block(const FinRR& f, double* red) {
+  if (f.flags[0]) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  for (int w = threadIdx.x / kWave; w < 4; w += blockDim.x / kWave) {
+    const double s = wave_sum(partial_sum4(f.part, f.nb, w * kWave + lane, 256));
+    if (lane == 0) red[w] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double v = 0.0;
+  for (int w = 0; w < 4; ++w) v += red[w];
+  fin_rr(f.sc, f.flags, v);
+}
+
 }  // namespace wn

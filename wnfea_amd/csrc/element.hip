@@ -1276,10 +1276,12 @@ __global__ __launch_bounds__(4 * P) void mf_patch_kernel(
     int n_patch, int M, int stride, const int* __restrict__ pnode, const ushort4* __restrict__ pconn,
     const unsigned short* __restrict__ poff, const uint2* __restrict__ pslot, const int* __restrict__ pe,
     const T* __restrict__ qdp, const double* __restrict__ E, const double* __restrict__ nu,
-    const int4* __restrict__ phead, Stage stage, T* __restrict__ part, const int* skip) {
+    const int4* __restrict__ phead, Stage stage, T* __restrict__ part, FinRR fin, const int* skip) {
   constexpr int NT = 4 * P, FS = force_stride<T>(), NC = 10 * P / 4;  // NC: 8-byte runs of slot codes
-  if (skip && *skip) return;
   extern __shared__ __align__(16) unsigned char patch_lds[];
+  if (fin.part && blockIdx.x == gridDim.x - 1)  // the block added for it
+    return fin_rr_block(fin, reinterpret_cast<double*>(patch_lds));
+  if (skip && *skip) return;
   T* xs = reinterpret_cast<T*>(patch_lds);                                    // [stride][4] scaled nodal values
   T* fl = xs + 4 * stride;                                                     // [P][10][FS] element forces
   unsigned short* ls = reinterpret_cast<unsigned short*>(fl + 10 * FS * P);  // [10 P] slot codes
@@ -1771,13 +1773,15 @@ static int patch_grid(int n_patch) { return 8 * ceil_div(std::max(1, n_patch), 8
 
 // the patch kernel for the layout's patch size
 template <typename T, bool Folded, class Stage>
-static void launch_patch(const MfOp& op, const T* qdp, const Stage& st, T* part, const int* skip, hipStream_t s) {
-  const dim3 grid(patch_grid(op.n_patch));
+static void launch_patch(const MfOp& op, const T* qdp, const Stage& st, T* part, const int* skip, hipStream_t s,
+                         const FinRR& fin = {}) {
+  const dim3 grid(patch_grid(op.n_patch) + (fin.part ? 1 : 0));
   const size_t lds = patch_lds_bytes(op, sizeof(T));
 #define WN_PATCH_LAUNCH1(PP, NS)                                                                                    \
   hipLaunchKernelGGL((mf_patch_kernel<T, PP, NS, Folded, Stage>), grid, dim3(4 * (PP)), lds, s, op.n_patch, op.M,   \
                      op.stride, op.pnode, reinterpret_cast<const ushort4*>(op.pconn), op.poff,                      \
-                     reinterpret_cast<const uint2*>(op.pslot), op.pe, qdp, op.E, op.nu, op.phead, st, part, skip)
+                     reinterpret_cast<const uint2*>(op.pslot), op.pe, qdp, op.E, op.nu, op.phead, st, part, fin,    \
+                     skip)
 #define WN_PATCH_LAUNCH(PP)                                                                                         \
   if (op.stride <= 8 * (PP)) WN_PATCH_LAUNCH1(PP, 2); else WN_PATCH_LAUNCH1(PP, kStageSlots)
   switch (op.patch) {
@@ -1919,22 +1923,11 @@ template <> const double* mf_qdp<double>(const MfSmooth& m) { return m.op->patch
 template <> const float* mf_qdp<float>(const MfSmooth& m) {
   return m.op->patch && m.gen == m.op->gen ? m.qdp32 : nullptr;
 }
-template <typename T> static T* mf_part(const MfSmooth& m);
-template <> double* mf_part<double>(const MfSmooth& m) { return m.op->part; }
-template <> float* mf_part<float>(const MfSmooth& m) { return m.part32; }
-
 template <typename T, typename Op>
 static int mf_smooth_run(const MfSmooth& m, const T* x, const Op& o, const int* skip, hipStream_t s) {
   if (!mf_smooth_ready<T>(m)) return kNotReady;
   const MfOp& op = *m.op;
   const T* sc = mf_scale<T>(m);
-  if (const T* qdp = mf_qdp<T>(m)) {
-    T* part = mf_part<T>(m);
-    launch_patch<T, std::is_same<T, float>::value>(op, qdp, StageScaled<T>{mf_scale_in<T>(m), x}, part, skip, s);
-    hipLaunchKernelGGL((mf_node_kernel<T, Op>), dim3(node_grid(op.n_nodes)), dim3(kNodeThreads), 0, s, op.n_nodes,
-                       op.nhead, op.novf, part, op.fix, sc, x, o, skip);
-    return static_cast<int>(hipGetLastError());
-  }
   if (op.M > 0 && op.affine)
     hipLaunchKernelGGL((c3d10_pa_elem_kernel<T, true>), dim3(elem_grid(op.M)), dim3(256), 0, s, op.M,
                        op.conn, mf_qd<T>(m), op.E, op.nu, mf_scale_in<T>(m), x, mf_fe<T>(m), skip, skip ? 1 : 0);
@@ -1963,10 +1956,10 @@ int mf_smooth_defect(const MfSmooth& m, const T* x, const T* b, T* res, const in
   return mf_smooth_run<T>(m, x, o, skip, s);
 }
 
-// The smoothing chain of the patch layout: a product (mf_smooth_product),
-// steps that complete one product and form the next (mf_smooth_step), and a
-// node kernel that completes the last (mf_smooth_end_*).  `from` names the
-// partial-sum buffer, 0 or 1, that holds the product to complete.
+// Smoothing in the patch layout: a product (mf_smooth_product), in the chain
+// steps that complete one product and form the next (mf_smooth_step), and node
+// kernels that complete one (mf_smooth_end_*).  `from` names the partial-sum
+// buffer, 0 or 1, that holds the product to complete.
 template <typename T> static T* mf_parts(const MfSmooth& m, int k);
 template <> double* mf_parts<double>(const MfSmooth& m, int k) { return k ? m.op->part2 : m.op->part; }
 template <> float* mf_parts<float>(const MfSmooth& m, int k) { return k ? m.part32b : m.part32; }
@@ -1974,15 +1967,20 @@ template <> double* mf_smooth_d2<double>(const MfSmooth& m) { return m.d64b; }
 template <> float* mf_smooth_d2<float>(const MfSmooth& m) { return m.d32b; }
 
 template <typename T>
-bool mf_smooth_chain(const MfSmooth& m) {
-  // (a relayout since the attachment may have dropped the second partial sums)
-  return mf_smooth_ready<T>(m) && mf_qdp<T>(m) && mf_smooth_d2<T>(m) && mf_parts<T>(m, 1);
+bool mf_smooth_patch(const MfSmooth& m) {
+  return mf_smooth_ready<T>(m) && mf_qdp<T>(m);
 }
 
 template <typename T>
-int mf_smooth_product(const MfSmooth& m, const T* x, const int* skip, hipStream_t s) {
+bool mf_smooth_chain(const MfSmooth& m) {
+  // (a relayout since the attachment may have dropped the second partial sums)
+  return mf_smooth_patch<T>(m) && mf_smooth_d2<T>(m) && mf_parts<T>(m, 1);
+}
+
+template <typename T>
+int mf_smooth_product(const MfSmooth& m, const T* x, const int* skip, hipStream_t s, const FinRR* fin) {
   launch_patch<T, std::is_same<T, float>::value>(*m.op, mf_qdp<T>(m), StageScaled<T>{mf_scale_in<T>(m), x},
-                                                 mf_parts<T>(m, 0), skip, s);
+                                                 mf_parts<T>(m, 0), skip, s, fin ? *fin : FinRR{});
   return static_cast<int>(hipGetLastError());
 }
 
@@ -2027,8 +2025,9 @@ int mf_smooth_end_cheb(const MfSmooth& m, int from, const T* x, T* x_out, const 
 }
 
 #define WN_CHAIN_INST(T)                                                                                          \
+  template bool mf_smooth_patch<T>(const MfSmooth&);                                                             \
   template bool mf_smooth_chain<T>(const MfSmooth&);                                                             \
-  template int mf_smooth_product<T>(const MfSmooth&, const T*, const int*, hipStream_t);                         \
+  template int mf_smooth_product<T>(const MfSmooth&, const T*, const int*, hipStream_t, const FinRR*);           \
   template int mf_smooth_step<T>(const MfSmooth&, int, const T*, T*, const T*, const T*, const T*, T*, T, T,     \
                                  const int*, hipStream_t);                                                       \
   template int mf_smooth_end_defect<T>(const MfSmooth&, int, const T*, const T*, T*, const int*, hipStream_t);   \
@@ -2043,27 +2042,6 @@ int mf_smooth_rho_blocks(const MfSmooth& m) {
   return mf_smooth_ready<T>(m) && mf_qdp<T>(m) ? node_grid(m.op->n_nodes) : 0;
 }
 
-template <typename T>
-int mf_smooth_cheb_rho(const MfSmooth& m, const T* x_in, T* x_out, const T* b, const T* dinv, T* d, T c1, T c2,
-                       const RhoReq& rq, const int* skip, hipStream_t s) {
-  const T* qdp = mf_smooth_ready<T>(m) ? mf_qdp<T>(m) : nullptr;
-  if (!qdp || !rq.r || !rq.partials) return kBadMode;
-  const MfOp& op = *m.op;
-  T* part = mf_part<T>(m);
-  launch_patch<T, std::is_same<T, float>::value>(op, qdp, StageScaled<T>{mf_scale_in<T>(m), x_in}, part, skip, s);
-  const dim3 grid(node_grid(op.n_nodes));
-  if (!dinv) {
-    const OpChebRho<3, T, true> o{{b, nullptr, x_in, x_out, d, c1, c2}, rq.r, rq.scale, rq.partials};
-    hipLaunchKernelGGL((mf_node_kernel<T, OpChebRho<3, T, true>>), grid, dim3(kNodeThreads), 0, s, op.n_nodes,
-                       op.nhead, op.novf, part, op.fix, mf_scale<T>(m), x_in, o, skip);
-  } else {
-    const OpChebRho<3, T> o{{b, dinv, x_in, x_out, d, c1, c2}, rq.r, rq.scale, rq.partials};
-    hipLaunchKernelGGL((mf_node_kernel<T, OpChebRho<3, T>>), grid, dim3(kNodeThreads), 0, s, op.n_nodes, op.nhead,
-                       op.novf, part, op.fix, mf_scale<T>(m), x_in, o, skip);
-  }
-  return static_cast<int>(hipGetLastError());
-}
-
 template int mf_smooth_cheb<double>(const MfSmooth&, const double*, double*, const double*, const double*, double*,
                                     double, double, const int*, hipStream_t);
 template int mf_smooth_cheb<float>(const MfSmooth&, const float*, float*, const float*, const float*, float*, float,
@@ -2073,9 +2051,4 @@ template int mf_smooth_defect<double>(const MfSmooth&, const double*, const doub
 template int mf_smooth_defect<float>(const MfSmooth&, const float*, const float*, float*, const int*, hipStream_t);
 template int mf_smooth_rho_blocks<double>(const MfSmooth&);
 template int mf_smooth_rho_blocks<float>(const MfSmooth&);
-template int mf_smooth_cheb_rho<double>(const MfSmooth&, const double*, double*, const double*, const double*,
-                                        double*, double, double, const RhoReq&, const int*, hipStream_t);
-template int mf_smooth_cheb_rho<float>(const MfSmooth&, const float*, float*, const float*, const float*, float*,
-                                       float, float, const RhoReq&, const int*, hipStream_t);
-
 }  // namespace wn

@@ -319,7 +319,7 @@ static int launch_sell(const SellMatrix& A, const XT* x, const Op& op, const Spm
   if (A.n_slices == 0) return kOk;
   const SellView<VT> v = A.view<VT>();
   if (!v.val) return kNotReady;
-  const int grid = sell_grid<VT>(A, t);
+  const int grid = sell_grid<VT>(A, t) + (OpFin<Op>::value ? 1 : 0);
   const int u = t.unroll_for<VT>(), xcd = t.xcd_for<VT>();
   switch (t.waves_for<VT>()) {
     case 2:
@@ -406,7 +406,8 @@ int spmv_residual64(const SellMatrix& A, const double* x, const double* b, doubl
 
 template <typename VT, typename T>
 int spmv_cheb(const SellMatrix& A, const T* x_in, T* x_out, const T* b, const T* dinv, T* d, double c1, double c2,
-              const SpmvTune& t, hipStream_t s, const RhoReq* rq) {
+              const SpmvTune& t, hipStream_t s, const RhoReq* rq, const FinRR* fin) {
+  if (rq && fin) return kBadMode;
   if (A.br != A.bc) return kBadArg;
 #define CALL(R, C)                                                                                          \
   {                                                                                                         \
@@ -415,8 +416,9 @@ int spmv_cheb(const SellMatrix& A, const T* x_in, T* x_out, const T* b, const T*
       if (rq) {                                                                                             \
         return launch_sell<R, C, VT, T>(A, x_in, OpChebRho<R, T>{op, rq->r, rq->scale, rq->partials}, t, s); \
       }                                                                                                     \
+      if (fin) return launch_sell<R, C, VT, T>(A, x_in, OpChebFin<R, T>{op, *fin}, t, s);                   \
     }                                                                                                       \
-    return rq ? (int)kBadMode : launch_sell<R, C, VT, T>(A, x_in, op, t, s);                                \
+    return rq || fin ? (int)kBadMode : launch_sell<R, C, VT, T>(A, x_in, op, t, s);                         \
   }
   if (A.br == 3) CALL(3, 3) else if (A.br == 6) CALL(6, 6) else return kBadArg;
 #undef CALL
@@ -472,7 +474,7 @@ int spmv_restrict_first(const SellMatrix& A, const T* x, T* y, const T* dinv, T*
 
 #define WN_VINST(VT, T)                                                                                          \
   template int spmv_cheb<VT, T>(const SellMatrix&, const T*, T*, const T*, const T*, T*, double, double,       \
-                                const SpmvTune&, hipStream_t, const RhoReq*);                                \
+                                const SpmvTune&, hipStream_t, const RhoReq*, const FinRR*);                  \
   template int spmv_defect<VT, T>(const SellMatrix&, const T*, const T*, T*, const SpmvTune&, hipStream_t);   \
   template int spmv_addto<VT, T>(const SellMatrix&, const T*, T*, const SpmvTune&, hipStream_t);              \
   template int spmv_restrict<VT, T>(const SellMatrix&, const T*, T*, const SpmvTune&, hipStream_t);           \

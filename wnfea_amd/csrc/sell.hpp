@@ -145,6 +145,9 @@ __device__ __forceinline__ bool guard_skip(const int* flags, int mode) {
   return flags && mode != 0 && flags[0] != 0;
 }
 
+// Ops that carry a FinRR in one more block.
+template <class Op> struct OpFin : std::false_type {};
+
 // Generic sliced-ELL block SpMV.  W wavefronts share one slice and split its
 // steps round-robin; their partial sums meet in LDS.  Each lane keeps U blocks
 // in flight per loop trip (U column loads, then U*BB value loads and U x
@@ -154,6 +157,10 @@ __device__ __forceinline__ bool guard_skip(const int* flags, int mode) {
 template <int BR, int BC, typename VT, typename XT, int W, int U, int K, class Op>
 __global__ __launch_bounds__(64 * W) void sell_spmv_kernel(SellView<VT> A, const XT* __restrict__ x, Op op,
                                                            int xcd_remap, const int* flags, int guard) {
+  if constexpr (OpFin<Op>::value) {
+    __shared__ double red[4];
+    if (blockIdx.x == gridDim.x - 1) return fin_rr_block(op.fin, red);  // the block added for it
+  }
   if (guard_skip(flags, guard)) return;
   using AT = typename AccT<VT>::type;
   constexpr int BB = BR * BC;
@@ -381,6 +388,13 @@ struct OpCheb {
     x_out[k] = p.x + dn;
   }
 };
+
+// OpCheb in a launch that finalises ||r||^2 as well.
+template <int BR, typename T>
+struct OpChebFin : OpCheb<BR, T> {
+  FinRR fin;
+};
+template <int BR, typename T> struct OpFin<OpChebFin<BR, T>> : std::true_type {};
 
 // OpCheb, also writing the partials of rho = r . (S x_out), S a per-DOF scale
 // (may be null): the last smoothing step of a preconditioner cycle hands the

@@ -297,7 +297,7 @@ static int level_degree(const AmgLevel& L) { return std::max(1, std::min(L.degre
 // iterate already (see spmv_restrict_first).
 template <typename VT, typename VTC, typename T, typename VS = VT, typename VSC = VTC>
 static int vcycle(Amg& g, int l, const T* b, T* x, const int* skip, hipStream_t s, const RhoReq* rq = nullptr,
-                  bool first_done = false) {
+                  bool first_done = false, const FinRR* fin = nullptr) {
   AmgLevel& L = *g.L[l];
   SpmvTune t = g.tune;
   t.flags = skip;
@@ -325,37 +325,51 @@ static int vcycle(Amg& g, int l, const T* b, T* x, const int* skip, hipStream_t 
   // rho = r . (S x) for the Krylov loop (see amg_rho_blocks)
   // a unit inverse diagonal is passed to the matrix-free steps as null
   const T* dinv_mf = level_unit<T>(L) ? nullptr : dinv;
-  auto cheb = [&](const T* xi, T* xo, int k, const RhoReq* q = nullptr) -> int {
-    if (mf && q) return mf_smooth_cheb_rho<T>(g.mfs, xi, xo, b, dinv_mf, d, T(c.c1[k]), T(c.c2[k]), *q, skip, s);
-    if (mf) return mf_smooth_cheb<T>(g.mfs, xi, xo, b, dinv_mf, d, T(c.c1[k]), T(c.c2[k]), skip, s);
-    return spmv_cheb<VS, T>(A, xi, xo, b, dinv, d, c.c1[k], c.c2[k], t, s, q);
+  const bool patch = mf && mf_smooth_patch<T>(g.mfs);
+  const bool chain = patch && mf_smooth_chain<T>(g.mfs);
+  T* d2 = chain ? mf_smooth_d2<T>(g.mfs) : nullptr;
+  const int* skip_fin = fin ? fin->flags + 2 : skip;  // what a launch that carries fin looks at
+  int from = 0;  // patch layout: where the product of cur is
+  // steps k0 .. k1 - 1 from cur; the patch layout then forms the product of
+  // the result.  f: carried by the first kernel.
+  auto smooth = [&](int k0, int k1, const FinRR* f) -> int {
+    int e = kOk;
+    if (patch) {
+      e = mf_smooth_product<T>(g.mfs, cur, f ? skip_fin : skip, s, f);
+      from = 0;
+    }
+    for (int k = k0; k < k1 && !e; ++k) {
+      const T c1 = T(c.c1[k]), c2 = T(c.c2[k]);
+      if (chain) {
+        e = mf_smooth_step<T>(g.mfs, from, cur, oth, b, dinv_mf, d, d2, c1, c2, skip, s);
+        from = 1 - from;
+        std::swap(d, d2);
+      } else if (patch) {
+        e = mf_smooth_end_cheb<T>(g.mfs, from, cur, oth, b, dinv_mf, d, c1, c2, nullptr, skip, s);
+        if (!e) e = mf_smooth_product<T>(g.mfs, oth, skip, s);
+      } else if (mf) {
+        e = mf_smooth_cheb<T>(g.mfs, cur, oth, b, dinv_mf, d, c1, c2, skip, s);
+      } else {
+        SpmvTune tk = t;
+        const FinRR* fk = k == k0 ? f : nullptr;
+        if (fk) tk.flags = skip_fin;
+        e = spmv_cheb<VS, T>(A, cur, oth, b, dinv, d, c.c1[k], c.c2[k], tk, s, nullptr, fk);
+      }
+      std::swap(cur, oth);
+    }
+    return e;
   };
   if (!first_done) {
     hipLaunchKernelGGL(cheb_first_kernel<T>, dim3(vec_grid(n)), dim3(256), 0, s, n, b, dinv, d, cur, T(c.c2[0]),
                        skip);
     if ((r = static_cast<int>(hipGetLastError()))) return r;
   }
-  // in the patch layout each step's completion is staged by the next product
-  const bool chain = mf && mf_smooth_chain<T>(g.mfs);
-  T* d2 = chain ? mf_smooth_d2<T>(g.mfs) : nullptr;
-  if (chain) {
-    if ((r = mf_smooth_product<T>(g.mfs, cur, skip, s))) return r;
-    int from = 0;
-    for (int k = 1; k < deg; ++k, from = 1 - from) {
-      if ((r = mf_smooth_step<T>(g.mfs, from, cur, oth, b, dinv_mf, d, d2, T(c.c1[k]), T(c.c2[k]), skip, s))) return r;
-      std::swap(cur, oth);
-      std::swap(d, d2);
-    }
-    if ((r = mf_smooth_end_defect<T>(g.mfs, from, cur, b, res, skip, s))) return r;
-  } else {
-    for (int k = 1; k < deg; ++k) {
-      if ((r = cheb(cur, oth, k))) return r;
-      std::swap(cur, oth);
-    }
-    // defect and restriction
-    r = mf ? mf_smooth_defect<T>(g.mfs, cur, b, res, skip, s) : spmv_defect<VT, T>(A, cur, b, res, t, s);
-    if (r) return r;
-  }
+  if ((r = smooth(1, deg, fin))) return r;
+  // defect and restriction
+  r = patch ? mf_smooth_end_defect<T>(g.mfs, from, cur, b, res, skip, s)
+      : mf  ? mf_smooth_defect<T>(g.mfs, cur, b, res, skip, s)
+            : spmv_defect<VT, T>(A, cur, b, res, t, s);
+  if (r) return r;
   AmgLevel& N = *g.L[l + 1];
   T** nv = level_vecs<T>(N);
   // a smoothed coarser level gets its first Chebyshev iterate from the
@@ -374,21 +388,12 @@ static int vcycle(Amg& g, int l, const T* b, T* x, const int* skip, hipStream_t 
   if ((r = vcycle<VTC, VTC, T, VSC, VSC>(g, l + 1, nv[0], nv[1], skip, s, nullptr, fuse_first))) return r;
   if ((r = spmv_addto<VT, T>(L.P, nv[1], cur, t, s))) return r;  // cur == post here
   oth = (cur == x) ? tmp : x;
-  if (chain) {
-    if ((r = mf_smooth_product<T>(g.mfs, cur, skip, s))) return r;
-    int from = 0;
-    for (int k = 0; k < deg - 1; ++k, from = 1 - from) {
-      if ((r = mf_smooth_step<T>(g.mfs, from, cur, oth, b, dinv_mf, d, d2, T(c.c1[k]), T(c.c2[k]), skip, s))) return r;
-      std::swap(cur, oth);
-      std::swap(d, d2);
-    }
+  if ((r = smooth(0, deg - 1, nullptr))) return r;
+  // the last step ends in x
+  if (patch)
     return mf_smooth_end_cheb<T>(g.mfs, from, cur, oth, b, dinv_mf, d, T(c.c1[deg - 1]), T(c.c2[deg - 1]), rq, skip, s);
-  }
-  for (int k = 0; k < deg; ++k) {
-    if ((r = cheb(cur, oth, k, k == deg - 1 ? rq : nullptr))) return r;
-    std::swap(cur, oth);
-  }
-  return kOk;
+  if (mf) return mf_smooth_cheb<T>(g.mfs, cur, oth, b, dinv_mf, d, T(c.c1[deg - 1]), T(c.c2[deg - 1]), skip, s);
+  return spmv_cheb<VS, T>(A, cur, oth, b, dinv, d, c.c1[deg - 1], c.c2[deg - 1], t, s, rq);
 }
 
 template <typename T>
@@ -433,6 +438,20 @@ int amg_rho_blocks(const Amg& g, int vt) {
   return 0;
 }
 
+// Whether the cycle of kind vt can carry a FinRR (given a first iterate, its
+// first kernel is a product with a block to spare).
+template <typename T>
+static bool carries_fin(const Amg& g) {
+  if (mf_smooth_ready<T>(g.mfs)) return mf_smooth_patch<T>(g.mfs);
+  return level_degree(*g.L[0]) > 1 && g.L[0]->A->n_slices > 0;
+}
+bool amg_carries_fin(const Amg& g, int vt) {
+  if (g.L.size() < 2) return false;
+  if (vt == 0) return (g.store & 1) && carries_fin<double>(g);
+  if (vt == 1) return (g.store & 2) && carries_fin<float>(g);
+  return false;
+}
+
 // One V-cycle, z = M r; with rq also the partials of rho = r . (S z) (see
 // amg_rho_blocks).  vt: 0 FP64 values and vectors, 1 FP32 values, 2 FP16
 // values on every level, 3 FP16 values on the finest level and FP32 below it,
@@ -441,19 +460,20 @@ int amg_rho_blocks(const Amg& g, int vt) {
 // the cycle nonsymmetric by O(eps16) and CG then stalls, so that split is not
 // offered.)
 int amg_apply(Amg& g, int vt, const void* r, void* z, const int* skip, hipStream_t s, const RhoReq* rq,
-              bool first_done) {
+              bool first_done, const FinRR* fin) {
   if (g.L.empty()) return kNotReady;
   const float* r32 = static_cast<const float*>(r);
   float* z32 = static_cast<float*>(z);
   if (rq && amg_rho_blocks(g, vt) <= 0) return kBadMode;
+  if (fin && !(first_done && amg_carries_fin(g, vt))) return kBadMode;
   switch (vt) {
     case 0:
       if (!(g.store & 1)) return kNotReady;
       return vcycle<double, double, double>(g, 0, static_cast<const double*>(r), static_cast<double*>(z), skip, s,
-                                            rq, first_done);
+                                            rq, first_done, fin);
     case 1:
       if (!(g.store & 2)) return kNotReady;
-      return vcycle<float, float, float>(g, 0, r32, z32, skip, s, rq, first_done);
+      return vcycle<float, float, float>(g, 0, r32, z32, skip, s, rq, first_done, fin);
     case 2:
       if (!(g.store & 4)) return kNotReady;
       return vcycle<_Float16, _Float16, float>(g, 0, r32, z32, skip, s);
@@ -517,6 +537,7 @@ __global__ void pcg_start_kernel(double* sc, int* flags, double rtol2) {
     sc[kScTol2] = rtol2 * sc[kScRR];
     flags[0] = (sc[kScRR] == 0.0) ? 1 : 0;
     flags[1] = 0;
+    flags[2] = flags[0];
   }
 }
 
@@ -673,7 +694,9 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
   // the kernels that use them (every block of the p update sums the rho
   // partials, every block of the x, r update the gamma partials), so an
   // iteration launches one one-block finalisation (rr and the done flag)
-  // instead of three.
+  // instead of three; where the cycle can carry it (see FinRR) that one too
+  // moves into the next iteration's first kernel, except at the end of a chunk,
+  // whose flags the host reads.
   const bool fused = !flexible;
   const RhoReq rq{reinterpret_cast<const double*>(k.r), scale, S.ws.partials};
   const RhoReq* cycle_rho = fused && nb_cycle_rho > 0 ? &rq : nullptr;
@@ -681,8 +704,13 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
   const int nb_gam = mf ? mf_grid(*mf) : spmv_partials<T>(A, t);
   const double* rho_part = fused ? S.ws.partials : nullptr;
   const double* gam_part = fused ? S.ws.partials : nullptr;
-  auto iteration = [&](hipStream_t st) -> int {
+  const bool carry = first_done && amg_carries_fin(*amg, amg_vt) && vec_grid(n) <= kFinRRMax;
+  FinRR pending;
+  auto iteration = [&](hipStream_t st, bool first_of_chunk, bool last_of_chunk) -> int {
     int e;
+    const FinRR now = pending;
+    const FinRR* fin = carry && !first_of_chunk ? &now : nullptr;
+    FinRR* later = carry && !last_of_chunk ? &pending : nullptr;
     const int first = -1;
     if (pkind == 1) {
       if ((e = launch_jacobi_dot<T>(n, k.r, dinv, k.z, S.ws, first, S.flags, st, !fused))) return e;
@@ -690,7 +718,7 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
     } else if (pkind == 2 && amg32) {
       const float* vin = sep32 ? rp32 : reinterpret_cast<const float*>(k.r);
       float* vout = sep32 ? S.zp32 : reinterpret_cast<float*>(k.z);
-      if ((e = amg_apply(*amg, amg_vt, vin, vout, S.flags, st, cycle_rho, first_done))) return e;
+      if ((e = amg_apply(*amg, amg_vt, vin, vout, S.flags, st, cycle_rho, first_done, fin))) return e;
       if (!cycle_rho &&
           (e = launch_rho<T, float>(n, k.r, vout, scale, S.ws, first, S.flags, st, flexible ? k.q : nullptr, !fused)))
         return e;
@@ -699,7 +727,7 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
       // FP64 cycle: in-place scaled input in k.z when S is given
       const T* vin = sep64 ? k.z : k.r;
       T* vout = k.q;  // q is free until the SpMV below
-      if ((e = amg_apply(*amg, 0, vin, vout, S.flags, st, cycle_rho, first_done))) return e;
+      if ((e = amg_apply(*amg, 0, vin, vout, S.flags, st, cycle_rho, first_done, fin))) return e;
       if (!cycle_rho && (e = launch_rho<T, T>(n, k.r, vout, scale, S.ws, first, S.flags, st, nullptr, !fused)))
         return e;
       if ((e = launch_update_p<T, T>(n, vout, scale, k.p, S.ws, first, S.flags, st, rho_part, nb_rho))) return e;
@@ -719,10 +747,10 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
     }
     if (sep32)
       return launch_update_xr<T, float>(n, x, k.r, k.p, k.q, rp32, scale, S.ws, S.flags, st, gam_part, nb_gam,
-                                        first_done ? &fi32 : nullptr);
+                                        first_done ? &fi32 : nullptr, later);
     if (sep64)
       return launch_update_xr<T, T>(n, x, k.r, k.p, k.q, k.z, scale, S.ws, S.flags, st, gam_part, nb_gam,
-                                    first_done ? &fi64 : nullptr);
+                                    first_done ? &fi64 : nullptr, later);
     return launch_update_xr<T, T>(n, x, k.r, k.p, k.q, nullptr, nullptr, S.ws, S.flags, st, gam_part, nb_gam);
   };
   std::vector<uint64_t> key;
@@ -756,7 +784,7 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
     if (S.use_graphs && chunk == check_every) {
       r = graph_for(S, key, [&](hipStream_t st) -> int {
         for (int c = 0; c < chunk; ++c) {
-          const int e = iteration(st);
+          const int e = iteration(st, c == 0, c == chunk - 1);
           if (e) return e;
         }
         return kOk;
@@ -765,7 +793,7 @@ int pcg_run(Solver& S, const SellMatrix& A, int pkind, const T* dinv, Amg* amg, 
       WN_HIP(hipGraphLaunch(S.gexec, s));
     } else {
       for (int c = 0; c < chunk; ++c)
-        if ((r = iteration(s))) return r;
+        if ((r = iteration(s, c == 0, c == chunk - 1))) return r;
     }
     it += chunk;
     WN_HIP(hipMemcpyAsync(S.h_flags, S.flags, sizeof(int) * 2, hipMemcpyDeviceToHost, s));

@@ -135,7 +135,7 @@ struct KVec {
 
 struct Solver {
   Workspace ws;
-  int* flags = nullptr;  // [0] done, [1] iterations
+  int* flags = nullptr;  // [0] done, [1] iterations, [2] done as of the last x, r update
   int* h_flags = nullptr;
   double* h_sc = nullptr;
   KVec<double> k64;
@@ -199,10 +199,12 @@ int amg_alloc_vectors(Amg& g, int prec_mask);
 // One V-cycle z = M r of kind vt; with rq also the partials of rho = r . (S z)
 // (amg_rho_blocks(g, vt) of them; kBadMode when that is 0).
 // first_done: the finest level's first Chebyshev iterate is in place already
-// (see amg_first_iter).
+// (see amg_first_iter); with fin (amg_carries_fin and first_done) the first
+// kernel carries that finalisation.
 int amg_apply(Amg& g, int vt, const void* r, void* z, const int* skip, hipStream_t s, const RhoReq* rq = nullptr,
-              bool first_done = false);
+              bool first_done = false, const FinRR* fin = nullptr);
 int amg_rho_blocks(const Amg& g, int vt);
+bool amg_carries_fin(const Amg& g, int vt);
 // Where the finest level's first Chebyshev iterate of a cycle of kind vt
 // (0: T double, 1: T float) with output z goes, so that the kernel writing
 // the cycle's input can form it (false: no such cycle).

@@ -161,28 +161,27 @@ int mf_smooth_defect(const MfSmooth& m, const T* x, const T* b, T* res, const in
 // Partials of rho = r . (S z) requested from the Chebyshev step that writes
 // a V-cycle's output z (scale null: S = I); nb partials, see
 // mf_smooth_rho_blocks and spmv_partials.  spmv_cheb takes it with values of
-// the vectors' type only.
+// the vectors' type only; so too a FinRR to finalise beside its own work (then
+// t.flags is not the flags it sets).
 struct RhoReq {
   const double* r;
   const double* scale;
   double* partials;
 };
-// The Chebyshev step above, also writing the RhoReq partials of its x_out
-// (patch layout only: kBadMode otherwise).
-template <typename T>
-int mf_smooth_cheb_rho(const MfSmooth& m, const T* x_in, T* x_out, const T* b, const T* dinv, T* d, T c1, T c2,
-                       const RhoReq& rq, const int* skip, hipStream_t s);
-// The smoothing chain of the patch layout (mf_smooth_chain: whether it can
-// run): a product of x, steps that complete the product in buffer `from` (0
-// or 1, the product's is 0) as a Chebyshev step and form the product of its
-// result in the other buffer, and the node kernel that completes the last.  A
-// step's x_out, d_out are buffers of their own (mf_smooth_d2: a second d);
-// dinv null: the unit diagonal.
+// Smoothing in the patch layout (mf_smooth_patch: attached to it), a product
+// and its completion apart: a product of x (with fin, carrying that
+// finalisation), into partial-sum buffer 0; node kernels that complete the
+// product in buffer `from`; and, where the chain runs (mf_smooth_chain), a step
+// that completes it as a Chebyshev step and forms the product of its result
+// in the other buffer.  The step's x_out, d_out are buffers of their own
+// (mf_smooth_d2: a second d); dinv null: the unit diagonal.
+template <typename T> bool mf_smooth_patch(const MfSmooth& m);
 template <typename T> T* mf_smooth_d2(const MfSmooth& m);
 template <> double* mf_smooth_d2<double>(const MfSmooth& m);
 template <> float* mf_smooth_d2<float>(const MfSmooth& m);
 template <typename T> bool mf_smooth_chain(const MfSmooth& m);
-template <typename T> int mf_smooth_product(const MfSmooth& m, const T* x, const int* skip, hipStream_t s);
+template <typename T>
+int mf_smooth_product(const MfSmooth& m, const T* x, const int* skip, hipStream_t s, const FinRR* fin = nullptr);
 template <typename T>
 int mf_smooth_step(const MfSmooth& m, int from, const T* x, T* x_out, const T* b, const T* dinv, const T* d, T* d_out,
                    T c1, T c2, const int* skip, hipStream_t s);
@@ -264,11 +263,12 @@ struct FirstIter {
 // x += alpha p; r -= alpha q; rr; optional rp = S r (and with fi the next
 // cycle's first iterate from it); raises flags[0] (done) when
 // rr <= sc[kScTol2]; with gam_part the kernel finalises gamma = p . A p from
-// its nb_gam partials and forms alpha itself
+// its nb_gam partials and forms alpha itself.  With `later` rr is left for the
+// kernel that is given *later (see FinRR).
 template <typename T, typename RT>
 int launch_update_xr(long long n, T* x, T* r, const T* p, const T* q, RT* rp, const double* scale, Workspace& w,
                      int* flags, hipStream_t s, const double* gam_part = nullptr, int nb_gam = 0,
-                     const FirstIter<RT>* fi = nullptr);
+                     const FirstIter<RT>* fi = nullptr, FinRR* later = nullptr);
 template <typename T> int launch_dot(long long n, const T* a, const T* b, Workspace& w, double* out, hipStream_t s);
 template <typename T>
 int launch_ir_update(long long n, double* u, const T* d, const double* sc_vec, const double* nrm2, hipStream_t s);
@@ -295,7 +295,7 @@ int spmv_residual64(const SellMatrix& A, const double* x, const double* b, doubl
 // T the vector/arithmetic type (double for VT = double, float otherwise).
 template <typename VT, typename T>
 int spmv_cheb(const SellMatrix& A, const T* x_in, T* x_out, const T* b, const T* dinv, T* d, double c1, double c2,
-              const SpmvTune& t, hipStream_t s, const RhoReq* rq = nullptr);
+              const SpmvTune& t, hipStream_t s, const RhoReq* rq = nullptr, const FinRR* fin = nullptr);
 template <typename VT, typename T>
 int spmv_defect(const SellMatrix& A, const T* x, const T* b, T* res, const SpmvTune& t, hipStream_t s);
 template <typename VT, typename T> int spmv_addto(const SellMatrix& A, const T* e, T* x, const SpmvTune& t,
