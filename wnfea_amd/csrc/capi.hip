@@ -269,6 +269,16 @@ void* wnfea_bsr_create(int br, int bc, int n_rows, int n_cols, const int* rowptr
     delete h;
     return nullptr;
   }
+  // Launch shape of a matrix nobody has tuned, by the blocks per lane: with
+  // four or more, four wavefronts share a slice and FP32 values go two blocks
+  // at a time (rows of 25 3x3 blocks on four lanes, one wavefront against
+  // that: FP32 24k rows 15.7 -> 8.4 us, 352k 68.9 -> 61.9; FP64 7.6k 12.3 ->
+  // 7.9, 352k 131.8 -> 119.0).  Shorter rows, the beam lattice's seven 6x6
+  // blocks on two lanes, gain nothing.
+  if (h->m.nnzb >= 4LL * h->m.lanes * h->m.n_rows && h->m.n_rows > 0) {
+    h->tune.set(0, 4, 1, 1);
+    h->tune.set(1, 4, 1, 2);
+  }
   return h;
 }
 

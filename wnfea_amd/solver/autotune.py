@@ -43,7 +43,7 @@ def _store_cache(cache: dict) -> None:
 
 # bumped whenever the SpMV kernels or the timing method change, so that cached
 # choices of an older build are not reused
-_KERNEL_REV = 5
+_KERNEL_REV = 6
 
 # GPU cycles of the spin kernel that holds the stream while the timed launches
 # are queued (about 1 ms at the shader clock), and the fastest shader clock of

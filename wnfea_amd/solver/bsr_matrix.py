@@ -198,7 +198,8 @@ class DeviceBSR:
         if x.dtype != dt or x.numel() != self.shape[1]:
             raise ValueError("x has the wrong dtype or length")
         if y is None:
-            y = torch.zeros(self.shape[0], dtype=dt, device=self.device)
+            # a product that does not read y writes all of it
+            y = (torch.empty if beta == 0.0 else torch.zeros)(self.shape[0], dtype=dt, device=self.device)
         _lib.check(self.lib.wnfea_bsr_spmv(self.handle, prec, _lib.dptr(x), _lib.dptr(y), float(alpha), float(beta),
                                            _lib.stream_of()), "wnfea_bsr_spmv")
         return y
