@@ -304,7 +304,9 @@ void wnfea_bsr_destroy(void *h);
 int wnfea_bsr_info(void *h, long long *out);
 
 /* SpMV launch shape: waves per slice (1, 2, 4), XCD-contiguous slice mapping,
- * blocks in flight per lane (1, 2, 4).  No reference counterpart (the
+ * blocks in flight per lane (1, 2, 4).  Until it is called: 4 waves, and 2
+ * blocks of FP32 values, where a lane has four blocks or more, else 1 and 1.
+ * No reference counterpart (the
  * reference's launch sizes are fixed heuristics, wnfea/solver/fast_kernels.py:243-260). */
 int wnfea_bsr_tune(void *h, int waves, int xcd_remap, int unroll);
 
