@@ -349,7 +349,7 @@ static int spmm_restrict_first(const SellMatrix& A, const T* x, T* y, const T* d
     MOpRestrictFirst<T, AT> op{y, dinv, x1, d1, T(c2)};         \
     return launch_spmm<R, C, VT, T, NR>(A, x, op, t, s);        \
   }
-  if (A.br == 6 && A.bc == 3) CALL(6, 3) else if (A.br == 6 && A.bc == 6) CALL(6, 6) else return kBadArg;
+  WN_MR_DISPATCH(A, CALL);  // 3-row blocks: a coarse space of the translations alone
 #undef CALL
 }
 
