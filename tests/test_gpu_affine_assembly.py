@@ -106,3 +106,15 @@ def test_equilibrated_copies(b, lanes):
         xr = xd.double().cpu().numpy()
         err = np.abs(A.spmv(xd, precision=prec).double().cpu().numpy() - M @ xr)
         assert np.all(err <= 30 * b * eps * (abs(M) @ np.abs(xr)))  # at most 30 b products per row
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("local", [0, 7])
+def test_element_with_a_lost_node_is_refused(local, value):
+    """A corner or a midside node whose position is not a number: det J is not
+    positive, on every path."""
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr
+    m = _model("cell")
+    m.mesh_nodes[m.solid_elements[2, local], 1] = value
+    with pytest.raises(ValueError, match="Non-positive Jacobian determinant in C3D10 element"):
+        assemble_c3d10_bsr(m)

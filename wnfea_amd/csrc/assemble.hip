@@ -47,7 +47,7 @@ __global__ __launch_bounds__(128) void affine_record_kernel(int M, const int* __
 #pragma unroll
     for (int c = 0; c < 3; ++c) X[i][c] = nodes[n3 + c];
   }
-  double d[3][3], size = 0.0, off = 0.0;
+  double d[3][3], size = 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k)
 #pragma unroll
@@ -56,11 +56,13 @@ __global__ __launch_bounds__(128) void affine_record_kernel(int M, const int* __
       size = fmax(size, fabs(d[k][c]));
     }
   constexpr int P[6] = {0, 1, 2, 0, 1, 2}, Q[6] = {1, 2, 0, 3, 3, 3};
+  bool flat = true;  // one comparison per coordinate: a NaN fails its own, where a maximum would drop it
 #pragma unroll
   for (int m = 0; m < 6; ++m)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) off = fmax(off, fabs(X[4 + m][c] - 0.5 * (X[P[m]][c] + X[Q[m]][c])));
-  if (!(off <= 1e-12 * size)) atomicOr(flags + 1, 1);
+    for (int c = 0; c < 3; ++c)
+      flat = flat && fabs(X[4 + m][c] - 0.5 * (X[P[m]][c] + X[Q[m]][c])) <= 1e-12 * size;
+  if (!flat) atomicOr(flags + 1, 1);
   // rows of the inverse of [d1 d2 d3]: the gradients of L_1, L_2, L_3
   double g[4][3];
 #pragma unroll
