@@ -118,3 +118,55 @@ def test_element_with_a_lost_node_is_refused(local, value):
     m.mesh_nodes[m.solid_elements[2, local], 1] = value
     with pytest.raises(ValueError, match="Non-positive Jacobian determinant in C3D10 element"):
         assemble_c3d10_bsr(m)
+
+
+def _straight(mesh):
+    """Whether every element counts as affine, from wnfea_c3d10_affine_records."""
+    import torch
+    from wnfea_amd import _lib
+    M = mesh["n_elements"]
+    rec = torch.empty((M, 16), dtype=torch.float64, device="cuda")
+    flags = torch.zeros(2, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.load().wnfea_c3d10_affine_records(
+        M, *[_lib.dptr(mesh[k]) for k in ("conn", "nodes", "E", "nu")], _lib.dptr(rec), _lib.dptr(flags),
+        _lib.stream_of()), "records")
+    return int(flags[1].item()) == 0
+
+
+@pytest.mark.parametrize("kind", ["cell", "five", "ibeam"])
+def test_rounded_midpoints_are_straight(kind):
+    """Generated meshes, and the same rotated and shifted after the midpoints
+    were made: each coordinate of a rotation is three products and two sums
+    (under 3 ulp of the largest), the shift away from the origin one more."""
+    from wnfea_amd.solver.solid_solver import mesh_to_device
+    m = _model(kind)
+    assert _straight(mesh_to_device(m))
+    a, b = 0.7, 0.4
+    Rz = np.array([[np.cos(a), -np.sin(a), 0], [np.sin(a), np.cos(a), 0], [0, 0, 1]])
+    Rx = np.array([[1, 0, 0], [0, np.cos(b), -np.sin(b)], [0, np.sin(b), np.cos(b)]])
+    m.mesh_nodes = m.mesh_nodes @ (Rx @ Rz).T + 2.0
+    assert _straight(mesh_to_device(m))
+
+
+def test_offsets_of_a_thin_element_are_kept():
+    """A midside node off its edge by 5e-14 of the cell's width is off by 5e-9
+    of its thickness: K is the element matrices', bit for bit."""
+    import torch
+    from wnfea_amd import _lib
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr
+    m, _ = generate_c3d10_structured_block(0.2, 0.1, 1e-6, 2, 1, 1, tets_per_hex=6)
+    assert _straight(assemble_c3d10_bsr(m).mesh)
+    mid = m.solid_elements[:, 4:]
+    m.mesh_nodes[mid[5, 1], 2] += 5e-15
+    s = assemble_c3d10_bsr(m, keep_plan=True)
+    L, mesh, plan = _lib.load(), s.mesh, s.mesh["plan"]
+    K, M = s.K.get_values(), mesh["n_elements"]
+    Ke = torch.empty((M, 30, 30), dtype=torch.float64, device="cuda")
+    bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _lib.check(L.wnfea_c3d10_ke(M, *[_lib.dptr(mesh[k]) for k in ("conn", "nodes", "E", "nu")], _lib.dptr(Ke),
+                                _lib.dptr(bad), _lib.stream_of()), "ke")
+    _lib.check(L.wnfea_bsr_assemble(s.K.handle, _lib.dptr(s.K.d_rowidx), _lib.dptr(s.K.d_colidx),
+                                    _lib.dptr(plan["cptr"]), _lib.dptr(plan["codes"]), _lib.dptr(Ke),
+                                    _lib.dptr(plan["fix"]), None, _lib.stream_of()), "assemble")
+    assert torch.equal(K, s.K.get_values())

@@ -31,8 +31,12 @@ namespace wn {
 constexpr int kRec = 16;  // doubles per element record
 
 // Records of M elements; flags[0] = e + 1 of an element with det J <= 0,
-// flags[1] = 1 when some element is not affine (its midside nodes off the edge
-// midpoints by more than 1e-12 of its largest corner distance).
+// flags[1] = 1 when some element is not affine: a midside node is off its
+// edge's midpoint by more than 8 ulp of the element's largest coordinate.
+// That covers what rounding the midpoint, or rotating the mesh afterwards,
+// leaves (1 and 2 ulp), and is no more than the rounding of J at a Gauss point
+// (a sum of ten nodes' terms).  An offset that is small against the element's
+// size alone can still be large against its thickness, and J would lose it.
 __global__ __launch_bounds__(128) void affine_record_kernel(int M, const int* __restrict__ conn,
                                                             const double* __restrict__ nodes,
                                                             const double* __restrict__ E,
@@ -47,21 +51,22 @@ __global__ __launch_bounds__(128) void affine_record_kernel(int M, const int* __
 #pragma unroll
     for (int c = 0; c < 3; ++c) X[i][c] = nodes[n3 + c];
   }
-  double d[3][3], size = 0.0;
+  double d[3][3], big = 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      d[k][c] = X[k + 1][c] - X[0][c];
-      size = fmax(size, fabs(d[k][c]));
-    }
+    for (int c = 0; c < 3; ++c) d[k][c] = X[k + 1][c] - X[0][c];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) big = fmax(big, fabs(X[i][c]));
   constexpr int P[6] = {0, 1, 2, 0, 1, 2}, Q[6] = {1, 2, 0, 3, 3, 3};
   bool flat = true;  // one comparison per coordinate: a NaN fails its own, where a maximum would drop it
 #pragma unroll
   for (int m = 0; m < 6; ++m)
 #pragma unroll
     for (int c = 0; c < 3; ++c)
-      flat = flat && fabs(X[4 + m][c] - 0.5 * (X[P[m]][c] + X[Q[m]][c])) <= 1e-12 * size;
+      flat = flat && fabs(X[4 + m][c] - 0.5 * (X[P[m]][c] + X[Q[m]][c])) <= 0x1p-49 * big;
   if (!flat) atomicOr(flags + 1, 1);
   // rows of the inverse of [d1 d2 d3]: the gradients of L_1, L_2, L_3
   double g[4][3];
