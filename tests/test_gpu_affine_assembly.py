@@ -170,3 +170,42 @@ def test_offsets_of_a_thin_element_are_kept():
                                     _lib.dptr(plan["cptr"]), _lib.dptr(plan["codes"]), _lib.dptr(Ke),
                                     _lib.dptr(plan["fix"]), None, _lib.stream_of()), "assemble")
     assert torch.equal(K, s.K.get_values())
+
+
+@pytest.mark.parametrize("b,npe,sym", [(3, 10, 0), (3, 10, 1), (3, 4, 0), (3, 4, 1), (6, 2, 1), (6, 3, 0)])
+def test_element_matrices_of_any_node_count(b, npe, sym):
+    """The contribution lists summed on the host, with and without the
+    symmetric part, for the node count known at compile time and others: at
+    most npe^2 terms a block, FP64."""
+    import torch
+    from wnfea_amd import _lib
+    from wnfea_amd.solver.bsr_matrix import DeviceBSR
+    rng = np.random.default_rng([b, npe, sym])
+    n, M = 70, 41
+    conn = np.array([np.sort(rng.choice(n, npe, replace=False)) for _ in range(M)])
+    e, a, c = (v.ravel() for v in np.meshgrid(np.arange(M), np.arange(npe), np.arange(npe), indexing="ij"))
+    key = conn[e, a] * n + conn[e, c]
+    order = np.argsort(key, kind="stable")
+    blocks, first = np.unique(key[order], return_index=True)
+    rows, cols = (blocks // n).astype(np.int32), (blocks % n).astype(np.int32)
+    rowptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    cptr = np.append(first, len(key)).astype(np.int64)
+    codes = (e * npe * npe + a * npe + c)[order].astype(np.int32)
+    Ke = rng.standard_normal((M, npe * b, npe * b))
+    fix = rng.integers(0, 1 << b, n).astype(np.uint8) * (rng.random(n) < 0.2)
+    S = 0.5 * (Ke + Ke.transpose(0, 2, 1)) if sym else Ke
+    Q = S.reshape(M, npe, b, npe, b)[e, a, :, c, :][order]
+    ref, mag = np.add.reduceat(Q, first), np.add.reduceat(np.abs(Q), first)
+    fr, fc = (fix[rows][:, None] >> np.arange(b)) & 1, (fix[cols][:, None] >> np.arange(b)) & 1
+    hit = (fr[:, :, None] | fc[:, None, :]).astype(bool)
+    ref[hit] = (np.eye(b, dtype=bool)[None] & (rows == cols)[:, None, None] & hit)[hit]
+    A = DeviceBSR(b, b, n, n, rowptr, cols)
+    t = lambda v: torch.as_tensor(np.ascontiguousarray(v), device="cuda")  # noqa: E731
+    d = [t(v) for v in (rows, cols, cptr, codes, Ke, fix)]
+    std = torch.full((len(rows), b * b), float("nan"), dtype=torch.float64, device="cuda")
+    _lib.check(_lib.load().wnfea_bsr_assemble_elem(A.handle, npe, sym, *[_lib.dptr(v) for v in d], _lib.dptr(std),
+                                                   _lib.stream_of()), "assemble_elem")
+    assert torch.equal(A.get_values().view(-1, b * b), std)
+    err = np.abs(std.cpu().numpy().reshape(ref.shape) - ref)
+    assert np.all(err <= npe * npe * 2.3e-16 * mag)
+    A.close()

@@ -280,20 +280,63 @@ int assemble_affine(SellMatrix& A, const long long* cptr, const int* codes, cons
 // Ke[M][npe B][npe B].  Block k = (i, j) sums the entries of its contributions
 // in list order (element order, then local pair order), each code =
 // e npe^2 + a npe + b addressing Ke[e][B a + r][B b + c]; sym: of the symmetric
-// part 0.5 (Ke + Ke^T).  One workgroup per step of a slice, whose 64 blocks
-// are summed one thread per entry (an element's rows of B are read by
+// part 0.5 (Ke + Ke^T).
+//
+// 3x3 blocks: one thread per block in standard order, its nine entries' loads
+// in flight together.  Bound by the diagonal blocks' chains of dependent loads
+// on small meshes (a code, then its element's entries, up to a few dozen
+// times) and by the element matrices' lines on large ones.  The tiles of the
+// 6x6 blocks below take such a chain for every entry of a thread, three here:
+// curved I-beams of 2 784, 13 920, 52 200 and 104 400 elements 81, 181, 384
+// and 794 us in tiles, 27, 100, 334 and 657 here.
+// NPE: nodes per element where it is known at compile time, else 0 (npe).
+template <int NPE>
+__global__ __launch_bounds__(256) void assemble_block3_kernel(
+    long long nnzb, int npe_, int sym, const int* __restrict__ rowidx, const int* __restrict__ colidx,
+    const long long* __restrict__ cptr, const int* __restrict__ codes, const double* __restrict__ Ke,
+    const unsigned char* __restrict__ node_fix, const long long* __restrict__ slot, double* __restrict__ v64,
+    double* __restrict__ vstd) {
+  const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (k >= nnzb) return;
+  const int npe = NPE ? NPE : npe_, D = 3 * npe, nn = npe * npe;
+  double acc[9] = {};
+  for (long long q = cptr[k]; q < cptr[k + 1]; ++q) {
+    const int code = codes[q], e = code / nn, ab = code - e * nn, a = ab / npe, b = ab - a * npe;
+    const double* kp = Ke + (size_t)e * D * D;
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        double v = kp[(size_t)(3 * a + r) * D + 3 * b + c];
+        if (sym) v = 0.5 * (v + kp[(size_t)(3 * b + c) * D + 3 * a + r]);
+        acc[3 * r + c] += v;
+      }
+  }
+  const int i = rowidx[k], j = colidx[k];
+  const unsigned fi = node_fix ? node_fix[i] : 0u, fj = node_fix ? node_fix[j] : 0u;
+  const long long sl = slot[k];
+#pragma unroll
+  for (int x = 0; x < 9; ++x) {
+    const double v = with_supports(acc[x], fi, fj, x / 3, x % 3, i == j);
+    v64[val_index<double>(sl, x, 9)] = v;
+    if (vstd) vstd[k * 9 + x] = v;
+  }
+}
+
+// 6x6 blocks: kTileSteps workgroups per slice take its steps in turn; a step's
+// 64 blocks are summed one thread per entry (an element's rows of B are read by
 // neighbouring threads) into LDS and stored in the layout's order, contiguous.
 // Bound by the element matrices' and the values' bytes; one thread per block
-// read every entry from another line and stored 16-byte pieces (104 544 beams,
-// 6x6: 394 us, here 68 us).
+// read every entry from another line and stored 16-byte pieces (104 544 beams:
+// 384 us, here 68 us; 240 beams 42 and 19).
 constexpr int kTileThreads = 256, kTileSteps = 4;  // workgroups per slice
 
-template <int B>
 __global__ __launch_bounds__(kTileThreads) void assemble_tile_kernel(
     SellView<double> A, const int* __restrict__ rstart, int npe, int sym, const long long* __restrict__ cptr,
     const int* __restrict__ codes, const double* __restrict__ Ke, const unsigned char* __restrict__ node_fix,
     double* __restrict__ v64, double* __restrict__ vstd) {
-  constexpr int BB = B * B, PAD = BB | 1, V = 2, FULL = BB / V, REM = BB - FULL * V;
+  constexpr int B = 6, BB = B * B, PAD = BB | 1, V = 2;  // V: entries per 16-byte chunk
+  static_assert(BB % V == 0, "the layout's chunks hold all of a block");
   __shared__ double tile[64][PAD];
   __shared__ long long s_k[64], s_c0[64], s_c1[64];  // block number (-1: none), its contributions
   __shared__ unsigned s_fix[64];                     // row bits, column bits << 8, diagonal << 16
@@ -338,34 +381,31 @@ __global__ __launch_bounds__(kTileThreads) void assemble_tile_kernel(
     __syncthreads();
     double* o = v64 + (base + 64LL * j) * BB;
     for (int f = t; f < 64 * BB; f += kTileThreads) {
-      const int fr = f - FULL * 64 * V;  // in the leftover entries' part of the region
-      const int l = fr < 0 ? f % (64 * V) / V : fr / max(REM, 1);
-      const int e = fr < 0 ? f / (64 * V) * V + f % V : FULL * V + fr % max(REM, 1);
+      const int l = f % (64 * V) / V, e = f / (64 * V) * V + f % V;
       if (s_k[l] >= 0) o[f] = tile[l][e];
     }
     __syncthreads();
   }
 }
 
-int assemble_elem(SellMatrix& A, int npe, int sym, const long long* cptr, const int* codes, const double* Ke,
-                  const unsigned char* node_fix, double* vals_std, hipStream_t s) {
+int assemble_elem(SellMatrix& A, int npe, int sym, const int* rowidx, const int* colidx, const long long* cptr,
+                  const int* codes, const double* Ke, const unsigned char* node_fix, double* vals_std, hipStream_t s) {
   if (A.br != A.bc || npe <= 0 || npe > 27) return kBadArg;
   int r = A.ensure_values(1, 0);
   if (r) return r;
   if (A.nnzb == 0) return kOk;
-  const dim3 grid(8 * ceil_div(A.n_slices, 8), kTileSteps), block(kTileThreads);
-  switch (A.br) {
-    case 3:
-      hipLaunchKernelGGL(assemble_tile_kernel<3>, grid, block, 0, s, A.view<double>(), A.d_rstart, npe, sym, cptr,
-                         codes, Ke, node_fix, A.d_v64, vals_std);
-      break;
-    case 6:
-      hipLaunchKernelGGL(assemble_tile_kernel<6>, grid, block, 0, s, A.view<double>(), A.d_rstart, npe, sym, cptr,
-                         codes, Ke, node_fix, A.d_v64, vals_std);
-      break;
-    default:
-      return kBadArg;
-  }
+  const dim3 grid3(ceil_div(A.nnzb, 256)), grid6(8 * ceil_div(A.n_slices, 8), kTileSteps);
+  if (A.br == 3 && npe == 10 && !sym)
+    hipLaunchKernelGGL(assemble_block3_kernel<10>, grid3, dim3(256), 0, s, A.nnzb, npe, 0, rowidx, colidx, cptr, codes,
+                       Ke, node_fix, A.d_slot, A.d_v64, vals_std);
+  else if (A.br == 3)
+    hipLaunchKernelGGL(assemble_block3_kernel<0>, grid3, dim3(256), 0, s, A.nnzb, npe, sym, rowidx, colidx, cptr,
+                       codes, Ke, node_fix, A.d_slot, A.d_v64, vals_std);
+  else if (A.br == 6)
+    hipLaunchKernelGGL(assemble_tile_kernel, grid6, dim3(kTileThreads), 0, s, A.view<double>(), A.d_rstart, npe, sym,
+                       cptr, codes, Ke, node_fix, A.d_v64, vals_std);
+  else
+    return kBadArg;
   return static_cast<int>(hipGetLastError());
 }
 

@@ -340,14 +340,17 @@ int wnfea_bsr_assemble(void* h, const int* rowidx, const int* colidx, const long
   if (!h) return kBadArg;
   auto* b = static_cast<WnBsr*>(h);
   if (b->m.nnzb > 0 && (!rowidx || !colidx || !cptr || !codes || !Ke)) return kBadArg;
-  return b->m.br == 3 ? assemble_elem(b->m, 10, 0, cptr, codes, Ke, node_fix, vals_std, S(stream)) : kBadArg;
+  return b->m.br == 3 ? assemble_elem(b->m, 10, 0, rowidx, colidx, cptr, codes, Ke, node_fix, vals_std,
+                                       S(stream))
+                       : kBadArg;
 }
 
 int wnfea_bsr_assemble_elem(void* h, int npe, int sym, const int* rowidx, const int* colidx, const long long* cptr,
                             const int* codes, const double* Ke, const unsigned char* node_fix, double* vals_std,
                             void* stream) {
   if (!h || !rowidx || !colidx || !cptr || !codes || !Ke) return kBadArg;
-  return assemble_elem(static_cast<WnBsr*>(h)->m, npe, sym, cptr, codes, Ke, node_fix, vals_std, S(stream));
+  return assemble_elem(static_cast<WnBsr*>(h)->m, npe, sym, rowidx, colidx, cptr, codes, Ke, node_fix, vals_std,
+                       S(stream));
 }
 
 int wnfea_c3d10_affine_records(int M, const int* conn, const double* nodes, const double* E, const double* nu,

@@ -313,8 +313,8 @@ int sell_to_std(const SellMatrix& A, double* vals_std, hipStream_t s);
 // Square element matrices Ke[M][npe*b][npe*b] (b = block size of A, 3 or 6)
 // into A's FP64 values through the contribution lists; sym != 0 assembles the
 // symmetric part 0.5 (Ke + Ke^T); node_fix bit c marks DOF c of a node fixed.
-int assemble_elem(SellMatrix& A, int npe, int sym, const long long* cptr, const int* codes, const double* Ke,
-                  const unsigned char* node_fix, double* vals_std, hipStream_t s);
+int assemble_elem(SellMatrix& A, int npe, int sym, const int* rowidx, const int* colidx, const long long* cptr,
+                  const int* codes, const double* Ke, const unsigned char* node_fix, double* vals_std, hipStream_t s);
 // The C3D10 matrix of an affine mesh from its element records (16 doubles each)
 int affine_records(int M, const int* conn, const double* nodes, const double* E, const double* nu, double* rec,
                    int* flags, hipStream_t s);
