@@ -334,11 +334,12 @@ int wnfea_bsr_assemble(void *h, const int *rowidx, const int *colidx, const long
 /* Element records of a C3D10 mesh for wnfea_bsr_assemble_affine: rec[M][16]
  * (device, 16-byte aligned) gets the four barycentric gradients and the
  * weighted Lame moduli of each element taken as affine.  flags[2] (device
- * int, zeroed by the caller): flags[0] = e + 1 of an element whose corners
- * have det J <= 0, flags[1] = 1 when some element is not affine (midside nodes
- * off the edge midpoints by more than 8 ulp of the element's largest
- * coordinate); the records of such a mesh do not describe it.  With wnfea_bsr_assemble_affine it replaces
- * the element stiffness loop and COO summation of assemble_c3d10_sparse_3dof
+ * int, zeroed by the caller): flags[0] = e + 1 of an element with det J <= 0 (a
+ * curved one: at a Gauss point, as wnfea_c3d10_ke reports), flags[1] = 1 when
+ * some element is not affine (midside nodes off the edge midpoints by more
+ * than 8 ulp of the element's largest coordinate); the records of such a mesh
+ * do not describe it.  With wnfea_bsr_assemble_affine it replaces the element
+ * stiffness loop and COO summation of assemble_c3d10_sparse_3dof
  * (wnfea/solver/solid_solver.py:62-127) where every element is affine. */
 int wnfea_c3d10_affine_records(int M, const int *conn, const double *nodes, const double *E, const double *nu,
                                double *rec, int *flags, void *stream);

@@ -120,8 +120,8 @@ def test_element_with_a_lost_node_is_refused(local, value):
         assemble_c3d10_bsr(m)
 
 
-def _straight(mesh):
-    """Whether every element counts as affine, from wnfea_c3d10_affine_records."""
+def _record_flags(mesh):
+    """[bad element + 1, curved] of wnfea_c3d10_affine_records."""
     import torch
     from wnfea_amd import _lib
     M = mesh["n_elements"]
@@ -130,7 +130,11 @@ def _straight(mesh):
     _lib.check(_lib.load().wnfea_c3d10_affine_records(
         M, *[_lib.dptr(mesh[k]) for k in ("conn", "nodes", "E", "nu")], _lib.dptr(rec), _lib.dptr(flags),
         _lib.stream_of()), "records")
-    return int(flags[1].item()) == 0
+    return flags.tolist()
+
+
+def _straight(mesh):
+    return _record_flags(mesh)[1] == 0
 
 
 @pytest.mark.parametrize("kind", ["cell", "five", "ibeam"])
@@ -209,3 +213,27 @@ def test_element_matrices_of_any_node_count(b, npe, sym):
     err = np.abs(std.cpu().numpy().reshape(ref.shape) - ref)
     assert np.all(err <= npe * npe * 2.3e-16 * mag)
     A.close()
+
+
+def test_records_report_a_curved_element_turned_inside_out():
+    """Corners in order, one midside node far off its edge: the records' flags
+    name the element, so the element matrices need no report of their own."""
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr, mesh_to_device
+    m = _model("cell")
+    X, T = m.mesh_nodes, m.solid_elements
+    e = 4
+    X[T[e, 4]] += 3.0 * (X[T[e, 1]] - X[T[e, 0]])
+    bad = []  # elements at that node with det J <= 0 at a Gauss point, by plain arithmetic
+    a, b = (5 - 5 ** 0.5) / 20, (5 + 3 * 5 ** 0.5) / 20
+    for k in range(len(T)):
+        for L in np.full((4, 4), a) + (b - a) * np.eye(4):
+            G = np.array([(4 * L[i] - 1) * X[T[k, i]] for i in range(4)])
+            for n, (p, q) in enumerate([(0, 1), (1, 2), (2, 0), (0, 3), (1, 3), (2, 3)]):
+                G[p] += 4 * L[q] * X[T[k, 4 + n]]
+                G[q] += 4 * L[p] * X[T[k, 4 + n]]
+            if np.linalg.det(G[1:] - G[0]) <= 0.0:
+                bad.append(k)
+    assert e in bad
+    assert _record_flags(mesh_to_device(m)) == [max(bad) + 1, 1]
+    with pytest.raises(ValueError, match=f"Non-positive Jacobian determinant in C3D10 element {max(bad)}"):
+        assemble_c3d10_bsr(m)

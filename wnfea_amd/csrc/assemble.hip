@@ -28,74 +28,8 @@
 
 namespace wn {
 
-constexpr int kRec = 16;  // doubles per element record
-
-// Records of M elements; flags[0] = e + 1 of an element with det J <= 0,
-// flags[1] = 1 when some element is not affine: a midside node is off its
-// edge's midpoint by more than 8 ulp of the element's largest coordinate.
-// That covers what rounding the midpoint, or rotating the mesh afterwards,
-// leaves (1 and 2 ulp), and is no more than the rounding of J at a Gauss point
-// (a sum of ten nodes' terms).  An offset that is small against the element's
-// size alone can still be large against its thickness, and J would lose it.
-__global__ __launch_bounds__(128) void affine_record_kernel(int M, const int* __restrict__ conn,
-                                                            const double* __restrict__ nodes,
-                                                            const double* __restrict__ E,
-                                                            const double* __restrict__ nu, double* __restrict__ rec,
-                                                            int* __restrict__ flags) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= M) return;
-  double X[10][3];
-#pragma unroll
-  for (int i = 0; i < 10; ++i) {
-    const size_t n3 = 3 * (size_t)conn[(size_t)e * 10 + i];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) X[i][c] = nodes[n3 + c];
-  }
-  double d[3][3], big = 0.0;
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) d[k][c] = X[k + 1][c] - X[0][c];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) big = fmax(big, fabs(X[i][c]));
-  constexpr int P[6] = {0, 1, 2, 0, 1, 2}, Q[6] = {1, 2, 0, 3, 3, 3};
-  bool flat = true;  // one comparison per coordinate: a NaN fails its own, where a maximum would drop it
-#pragma unroll
-  for (int m = 0; m < 6; ++m)
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      flat = flat && fabs(X[4 + m][c] - 0.5 * (X[P[m]][c] + X[Q[m]][c])) <= 0x1p-49 * big;
-  if (!flat) atomicOr(flags + 1, 1);
-  // rows of the inverse of [d1 d2 d3]: the gradients of L_1, L_2, L_3
-  double g[4][3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const double* a = d[(k + 1) % 3];
-    const double* b = d[(k + 2) % 3];
-    g[k + 1][0] = a[1] * b[2] - a[2] * b[1];
-    g[k + 1][1] = a[2] * b[0] - a[0] * b[2];
-    g[k + 1][2] = a[0] * b[1] - a[1] * b[0];
-  }
-  const double det = d[0][0] * g[1][0] + d[0][1] * g[1][1] + d[0][2] * g[1][2];
-  if (!(det > 0.0)) atomicMax(flags, e + 1);
-  const double id = 1.0 / det;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-#pragma unroll
-    for (int k = 1; k < 4; ++k) g[k][c] *= id;
-    g[0][c] = -(g[1][c] + g[2][c] + g[3][c]);
-  }
-  const double Ev = E[e], nv = nu[e], w = det / 120.0;
-  const double pad[4] = {w * (Ev * nv / ((1.0 + nv) * (1.0 - 2.0 * nv))), w * (Ev / (2.0 * (1.0 + nv))), 0.0, 0.0};
-  double2* o = reinterpret_cast<double2*>(rec + (size_t)e * kRec);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    o[2 * k] = make_double2(g[k][0], g[k][1]);
-    o[2 * k + 1] = make_double2(g[k][2], pad[k]);
-  }
-}
+// Element records (affine_records in element.hip): four gradients of four doubles.
+constexpr int kRec = 16;
 
 // corner pair of local node i: (i, i) for a corner, its edge's ends for a midside node
 __device__ __forceinline__ int pair_p(int i) { return i < 4 ? i : (0x210210 >> (4 * i - 16)) & 7; }
@@ -252,13 +186,6 @@ __global__ __launch_bounds__(256) void assemble_affine_diag_kernel(
   const unsigned f = node_fix ? node_fix[row] : 0u;
   const long long slot = base + 64LL * (bd / A.lanes) + (bd % A.lanes) * rps + r0;
   v64[val_index<double>(slot, sub, 9)] = with_supports(v, f, f, r, c, true);
-}
-
-int affine_records(int M, const int* conn, const double* nodes, const double* E, const double* nu, double* rec,
-                   int* flags, hipStream_t s) {
-  if (M <= 0) return kOk;
-  hipLaunchKernelGGL(affine_record_kernel, dim3(ceil_div(M, 128)), dim3(128), 0, s, M, conn, nodes, E, nu, rec, flags);
-  return static_cast<int>(hipGetLastError());
 }
 
 int assemble_affine(SellMatrix& A, const long long* cptr, const int* codes, const double* rec,

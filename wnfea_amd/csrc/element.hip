@@ -68,9 +68,8 @@ int upload_element_consts(hipStream_t s) {
   return kOk;
 }
 
-// Cartesian gradient of node `a` at Gauss point `g`; returns det J.
-__device__ __forceinline__ double node_gradient(const double (*X)[3], int g, int a, double grad[3]) {
-  double J[3][3];
+// J at Gauss point `g` and the cofactors of its first row; returns det J.
+__device__ __forceinline__ double jacobian(const double (*X)[3], int g, double (&J)[3][3], double (&cof)[3]) {
 #pragma unroll
   for (int r = 0; r < 3; ++r)
 #pragma unroll
@@ -80,10 +79,17 @@ __device__ __forceinline__ double node_gradient(const double (*X)[3], int g, int
       for (int i = 0; i < 10; ++i) s = fma(c_dndxi[g][r][i], X[i][c], s);
       J[r][c] = s;
     }
-  const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-  const double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-  const double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-  const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
+  cof[0] = J[1][1] * J[2][2] - J[1][2] * J[2][1];
+  cof[1] = J[1][2] * J[2][0] - J[1][0] * J[2][2];
+  cof[2] = J[1][0] * J[2][1] - J[1][1] * J[2][0];
+  return J[0][0] * cof[0] + J[0][1] * cof[1] + J[0][2] * cof[2];
+}
+
+// Cartesian gradient of node `a` at Gauss point `g`; returns det J.
+__device__ __forceinline__ double node_gradient(const double (*X)[3], int g, int a, double grad[3]) {
+  double J[3][3], cof[3];
+  const double det = jacobian(X, g, J, cof);
+  const double c00 = cof[0], c01 = cof[1], c02 = cof[2];
   const double id = 1.0 / det;
   const double inv[3][3] = {
       {c00 * id, (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id, (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id},
@@ -93,6 +99,84 @@ __device__ __forceinline__ double node_gradient(const double (*X)[3], int g, int
 #pragma unroll
   for (int r = 0; r < 3; ++r) grad[r] = inv[r][0] * d0 + inv[r][1] * d1 + inv[r][2] * d2;
   return det;
+}
+
+// Records of M affine elements for the assembly without element matrices
+// (assemble.hip): the gradients of the barycentric coordinates, each padded to
+// 32 bytes with lambda V/20 and mu V/20 in the first two pads.  flags[0] =
+// e + 1 of an element with det J <= 0, at its Gauss points where it is not
+// affine: the caller learns all that the element matrices could tell it from
+// one read, and launches those, if it needs them, without waiting again.
+// flags[1] = 1 when some element is not affine: a midside node is off its
+// edge's midpoint by more than 8 ulp of the element's largest coordinate.
+// That covers what rounding the midpoint, or rotating the mesh afterwards,
+// leaves (1 and 2 ulp), and is no more than the rounding of J at a Gauss point
+// (a sum of ten nodes' terms).  An offset that is small against the element's
+// size alone can still be large against its thickness, and J would lose it.
+__global__ __launch_bounds__(128) void affine_record_kernel(int M, const int* __restrict__ conn,
+                                                            const double* __restrict__ nodes,
+                                                            const double* __restrict__ E,
+                                                            const double* __restrict__ nu, double* __restrict__ rec,
+                                                            int* __restrict__ flags) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= M) return;
+  double X[10][3];
+#pragma unroll
+  for (int i = 0; i < 10; ++i) {
+    const size_t n3 = 3 * (size_t)conn[(size_t)e * 10 + i];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) X[i][c] = nodes[n3 + c];
+  }
+  double d[3][3], big = 0.0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) d[k][c] = X[k + 1][c] - X[0][c];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) big = fmax(big, fabs(X[i][c]));
+  constexpr int P[6] = {0, 1, 2, 0, 1, 2}, Q[6] = {1, 2, 0, 3, 3, 3};
+  bool flat = true;  // one comparison per coordinate: a NaN fails its own, where a maximum would drop it
+#pragma unroll
+  for (int m = 0; m < 6; ++m)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      flat = flat && fabs(X[4 + m][c] - 0.5 * (X[P[m]][c] + X[Q[m]][c])) <= 0x1p-49 * big;
+  // rows of the inverse of [d1 d2 d3]: the gradients of L_1, L_2, L_3
+  double g[4][3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double* a = d[(k + 1) % 3];
+    const double* b = d[(k + 2) % 3];
+    g[k + 1][0] = a[1] * b[2] - a[2] * b[1];
+    g[k + 1][1] = a[2] * b[0] - a[0] * b[2];
+    g[k + 1][2] = a[0] * b[1] - a[1] * b[0];
+  }
+  const double det = d[0][0] * g[1][0] + d[0][1] * g[1][1] + d[0][2] * g[1][2];
+  bool good = det > 0.0;
+  if (!flat) {
+    atomicOr(flags + 1, 1);
+    double J[3][3], cof[3];
+    good = true;
+    for (int g4 = 0; g4 < 4; ++g4) good = good && jacobian(X, g4, J, cof) > 0.0;
+  }
+  if (!good) atomicMax(flags, e + 1);
+  const double id = 1.0 / det;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+#pragma unroll
+    for (int k = 1; k < 4; ++k) g[k][c] *= id;
+    g[0][c] = -(g[1][c] + g[2][c] + g[3][c]);
+  }
+  const double Ev = E[e], nv = nu[e], w = det / 120.0;
+  const double pad[4] = {w * (Ev * nv / ((1.0 + nv) * (1.0 - 2.0 * nv))), w * (Ev / (2.0 * (1.0 + nv))), 0.0, 0.0};
+  double2* o = reinterpret_cast<double2*>(rec + (size_t)e * 16);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    o[2 * k] = make_double2(g[k][0], g[k][1]);
+    o[2 * k + 1] = make_double2(g[k][2], pad[k]);
+  }
 }
 
 constexpr int kElemPerBlock = 4;  // 4 wavefronts, one element each
@@ -1541,6 +1625,15 @@ int launch_ke(int M, const int* conn, const double* nodes, const double* E, cons
   else
     hipLaunchKernelGGL(c3d10_ke_kernel, dim3(ceil_div(M, kElemPerBlock)), dim3(256), 0, s, M, conn, nodes, E, nu, Ke,
                        bad);
+  return static_cast<int>(hipGetLastError());
+}
+
+int affine_records(int M, const int* conn, const double* nodes, const double* E, const double* nu, double* rec,
+                   int* flags, hipStream_t s) {
+  if (M <= 0) return kOk;
+  const int r = upload_element_consts(s);
+  if (r) return r;
+  hipLaunchKernelGGL(affine_record_kernel, dim3(ceil_div(M, 128)), dim3(128), 0, s, M, conn, nodes, E, nu, rec, flags);
   return static_cast<int>(hipGetLastError());
 }
 

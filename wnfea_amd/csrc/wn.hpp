@@ -315,7 +315,8 @@ int sell_to_std(const SellMatrix& A, double* vals_std, hipStream_t s);
 // symmetric part 0.5 (Ke + Ke^T); node_fix bit c marks DOF c of a node fixed.
 int assemble_elem(SellMatrix& A, int npe, int sym, const int* rowidx, const int* colidx, const long long* cptr,
                   const int* codes, const double* Ke, const unsigned char* node_fix, double* vals_std, hipStream_t s);
-// The C3D10 matrix of an affine mesh from its element records (16 doubles each)
+// The C3D10 matrix of an affine mesh from its element records (16 doubles each,
+// element.hip)
 int affine_records(int M, const int* conn, const double* nodes, const double* E, const double* nu, double* rec,
                    int* flags, hipStream_t s);
 int assemble_affine(SellMatrix& A, const long long* cptr, const int* codes, const double* rec,

@@ -193,21 +193,18 @@ def _assemble_values(K: DeviceBSR, mesh: dict, cptr, codes, fix) -> None:
     _lib.check(L.wnfea_c3d10_affine_records(*args, _lib.dptr(rec), _lib.dptr(flags), stream),
                "wnfea_c3d10_affine_records")
     bad, curved = flags.tolist()
-    if not curved and not bad:
-        _lib.check(L.wnfea_bsr_assemble_affine(K.handle, _lib.dptr(cptr), _lib.dptr(codes), _lib.dptr(rec),
-                                               _lib.dptr(fix), stream), "wnfea_bsr_assemble_affine")
-        return
-    if curved:
-        Ke = torch.empty((M, 30, 30), dtype=torch.float64, device=dev)
-        flags.zero_()
-        _lib.check(L.wnfea_c3d10_ke(*args, _lib.dptr(Ke), _lib.dptr(flags), stream), "wnfea_c3d10_ke")
-        _lib.check(L.wnfea_bsr_assemble(K.handle, _lib.dptr(K.d_rowidx), _lib.dptr(K.d_colidx), _lib.dptr(cptr),
-                                        _lib.dptr(codes), _lib.dptr(Ke), _lib.dptr(fix), None, stream),
-                   "wnfea_bsr_assemble")
-        bad = int(flags[0].item())
     if bad:
         raise ValueError(f"Non-positive Jacobian determinant in C3D10 element {bad - 1}. "
                          "Element is inverted, degenerate, or has bad node numbering.")
+    if not curved:
+        _lib.check(L.wnfea_bsr_assemble_affine(K.handle, _lib.dptr(cptr), _lib.dptr(codes), _lib.dptr(rec),
+                                               _lib.dptr(fix), stream), "wnfea_bsr_assemble_affine")
+        return
+    Ke = torch.empty((M, 30, 30), dtype=torch.float64, device=dev)
+    _lib.check(L.wnfea_c3d10_ke(*args, _lib.dptr(Ke), _lib.dptr(flags), stream), "wnfea_c3d10_ke")
+    _lib.check(L.wnfea_bsr_assemble(K.handle, _lib.dptr(K.d_rowidx), _lib.dptr(K.d_colidx), _lib.dptr(cptr),
+                                    _lib.dptr(codes), _lib.dptr(Ke), _lib.dptr(fix), None, stream),
+               "wnfea_bsr_assemble")
 
 
 def reassemble_c3d10_values(system: SolidSystem, E=None, nu=None) -> SolidSystem:
