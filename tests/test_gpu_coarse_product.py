@@ -31,3 +31,38 @@ def test_cycle_is_the_inverse_product(cells, rows):
     mag = np.abs(inv32) @ np.abs(r32.astype(np.float64))
     assert np.all(np.abs(z32 - ref) <= 6.0e-8 * np.abs(ref) + rows * 2.3e-16 * mag)
     amg.close()
+
+
+def test_captured_iterations_follow_the_coarse_precision():
+    """Sixteen captured CG iterations with the FP32 cycle's coarsest product
+    switched between the FP32 and the FP64 inverse: the bits of host launches
+    at each setting, also where the iterations of another one were captured
+    last."""
+    import torch
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr, build_amg, pcg_device, set_graphs
+    m, _ = generate_c3d10_structured_block(1.0, 0.1, 0.1, 20, 2, 2, tip_load_total=-1000.0, tets_per_hex=6,
+                                           load_direction="z")
+    system = assemble_c3d10_bsr(m, want_fp64_equilibrated=True)
+    amg = build_amg(system, storage=("fp64", "fp32"), autotune=False, coarse_size=600)
+    kw = dict(rtol=1e-30, max_iter=16, check_every=8, preconditioner="amg", precision="fp64", amg=amg,
+              amg_precision="fp32")
+    host, got = {}, []
+    try:
+        assert len(amg.levels) == 2
+        for prec in ("fp32", "fp64"):
+            amg.set_coarse_precision(prec)
+            host[prec] = pcg_device(system, **kw)[0].cpu()
+        assert not torch.equal(host["fp32"], host["fp64"])
+        set_graphs(True)
+        for prec in ("fp32", "fp64", "fp64", "fp32"):
+            amg.set_coarse_precision(prec)
+            x = pcg_device(system, **kw)[0]
+            got.append((prec, x.data_ptr(), x.cpu()))
+            del x  # the next call's solution takes its place
+    finally:
+        set_graphs(False)
+        amg.close()
+    assert len({p for _, p, _ in got}) == 1  # the same buffers throughout
+    for prec, _, x in got:
+        assert torch.equal(x, host[prec]), prec

@@ -578,7 +578,7 @@ static void key_mf(std::vector<uint64_t>& k, const MfOp& m) {
 static void key_amg(std::vector<uint64_t>& k, const Amg* g) {
   key_push(k, g);
   if (!g) return;
-  for (int v : {g->store, g->n_coarse, (int)g->L.size()}) key_push(k, v);
+  for (int v : {g->store, g->n_coarse, g->coarse_fp64, (int)g->L.size()}) key_push(k, v);
   for (const void* p : {(const void*)g->inv, (const void*)g->inv32, (const void*)g->tiles64, (const void*)g->tiles32,
                         (const void*)g->tij, (const void*)g->tpart, (const void*)g->mfs.op,
                         (const void*)g->mfs.s64, (const void*)g->mfs.s64e, (const void*)g->mfs.s32,
@@ -591,7 +591,7 @@ static void key_amg(std::vector<uint64_t>& k, const Amg* g) {
   key_tune(k, g->tune);
   for (const auto& lp : g->L) {
     const AmgLevel& l = *lp;
-    for (int v : {l.n, l.degree, (int)l.has_PR}) key_push(k, v);
+    for (int v : {l.n, l.degree, (int)l.has_PR, (int)l.unit64, (int)l.unit32}) key_push(k, v);
     key_push(k, l.lmax);
     key_push(k, l.ratio);
     key_push(k, l.dinv64);
