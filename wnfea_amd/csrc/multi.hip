@@ -11,6 +11,7 @@
 // solver: FP64 Krylov vectors, SpMM and updates; the V-cycle in FP32 on S K S
 // as z = S M(S r).
 #include <cmath>
+#include "multi_state.hpp"
 #include "sell.hpp"
 #include "solver.hpp"
 
@@ -448,50 +449,6 @@ static int mr_grid(long long n) {
   return static_cast<int>(g < 1 ? 1 : g);
 }
 
-// Per-level column vectors of the multi-column cycle (b, x, tmp, d, res).
-template <typename T>
-struct MrLevel {
-  T* v[5] = {};
-};
-
-struct MultiState {
-  int nr = 0;
-  long long n = 0;
-  std::vector<MrLevel<float>> lv32;
-  std::vector<MrLevel<double>> lv64;
-  std::vector<int> level_n;  // rows the level vectors were sized for
-  double *r = nullptr, *p = nullptr, *q = nullptr, *zs = nullptr;  // FP64 n x NR
-  float *rp32 = nullptr, *zp32 = nullptr;                           // FP32 n x NR
-  double* partials = nullptr;  // NR x max blocks
-  int max_blocks = 0;
-  double* sc = nullptr;  // per-column scalars: kMs* x NR
-  int* flags = nullptr;  // [0] all done, [1] iteration, [2..2+NR) done per column, [2+NR..) iterations per column
-  double* h_sc = nullptr;
-  int* h_flags = nullptr;
-  void release() {
-    for (auto& l : lv32)
-      for (auto* p_ : l.v) if (p_) (void)hipFree(p_);
-    for (auto& l : lv64)
-      for (auto* p_ : l.v) if (p_) (void)hipFree(p_);
-    lv32.clear();
-    lv64.clear();
-    for (void* p_ : {(void*)r, (void*)p, (void*)q, (void*)zs, (void*)rp32, (void*)zp32, (void*)partials, (void*)sc,
-                     (void*)flags})
-      if (p_) (void)hipFree(p_);
-    if (h_sc) (void)hipHostFree(h_sc);
-    if (h_flags) (void)hipHostFree(h_flags);
-    r = p = q = zs = nullptr;
-    rp32 = zp32 = nullptr;
-    partials = sc = h_sc = nullptr;
-    flags = h_flags = nullptr;
-    n = 0;
-    nr = 0;
-    level_n.clear();
-  }
-};
-
-enum MsIdx { kMsRho = 0, kMsRhoPrev, kMsBeta, kMsAlpha, kMsGamma, kMsRR, kMsRR0, kMsTol2, kMsCount };
-
 static void multi_free(void* p) {
   auto* m = static_cast<MultiState*>(p);
   m->release();
@@ -503,44 +460,10 @@ static int multi_ensure(Solver& S, long long n, int nr, const Amg* g, int need64
     S.multi = new MultiState();
     S.multi_free = multi_free;
   }
-  MultiState& M = *static_cast<MultiState*>(S.multi);
-  const int blocks = std::max(n_blocks + 8, 4096);
   std::vector<int> level_n;
   if (g)
     for (const auto& l : g->L) level_n.push_back(l->n);
-  bool same = M.r && M.n >= n && M.nr == nr && M.max_blocks >= blocks && M.level_n.size() == level_n.size() &&
-              M.lv32.size() == level_n.size() && (!need64cycle || M.lv64.size() == level_n.size());
-  for (size_t l = 0; same && l < level_n.size(); ++l) same = M.level_n[l] >= level_n[l];
-  if (same) return kOk;
-  M.release();
-  M.n = n;
-  M.nr = nr;
-  M.level_n = level_n;
-  M.max_blocks = blocks;
-  const size_t nv = (size_t)n * nr;
-  WN_HIP(hipMalloc(&M.r, sizeof(double) * nv));
-  WN_HIP(hipMalloc(&M.p, sizeof(double) * nv));
-  WN_HIP(hipMalloc(&M.q, sizeof(double) * nv));
-  WN_HIP(hipMalloc(&M.zs, sizeof(double) * nv));
-  WN_HIP(hipMalloc(&M.rp32, sizeof(float) * nv));
-  WN_HIP(hipMalloc(&M.zp32, sizeof(float) * nv));
-  WN_HIP(hipMalloc(&M.partials, sizeof(double) * nr * (size_t)blocks));
-  WN_HIP(hipMalloc(&M.sc, sizeof(double) * kMsCount * nr));
-  WN_HIP(hipMalloc(&M.flags, sizeof(int) * (2 + 2 * nr)));
-  WN_HIP(hipHostMalloc(&M.h_sc, sizeof(double) * kMsCount * nr, 0));
-  WN_HIP(hipHostMalloc(&M.h_flags, sizeof(int) * (2 + 2 * nr), 0));
-  if (g) {
-    M.lv32.resize(g->L.size());
-    if (need64cycle) M.lv64.resize(g->L.size());
-    for (size_t l = 0; l < g->L.size(); ++l) {
-      const size_t m = (size_t)std::max(g->L[l]->n, 1) * nr;
-      for (int k = 0; k < 5; ++k) {
-        WN_HIP(hipMalloc(&M.lv32[l].v[k], sizeof(float) * m));
-        if (need64cycle) WN_HIP(hipMalloc(&M.lv64[l].v[k], sizeof(double) * m));
-      }
-    }
-  }
-  return kOk;
+  return static_cast<MultiState*>(S.multi)->ensure(n, nr, level_n, need64cycle, std::max(n_blocks + 8, 4096));
 }
 
 template <typename T> static std::vector<MrLevel<T>>& mr_levels(MultiState& M);
