@@ -66,3 +66,43 @@ def test_captured_iterations_follow_the_coarse_precision():
     assert len({p for _, p, _ in got}) == 1  # the same buffers throughout
     for prec, _, x in got:
         assert torch.equal(x, host[prec]), prec
+
+
+@pytest.mark.parametrize("group", [4, 8])
+@pytest.mark.parametrize("cells,rows", [((1, 1, 1), 81), ((3, 1, 1), 189), ((16, 2, 2), 2475), ((20, 2, 2), 3075)])
+def test_columns_are_the_inverse_product(cells, rows, group):
+    """Several columns on a hierarchy of one level, whose rows end inside a run
+    of 32 columns and a block of 16 rows.  The first CG iterate of column k is
+    alpha_k S z_k, z_k = inv32 (S b_k)_32 with the sum in FP64 and rounded
+    once: alpha_k, one factor per column, is taken from the median entry,
+    which adds that entry's own rounding."""
+    import torch
+    from wnfea_amd import _lib
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block
+    from wnfea_amd.solver.solid_solver import _Solver, assemble_c3d10_bsr, build_amg
+    print(f"coarsest product of {rows} rows, {group} columns", flush=True)
+    m, _ = generate_c3d10_structured_block(0.05 * cells[0], 0.1, 0.1, *cells, tip_load_total=-1000.0, tets_per_hex=6,
+                                           load_direction="z")
+    system = assemble_c3d10_bsr(m)
+    amg = build_amg(system, storage=("fp32",), autotune=False)
+    assert len(amg.levels) == 1 and amg.coarse_inv.shape[0] == rows
+    B = np.random.default_rng(rows).standard_normal((rows, group))
+    Bd = torch.as_tensor(B, device="cuda")
+    X = torch.empty_like(Bd)
+    its, rel = (_lib.ctypes.c_int * group)(), (_lib.ctypes.c_double * group)()
+    _lib.check(_lib.load().wnfea_pcg_multi(_Solver.get(), system.K.handle, amg.handle, 1, _lib.dptr(system.scale), group,
+                                           _lib.dptr(Bd), _lib.dptr(X), 1e-30, 1, 1, its, rel, _lib.stream_of()), "pcg")
+    assert list(its) == [1] * group
+    S = system.scale.cpu().numpy()[:, None]
+    r32 = (S * B).astype(np.float32).astype(np.float64)
+    inv32 = amg.coarse_inv.astype(np.float32).astype(np.float64)
+    z, mag = inv32 @ r32, np.abs(inv32) @ np.abs(r32)
+    bound = 6.0e-8 * np.abs(z) + rows * 2.3e-16 * mag
+    x = X.cpu().numpy() / S
+    for k in range(group):
+        j = np.argsort(np.abs(z[:, k]))[rows // 2]
+        alpha = x[j, k] / z[j, k]
+        assert alpha > 0.0
+        slack = bound[j, k] / abs(z[j, k])
+        assert np.all(np.abs(x[:, k] / alpha - z[:, k]) <= 1.01 * (bound[:, k] + slack * np.abs(z[:, k])))
+    amg.close()

@@ -394,12 +394,15 @@ __global__ void mr_cheb_first_kernel(long long n, const T* __restrict__ b, const
 // X[i][k] = sum_j inv[i][j] B[j][k] on the coarsest level, products and sums
 // in FP64 (v_mfma_f64_16x16x4f64: lane l supplies A[l % 16][l / 16] and
 // B[l / 16][l % 16], result r of lane l is D[4 r + l / 16][l % 16]).  A
-// workgroup owns 16 rows; its 16 wavefronts take every 16th run of 16 columns
-// of the inverse, each lane four consecutive entries of its row, and meet in
-// LDS in wavefront order.  Bound by the inverse's bytes, and on a small level
-// by the chain of loads; one 256-thread workgroup per row with 8 FP64
-// reductions each took 19.5 us at 2 082 rows (194 us at 10 740), this kernel
-// 13.7 us.
+// workgroup owns 16 rows; its 16 wavefronts take every 16th run of 32 columns
+// of the inverse, each lane twice four consecutive entries of its row in one
+// load, and meet in LDS in wavefront order.  Bound by the inverse's bytes, and
+// on a small level by the chain of loads.  FP32 inverse, us, 8 columns: 256
+// threads per row and 8 FP64 reductions 21.1 at 2 244 rows, 172 at 8 622, 265
+// at 10 740; runs of 16 columns in single loads 175 and 229 at the last two;
+// here 10.2, 89 and 131.  4 columns: 14.0, 116 and 176; 15.1 and 164 at the
+// first two; here 9.7, 83 and 124.  Runs of 64 columns, or 8 wavefronts (which
+// fit the chip in one round up to 16 384 rows), are up to 8 % slower.
 typedef double mr_d4 __attribute__((ext_vector_type(4)));
 constexpr int kMrCoarseWaves = 16;
 
@@ -408,26 +411,41 @@ __global__ __launch_bounds__(64 * kMrCoarseWaves) void mr_coarse_kernel(int n, c
                                                                         const T* __restrict__ b, T* __restrict__ x,
                                                                         const int* skip) {
   if (skip && *skip) return;
-  __shared__ double red[kMrCoarseWaves][16][NR];
+  constexpr int W = kMrCoarseWaves, U = 2, RUN = 16 * U;  // RUN: columns a wavefront takes at a time
+  using V4 = T __attribute__((ext_vector_type(4), aligned(sizeof(T))));  // rows start at any multiple of T
+  __shared__ double red[W][16][NR];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lk = lane >> 4;
   const int i = blockIdx.x * 16 + lr;
   const T* __restrict__ row = inv + (size_t)min(i, n - 1) * n;
+  const T* __restrict__ col = b + (lr < NR ? lr : 0);
   mr_d4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int k0 = 16 * wave; k0 < n; k0 += 16 * kMrCoarseWaves) {
+  int k0 = RUN * wave;
+  for (; k0 + RUN <= n; k0 += RUN * W) {
     const int k = k0 + 4 * lk;
-    T av[4], bv[4];
+    V4 av[U];
+    T bv[U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) av[u] = *reinterpret_cast<const V4*>(row + k + 16 * u);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bv[u][e] = col[(size_t)(k + 16 * u + e) * NR];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(double(av[u][e]), lr < NR ? double(bv[u][e]) : 0.0, acc, 0, 0, 0);
+  }
+  // the last, partial run, whose wavefront ends there: clamped, in bounds
+  for (; k0 < n; k0 += 16) {
+    const int k = k0 + 4 * lk;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int kk = min(k + e, n - 1);  // in bounds; the padding's products are zero through bv
-      av[e] = row[kk];
-      bv[e] = b[(size_t)kk * NR + (lr < NR ? lr : 0)];
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool ok = k + e < n && lr < NR;
-      const double a = k + e < n ? double(av[e]) : 0.0;
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, ok ? double(bv[e]) : 0.0, acc, 0, 0, 0);
+      const bool in = k + e < n;
+      const int kk = min(k + e, n - 1);
+      const double av = in ? double(row[kk]) : 0.0, bv = in && lr < NR ? double(col[(size_t)kk * NR]) : 0.0;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc, 0, 0, 0);
     }
   }
 #pragma unroll
@@ -438,7 +456,7 @@ __global__ __launch_bounds__(64 * kMrCoarseWaves) void mr_coarse_kernel(int n, c
     const int r = t / NR, k = t % NR, o = blockIdx.x * 16 + r;
     double v = 0.0;
 #pragma unroll
-    for (int w = 0; w < kMrCoarseWaves; ++w) v += red[w][r][k];
+    for (int w = 0; w < W; ++w) v += red[w][r][k];
     if (o < n) x[(size_t)o * NR + k] = T(v);
   }
 }
