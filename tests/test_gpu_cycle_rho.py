@@ -96,3 +96,11 @@ def test_carried_finalisation_matrix_free(cells, cycle):
         assert it == runs[0][1] and rel == runs[0][3] <= 1e-8 and torch.equal(u, runs[0][0])
     op.close()
     amg.close()
+
+
+@pytest.mark.timeout(120)
+@pytest.mark.parametrize("nx", [5120, 5121])
+def test_cg_iterates_where_the_rho_pass_returns(nx):
+    """On both sides of the 2 560 partials (slices of 32 rows, padded to the 8
+    XCDs) up to which the last product forms rho."""
+    test_cg_iterates(3, nx, "fp64", "fp64")

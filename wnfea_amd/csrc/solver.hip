@@ -424,12 +424,21 @@ int amg_first_launch(const FirstIter<T>& f, long long n, const T* b, const int* 
 template int amg_first_launch<double>(const FirstIter<double>&, long long, const double*, const int*, hipStream_t);
 template int amg_first_launch<float>(const FirstIter<float>&, long long, const float*, const int*, hipStream_t);
 
-// Partials the cycle of kind vt writes for a RhoReq (0: that cycle cannot
-// form rho: its values and vectors differ in type, or its finest level is
-// smoothed matrix-free element by element).
+// Partials the cycle of kind vt writes for a RhoReq (0: that cycle does not
+// form rho: its values and vectors differ in type, its finest level is
+// smoothed matrix-free element by element, or assembled with more than
+// kCycleRhoMax partials).  A product writes one partial per slice, and every
+// workgroup of the p update adds all of them up: with many, that costs more
+// than the rho pass, whose partials are at most 2048.  A whole I-beam solve
+// with the separate pass against without, FP32 cycle, ms: 2 232 partials (107
+// 055 rows) 5.20 / 5.18, 3 040 6.13 / 6.15, 5 528 9.57 / 9.69, 11 008 15.35 /
+// 15.65; FP64 7.09 / 7.05, 8.49 / 8.53, 13.88 / 13.97, 23.40 / 23.68.
+constexpr int kCycleRhoMax = 2560;
 template <typename T>
 static int rho_blocks(const Amg& g) {
-  return mf_smooth_ready<T>(g.mfs) ? mf_smooth_rho_blocks<T>(g.mfs) : spmv_partials<T>(*g.L[0]->A, g.tune);
+  if (mf_smooth_ready<T>(g.mfs)) return mf_smooth_rho_blocks<T>(g.mfs);
+  const int nb = spmv_partials<T>(*g.L[0]->A, g.tune);
+  return nb <= kCycleRhoMax ? nb : 0;
 }
 int amg_rho_blocks(const Amg& g, int vt) {
   if (g.L.size() < 2) return 0;
