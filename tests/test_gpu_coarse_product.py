@@ -106,3 +106,30 @@ def test_columns_are_the_inverse_product(cells, rows, group):
         slack = bound[j, k] / abs(z[j, k])
         assert np.all(np.abs(x[:, k] / alpha - z[:, k]) <= 1.01 * (bound[:, k] + slack * np.abs(z[:, k])))
     amg.close()
+
+
+@pytest.mark.parametrize("cells,rows", [((1, 1, 1), 81), ((16, 2, 2), 2475), ((20, 2, 2), 3075)])
+def test_fp32_cycle_on_the_fp64_inverse(cells, rows):
+    """An FP32 cycle told to apply the FP64 inverse: by rows up to 2 048, by
+    tiles beyond.  Only its input and its result are rounded to FP32."""
+    import torch
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block
+    from wnfea_amd.solver.solid_solver import assemble_c3d10_bsr, build_amg
+    print(f"FP64 coarsest product of {rows} rows in an FP32 cycle", flush=True)
+    m, _ = generate_c3d10_structured_block(1.0, 0.1, 0.1, *cells, tip_load_total=-1000.0, tets_per_hex=6,
+                                           load_direction="z")
+    amg = build_amg(assemble_c3d10_bsr(m, want_fp64_equilibrated=True), storage=("fp64", "fp32"), autotune=False)
+    inv = amg.coarse_inv
+    assert len(amg.levels) == 1 and inv.shape[0] == rows
+    r32 = np.random.default_rng(rows).standard_normal(rows).astype(np.float32)
+    rd = torch.as_tensor(r32, device="cuda")
+    plain = amg.vcycle(rd)
+    amg.set_coarse_precision("fp64")
+    z = amg.vcycle(rd)
+    amg.set_coarse_precision("fp32")
+    assert torch.equal(amg.vcycle(rd), plain) and not torch.equal(z, plain)
+    ref = inv @ r32.astype(np.float64)
+    mag = np.abs(inv) @ np.abs(r32.astype(np.float64))
+    err = np.abs(z.double().cpu().numpy() - ref)
+    assert np.all(err <= 6.0e-8 * np.abs(ref) + rows * 2.3e-16 * mag)
+    amg.close()

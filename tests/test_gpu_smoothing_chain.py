@@ -44,3 +44,46 @@ def test_chain_is_the_per_element_cycle(cells, patches, degree):
     finally:
         op.close()
         amg.close()
+
+
+@pytest.mark.parametrize("degree", [1, 2])
+def test_nodes_of_no_element_take_the_node_kernels(degree):
+    """A clamped node that belongs to no element, and so to no patch, amid the
+    others and one at their end: the chain, whose patches store the steps of
+    the nodes they hold, stays off, and the cycle is the per-element path's on
+    every node, these two included."""
+    import dataclasses
+
+    import torch
+    from wnfea_amd.mesh.solid_generator import generate_c3d10_structured_block
+    from wnfea_amd.solver.solid_solver import (MatrixFreeOperator, assemble_c3d10_bsr, build_amg, solve_mixed,
+                                               true_residual)
+    print(f"nodes of no element, degree {degree}", flush=True)
+    m, _ = generate_c3d10_structured_block(0.3, 0.04, 0.04, 12, 2, 2, tip_load_total=-1000.0, tets_per_hex=6,
+                                           load_direction="z")
+    n, k = len(m.mesh_nodes), 100
+    m.mesh_nodes = np.vstack([m.mesh_nodes[:k], [[0.1, 0.1, 0.1]], m.mesh_nodes[k:], [[0.2, 0.1, 0.1]]])
+    m.solid_elements = m.solid_elements + (m.solid_elements >= k)
+    clamp = m.supports[0]
+    for item in (*m.supports, *m.loads):
+        item.node_id += int(item.node_id >= k)
+    m.supports += [dataclasses.replace(clamp, node_id=i) for i in (k, n + 1)]
+    system = assemble_c3d10_bsr(m, want_fp64_equilibrated=True)
+    own = torch.tensor([3 * k, 3 * k + 1, 3 * k + 2, 3 * n + 3, 3 * n + 4, 3 * n + 5], device="cuda")
+    assert bool(torch.as_tensor(system.fixed_mask, device="cuda")[own].all())
+    amg = build_amg(system, storage=("fp64", "fp32"), autotune=False, level_degrees=[degree], coarse_size=400)
+    op = MatrixFreeOperator(system)
+    try:
+        op.attach_smoother(amg)
+        rd = torch.as_tensor(np.random.default_rng(7).standard_normal(system.n_dofs), device="cuda")
+        z64, z32 = amg.vcycle(rd), amg.vcycle(rd.float())
+        for prec in ("fp64", "fp32"):
+            u, _, _, rel, _ = solve_mixed(system, amg, tol=1e-8, amg_precision=prec, operator=op)
+            assert rel <= 1e-8 and true_residual(system, u) <= 1.5e-8, prec
+        op.set_patch(0)
+        z64e, z32e = amg.vcycle(rd), amg.vcycle(rd.float())
+        assert _rel(z64, z64e) <= 1e-13 and _rel(z32, z32e) <= 1e-5
+        assert _rel(z64[own], z64e[own]) <= 1e-13 and _rel(z32[own], z32e[own]) <= 1e-5
+    finally:
+        op.close()
+        amg.close()
