@@ -1241,7 +1241,7 @@ def main() -> int:
                       "launches_per_iteration": 3,
                       "kernel": f"sell_spmv_kernel<6,6,float,float,"
                                 f"{cycle_tune['fp32']['waves'] if cycle_tune else tune['waves']},"
-                                f"{cycle_tune['fp32']['unroll'] if cycle_tune else tune['unroll']},OpCheb<6,float>> "
+                                f"{cycle_tune['fp32']['unroll'] if cycle_tune else tune['unroll']},1,OpCheb<6,float>> "
                                 f"(FP32 Chebyshev smoothing step of AMG level 1: {lv1['n']} rows, {nnzb1} 6x6 blocks)",
                       "fp64_twin": {"avg_launch_us": round(t_ch64 * 1e6, 2), "algorithmic_bytes": ch64,
                                     "frac": round(ch64 / t_ch64 / 1e9 / HBM_PEAK_GBS, 4)}} if has_l1 else

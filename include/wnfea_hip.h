@@ -157,8 +157,8 @@ int wnfea_adjoint_grad(int M, const int *conn, const double *nodes, const double
 
 /* Co-rotational internal forces of 2-node beams, FP64, deterministic.
  * conn[M][2], nodes[N][3], props[M][6] = (E, G, A, Iy, Iz, J), U[N][6]
- * (device); fe_work[M][12] device scratch (required, not used: the element
- * forces stay on the chip); n2e_ptr/n2e the node incidence
+ * (device); fe_work is not used and may be NULL (the element forces stay on
+ * the chip); n2e_ptr/n2e the node incidence
  * (wnfea_node_incidence with npe = 2); F[N][6] (accumulate != 0 adds).
  * Replaces hip_compute_beam_forces (wnfea/solver/native/hip_kernels.cpp:53-241),
  * compute_corotational_element_forces (wnfea/solver/corotational_beam.py:178-233)
@@ -354,7 +354,8 @@ int wnfea_bsr_assemble_affine(void *h, const long long *cptr, const int *codes, 
 /* Element matrices Ke[M][npe*b][npe*b] of b x b-block matrix h (b = 3 or 6)
  * through the contribution lists (codes e*npe*npe + a*npe + c); sym != 0
  * assembles 0.5 (Ke + Ke^T); node_fix bits as wnfea_bsr_assemble (bit c =
- * DOF c fixed).  Replaces the beam branch of assemble_global_system_sparse
+ * DOF c fixed).  rowidx and colidx are read for 3x3 blocks alone, but may not
+ * be NULL.  Replaces the beam branch of assemble_global_system_sparse
  * (wnfea/solver/assembler.py:285-450) and hip_assemble_beam_system_csr
  * (wnfea/solver/fast_kernels.py:666-763). */
 int wnfea_bsr_assemble_elem(void *h, int npe, int sym, const int *rowidx, const int *colidx, const long long *cptr,
@@ -366,6 +367,7 @@ int wnfea_bsr_diag(void *h, const long long *diag_block, double *diag, void *str
 
 /* FP32 values of S K S with S = diag(scale) (device), plus the FP64 copy
  * (want64e) and an FP16 copy (want16) for lower-precision preconditioning.
+ * rowidx and colidx may not be NULL, but are not read for 3x3 and 6x6 blocks.
  * Replaces the equilibration of BlockBeamAMGPreconditioner
  * (wnfea/solver/amg_preconditioner.py:180-185) and its FP16 value copies
  * (wnfea/solver/native/hip_kernels.cpp:1924-2060, precision_mode 2). */

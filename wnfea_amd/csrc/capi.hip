@@ -153,7 +153,8 @@ int wnfea_adjoint_grad(int M, const int* conn, const double* nodes, const double
 int wnfea_beam_forces(int M, int n_nodes, const int* conn, const double* nodes, const double* props, const double* U,
                       const int* n2e_ptr, const int* n2e, double* fe_work, double* F, int accumulate, void* stream) {
   if (M < 0 || n_nodes < 0) return kBadArg;
-  if (M > 0 && (!conn || !nodes || !props || !U || !fe_work)) return kBadArg;
+  (void)fe_work;
+  if (M > 0 && (!conn || !nodes || !props || !U)) return kBadArg;
   if (n_nodes > 0 && (!n2e_ptr || !n2e || !F)) return kBadArg;
   return launch_beam_forces(M, n_nodes, conn, nodes, props, U, n2e_ptr, n2e, F, accumulate, S(stream));
 }

@@ -821,7 +821,7 @@ __device__ __forceinline__ void gauss_point_consts(int g, T (&c4)[4], T (&cc)[4]
 
 // The edge between vertices v and v ^ m of a tetrahedron, as its midside node
 // (Abaqus order): kEdgeOf[v][m - 1].
-__host__ __device__ constexpr int kEdgeOf[4][3] = {{4, 6, 7}, {4, 8, 5}, {9, 6, 5}, {9, 8, 7}};
+constexpr int kEdgeOf[4][3] = {{4, 6, 7}, {4, 8, 5}, {9, 6, 5}, {9, 8, 7}};
 
 // The element forces of an affine element by vertices instead of Gauss points:
 // its strain is linear, so the strains at the four vertices determine it, and

@@ -19,18 +19,6 @@ namespace wn {
 
 constexpr int kMrBlock = 256;
 
-template <typename XT, int NR>
-__device__ __forceinline__ void load_cols(const XT* __restrict__ p, XT (&v)[NR]) {
-  constexpr int V = 16 / (int)sizeof(XT);
-  static_assert(NR % V == 0, "columns must fill 16-byte loads");
-#pragma unroll
-  for (int g = 0; g < NR / V; ++g) {
-    const VecN<XT, V> c = *reinterpret_cast<const VecN<XT, V>*>(p + g * V);
-#pragma unroll
-    for (int i = 0; i < V; ++i) v[g * V + i] = c.e[i];
-  }
-}
-
 // Sliced-ELL block SpMM (layout of sell.hpp) on NR interleaved columns.
 //
 // Bound: L1 and instruction issue.  A block's BC x rows (96 bytes for FP32
@@ -57,7 +45,7 @@ __device__ __forceinline__ void load_cols(const XT* __restrict__ p, XT (&v)[NR])
 // and gains nothing; one scalar column per lane, three times the loads, takes
 // 75 / 80 / 45.)
 template <int BR, int BC, typename XT, int NR>
-constexpr int spmm_waves() {  // wavefronts per workgroup: at most 56 KB of LDS
+constexpr int spmm_waves() {  // wavefronts per workgroup: at most 48 KB of LDS for x
   return BC * NR * (int)sizeof(XT) > 208 ? 2 : 4;
 }
 

@@ -136,8 +136,9 @@ int SellMatrix::build(int br_, int bc_, int n_rows_, int n_cols_, const int* row
         col[sl] = colidx[rowptr[g] + j];
         slot[rowptr[g] + j] = sl;
       }
-      // padding slots keep column 0 and value 0; lanes stop at their own
-      // step count, so they are never read.
+      // padding slots keep column 0, and value 0 (ensure_values clears every
+      // slot): the products stop at each lane's own step count, but kernels
+      // that take a step whole (sell_to_std_kernel, the SpMM's loads) read them
     }
   WN_HIP(hipMalloc(&d_off, sizeof(long long) * off.size()));
   WN_HIP(hipMalloc(&d_rinfo, sizeof(int2) * rinfo.size()));

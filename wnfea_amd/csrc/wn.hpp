@@ -190,7 +190,8 @@ int mf_smooth_end_defect(const MfSmooth& m, int from, const T* x, const T* b, T*
 template <typename T>
 int mf_smooth_end_cheb(const MfSmooth& m, int from, const T* x, T* x_out, const T* b, const T* dinv, T* d, T c1, T c2,
                        const RhoReq* rq, const int* skip, hipStream_t s);
-// Partials mf_smooth_cheb_rho writes in precision T (0: it cannot run).
+// Partials mf_smooth_end_cheb writes for a RhoReq in precision T (0: not in the
+// patch layout).
 template <typename T>
 int mf_smooth_rho_blocks(const MfSmooth& m);
 std::vector<int> mf_chunks(const std::vector<int>& n2e_ptr);
@@ -227,9 +228,10 @@ int launch_adjoint_dot(int M, const int* conn, const double* E, const double* fe
 
 // -------- vector kernels (blas.hip)
 int vec_grid(long long n);
-// one-block finalisation of block partials (FinMode in common.hpp)
+// squared norms of a - b over groups of nodes (blas.hip)
 int launch_group_norms2(int n_groups, int n_chunks, int dpn, const int* cptr, const int* chunk, const int* perm,
                         const double* a, const double* b, double* partials, double* out, hipStream_t s);
+// one-block finalisation of block partials (FinMode in common.hpp)
 int launch_finalize(const double* partials, int nb, int K, int mode, double* out, double* sc, int* flags, int first,
                     const int* skip, hipStream_t s);
 template <typename T> int launch_fill(long long n, T* x, T v, hipStream_t s);

@@ -80,7 +80,6 @@ class BeamSystem:
         self.d = {"nodes": t(nodes), "conn": t(conn), "props": t(props), "n2e_ptr": t(n2e_ptr), "n2e": t(n2e),
                   "cptr": t(cptr), "codes": t(codes[:max(nc, 1)].copy()), "fix": t(node_fix)}
         self.n_nodes, self.n_beams = n, M
-        self.fe = torch.empty((max(M, 1), 12), dtype=torch.float64, device=dev)
         K = DeviceBSR(6, 6, n, n, rowptr, colidx, sigma)
         F = model.load_vector(6)
         F[fixed] = 0.0
@@ -111,7 +110,7 @@ class BeamSystem:
         d = self.d
         _lib.check(L.wnfea_beam_forces(self.n_beams, self.n_nodes, _lib.dptr(d["conn"]), _lib.dptr(d["nodes"]),
                                        _lib.dptr(d["props"]), _lib.dptr(U), _lib.dptr(d["n2e_ptr"]),
-                                       _lib.dptr(d["n2e"]), _lib.dptr(self.fe), _lib.dptr(F), 0, _lib.stream_of()),
+                                       _lib.dptr(d["n2e"]), None, _lib.dptr(F), 0, _lib.stream_of()),
                    "wnfea_beam_forces")
         return F
 

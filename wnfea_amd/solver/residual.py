@@ -87,7 +87,7 @@ class _ForceContext:
             t = lambda a: torch.as_tensor(a, device=dev)  # noqa: E731
             props = np.ascontiguousarray(beam_props(model))
             self.beams = {"M": M, "conn": t(conn), "nodes": t(nodes), "props": t(props), "ptr": t(ptr),
-                          "inc": t(inc), "fe": torch.empty((M, 12), dtype=torch.float64, device=dev)}
+                          "inc": t(inc)}
         self.solids = None
         if getattr(model, "solid_elements", None) is not None and len(model.solid_elements):
             m = mesh_to_device(model, dev)
@@ -111,8 +111,8 @@ class _ForceContext:
             b = self.beams
             _lib.check(L.wnfea_beam_forces(b["M"], self.n, _lib.dptr(b["conn"]), _lib.dptr(b["nodes"]),
                                            _lib.dptr(b["props"]), _lib.dptr(U), _lib.dptr(b["ptr"]),
-                                           _lib.dptr(b["inc"]), _lib.dptr(b["fe"]), _lib.dptr(F), 0,
-                                           _lib.stream_of()), "wnfea_beam_forces")
+                                           _lib.dptr(b["inc"]), None, _lib.dptr(F), 0, _lib.stream_of()),
+                       "wnfea_beam_forces")
             acc = 1
         if self.solids is not None:
             m = self.solids

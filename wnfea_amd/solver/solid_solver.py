@@ -209,9 +209,10 @@ def _assemble_values(K: DeviceBSR, mesh: dict, cptr, codes, fix) -> None:
 
 def reassemble_c3d10_values(system: SolidSystem, E=None, nu=None) -> SolidSystem:
     """Assemble new per-element moduli (device tensors or arrays of length M)
-    into the resident K of a system built with keep_plan=True: element
-    stiffnesses, the deterministic gather, the diagonal, the scaling and the
-    equilibrated copies are recomputed in place; the pattern is unchanged."""
+    into the resident K of a system built with keep_plan=True: the values (from
+    element records, or on a mesh with curved elements from element
+    stiffnesses), the diagonal, the scaling and the equilibrated copies are
+    recomputed in place; the pattern is unchanged."""
     import torch
     mesh = system.mesh
     plan = mesh.get("plan")
