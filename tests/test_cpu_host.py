@@ -105,12 +105,23 @@ def test_node_graph_matches_reference_construction():
     assert A.dtype == np.int8 and np.all(A.data == 1)
 
 
-def test_rcm_matches_golden_and_scipy():
+def test_rcm_matches_golden_and_scipy(monkeypatch):
+    """The order of this machine's scipy, and the committed one from its own
+    start: numpy's argsort, whose first entry starts the one component, breaks
+    ties between equal degrees by the machine's vector width."""
+    from wnfea_amd.mesh import rcm
     from wnfea_amd.mesh.rcm import compute_node_adjacency_matrix, compute_rcm_order
     model = G.c0_model()
     A = compute_node_adjacency_matrix(len(model.mesh_nodes), None, model.solid_elements)
-    n2o, o2n = compute_rcm_order(A)
-    assert np.array_equal(n2o, np.load(os.path.join(GOLDEN, "c0_rcm_new_to_old.npy")))
+    assert np.array_equal(compute_rcm_order(A)[0], csg.reverse_cuthill_mckee(A, symmetric_mode=True))
+    golden = np.load(os.path.join(GOLDEN, "c0_rcm_new_to_old.npy"))
+    seed, first = rcm.rcm_seed_order(A), golden[-1]
+    degree = np.diff(A.indptr)
+    assert degree[first] == degree[seed[0]] == degree.min()
+    with monkeypatch.context() as mp:
+        mp.setattr(rcm, "rcm_seed_order", lambda _: np.append(first, seed[seed != first]).astype(np.int32))
+        n2o, o2n = compute_rcm_order(A)
+    assert np.array_equal(n2o, golden)
     assert np.array_equal(o2n[n2o], np.arange(len(n2o)))
     rng = np.random.default_rng(11)
     for t in range(40):

@@ -263,13 +263,19 @@ def test_stress_field_vs_golden(c0):
 
 # ---------------------------------------------------------------- RCM
 def test_oracle_rcm_matches_golden_and_scipy():
-    """C0 node graph: oracle RCM = the committed scipy permutation; random
-    symmetric graphs (with isolated nodes and several components): oracle =
-    scipy.sparse.csgraph.reverse_cuthill_mckee."""
+    """C0 node graph: oracle RCM = the committed scipy permutation, started
+    where that one starts (numpy's argsort, whose first entry starts the one
+    component, breaks ties between equal degrees by the machine's vector
+    width); random symmetric graphs (with isolated nodes and several
+    components): oracle = scipy.sparse.csgraph.reverse_cuthill_mckee."""
     model = G.c0_model()
     adj = G.node_graph(len(model.mesh_nodes), model.solid_elements)
     golden = np.load(os.path.join(GOLDEN, "c0_rcm_new_to_old.npy"))
-    assert np.array_equal(O.rcm(adj), golden)
+    degree = np.diff(adj.indptr)
+    assert degree[golden[-1]] == degree.min()
+    rest = np.argsort(degree)
+    assert np.array_equal(O.rcm(adj, np.append(golden[-1], rest[rest != golden[-1]])), golden)
+    assert np.array_equal(O.rcm(adj), csg.reverse_cuthill_mckee(adj, symmetric_mode=True))
     rng = np.random.default_rng(7)
     for t in range(60):
         n = int(rng.integers(1, 120))
