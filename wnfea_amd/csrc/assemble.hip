@@ -20,9 +20,10 @@
 // have one to six contributions and one lane each; diagonal blocks have up to
 // a few dozen and sixteen lanes each.  Lanes follow the layout's slots, so
 // values are stored as contiguous 1 KB chunks.  117 585 rows, 69 600 elements:
-// element matrices and their gather 145 + 440 us, here records 10.5,
-// off-diagonal blocks 188 (ten 16-byte gathers per contribution) and diagonal
-// blocks 34 us.
+// element matrices and their gather 145 + 440 us, here records 9,
+// off-diagonal blocks 187 (ten 16-byte gathers per contribution) and diagonal
+// blocks 33 us.  Against blocks in higher precision the error is that of the
+// element matrices to about a tenth (9.0e-15 of the norm against 8.0e-15).
 #include "sell.hpp"
 #include "wn.hpp"
 

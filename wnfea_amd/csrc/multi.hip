@@ -41,7 +41,7 @@ constexpr int kMrBlock = 256;
 // Chebyshev step / FP64 product / 6x6 level-1 step, us: all columns per lane
 // with x from L1 and four wavefronts per slice 72 / 107 / 50; four columns
 // per lane with x from L1 and the reduce-scatter 45 / 72 / 27; this kernel
-// 44 / 58 / 26.  (Loading a step's x during the one before costs 22 registers
+// 44 / 58 / 30 (kernel trace of a solve of 12 load cases).  (Loading a step's x during the one before costs 22 registers
 // and gains nothing; one scalar column per lane, three times the loads, takes
 // 75 / 80 / 45.)
 template <int BR, int BC, typename XT, int NR>
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(1024) void mr_finalize_kernel(const double* __restr
   if (mode != kMrStart && flags[0]) return;
   // wavefront w: column w mod NR, every (16 / NR)-th run of 64 partials; the
   // columns' loads run side by side, eight in flight per lane (one column
-  // after the other was eight serial memory latencies: 9.9 us, here 3.5 us)
+  // after the other was eight serial memory latencies: 9.9 us, here 4.6 us)
   constexpr int S = 16 / NR, U = 8;
   __shared__ double red[NR][S];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
